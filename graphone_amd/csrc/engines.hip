@@ -505,6 +505,11 @@ __global__ void dstamp_init_kernel(uint32_t n, uint32_t src, unsigned long long*
         ds[v] = (v == src) ? 0ull : (static_cast<unsigned long long>(kInf) << 32);
 }
 
+__global__ void depth_init_kernel(uint32_t n, uint32_t src, uint32_t* __restrict__ depth) {
+    const uint32_t stride = gridDim.x * blockDim.x;
+    for (uint32_t v = blockIdx.x * blockDim.x + threadIdx.x; v < n; v += stride) depth[v] = v == src ? 0u : kInf;
+}
+
 __global__ void dstamp_extract_kernel(uint32_t n, const unsigned long long* __restrict__ ds,
                                       uint32_t* __restrict__ dist) {
     const uint32_t stride = gridDim.x * blockDim.x;
@@ -564,52 +569,69 @@ g1_status ensure_road_work(g1_graph* g, hipStream_t s) {
     return G1_OK;
 }
 
-// Runs one query on the road engine; *ok = false when it must be run elsewhere.
+// Runs one query on the road engine, its result in out; *ok = false when it must be run elsewhere. The
+// record lives in pinned host memory: the kernel reads the query from it and writes the outcome to it, so a
+// run is three or four launches and one stream synchronization. A small graph's query runs with its distances
+// in LDS (road_lds_kernel); if that reports status 2 (a distance past 16 bits, or a list overflow) the query
+// runs on the global-memory kernel.
 template <bool kSssp>
-g1_status run_road(g1_graph* g, uint32_t src, uint32_t* depth, g1_run_stats* st, hipStream_t s, bool* ok) {
+g1_status run_road(g1_graph* g, uint32_t src, uint32_t* out, g1_run_stats* st, hipStream_t s, bool* ok) {
     G1_TRY(ensure_road_work(g, s));
-    RoadQuery* hq = reinterpret_cast<RoadQuery*>(g->h_ctr + 128);  // pinned staging
-    memset(hq, 0, sizeof(RoadQuery));
-    G1_CHECK(kSssp || depth != nullptr, G1_ERR_INTERNAL, "road engine: BFS without a depth array");
-    hq->sssp = kSssp ? 1u : 0u;
-    hq->dstamp = g->dstamp;
-    hq->depth = depth;
-    hq->q[0] = g->q[0];
-    hq->q[1] = g->q[1];
-    hq->far[0] = g->road_far[0];
-    hq->far[1] = g->road_far[1];
-    hq->src = src;
-    const RoadQuery staged = *hq;
+    const uint32_t n = g->n;
+    RoadQuery* hq = reinterpret_cast<RoadQuery*>(g->h_ctr + 128);
     const uint64_t qcap = std::min<uint64_t>(static_cast<uint64_t>(g->seg_cap) * kSegments, 0xFFFFFFFFull);
-    // A small graph's SSSP runs with its distances in LDS (road_lds_sssp_kernel); if that reports status 2
-    // (a distance past 16 bits, or a far-list overflow) it leaves the distance words untouched and the
-    // query runs on the global-memory kernel.
-    int tok = -1;
-    for (int pass = (kSssp && g->n <= kRoadLdsMaxN) ? 0 : 1; pass < 2; ++pass) {
-        *hq = staged;
-        G1_HIP(hipMemcpyAsync(g->road_q, hq, sizeof(RoadQuery), hipMemcpyHostToDevice, s));
-        tok = prof_begin(g, kSssp ? "road_sssp" : "road_bfs", s);
-        RoadQuery* dq = static_cast<RoadQuery*>(g->road_q);
+    for (int pass = n <= kRoadLdsMaxN ? 0 : 1; pass < 2; ++pass) {
+        memset(hq, 0, sizeof(RoadQuery));
+        hq->sssp = kSssp ? 1u : 0u;
+        hq->dstamp = g->dstamp;
+        hq->depth = out;
+        for (int i = 0; i < 2; ++i) {
+            hq->q[i] = g->q[i];
+            hq->far[i] = g->road_far[i];
+        }
+        hq->src = src;
+        hq->status = 2;
+        const uint32_t init_blocks = grid_for(n, 256, kMaxPushBlocks);
+        if (pass == 1) {
+            if (kSssp) dstamp_init_kernel<<<init_blocks, 256, 0, s>>>(n, src, g->dstamp);
+            else depth_init_kernel<<<init_blocks, 256, 0, s>>>(n, src, out);
+            G1_LAUNCHED();
+        }
+        G1_HIP(hipEventRecord(g->ev[0], s));
+        const int tok = prof_begin(g, kSssp ? "road_sssp" : "road_bfs", s);
         if (pass == 0) {
-            road_lds_sssp_kernel<<<1, kRoadThreads, 0, s>>>(g->n, g->row_off, g->col, g->w, dq, road_delta(g, true),
-                                                            g->road_far_cap, static_cast<uint32_t>(qcap), kHistIters);
+            road_lds_kernel<<<1, kRoadThreads, 0, s>>>(n, g->row_off, g->col, g->w, hq, road_delta(g, true),
+                                                       g->road_far_cap, static_cast<uint32_t>(qcap), kHistIters);
         } else {
-            road_query_kernel<<<1, kRoadThreads, 0, s>>>(g->row_off, g->col, g->w, dq, road_delta(g, false), g->road_far_cap,
-                                                         static_cast<uint32_t>(qcap), kHistIters);
+            road_query_kernel<<<1, kRoadThreads, 0, s>>>(g->row_off, g->col, g->w, hq, road_delta(g, false),
+                                                         g->road_far_cap, static_cast<uint32_t>(qcap), kHistIters);
         }
         G1_LAUNCHED();
         prof_end(g, tok, s, 0.0);
-        G1_HIP(hipMemcpyAsync(hq, g->road_q, sizeof(RoadQuery), hipMemcpyDeviceToHost, s));
+        G1_HIP(hipEventRecord(g->ev[1], s));
+        if (pass == 1 && kSssp) {
+            dstamp_extract_kernel<<<init_blocks, 256, 0, s>>>(n, g->dstamp, out);
+            G1_LAUNCHED();
+        }
+        reached_stats_kernel<<<init_blocks, 256, 0, s>>>(n, out, g->row_off, g->slots + 2 * kMaxPushBlocks,
+                                                         g->slots + 3 * kMaxPushBlocks);
+        G1_LAUNCHED();
+        push_finish_kernel<<<1, 256, 0, s>>>(g->slots, g->ctr, g->overflow, nullptr, 0, g->h_ctr, nullptr);
+        G1_LAUNCHED();
         G1_HIP(hipStreamSynchronize(s));
-        if (hq->status == 0) break;
+        *ok = hq->status == 0;
+        prof_set_bytes(g, tok, *ok ? 16.0 * static_cast<double>(hq->frontier_sum) + 12.0 * static_cast<double>(hq->edges_sum) : 0.0);
+        if (*ok) break;
     }
-    *ok = hq->status == 0;
+    G1_TRY(prof_flush(g));
     if (!*ok) return G1_OK;
-    prof_set_bytes(g, tok, 16.0 * static_cast<double>(hq->frontier_sum) + 12.0 * static_cast<double>(hq->edges_sum));
+    G1_TRY(elapsed(g, st));
     st->iterations = hq->iterations;
     st->push_iterations = hq->iterations;
     st->frontier_sum = hq->frontier_sum;
     st->edges_sum = hq->edges_sum;
+    st->reached = g->h_ctr[4];
+    st->reached_edges = g->h_ctr[5];
     return G1_OK;
 }
 
@@ -649,43 +671,61 @@ g1_status road_batch_run(g1_graph* g, const uint32_t* kinds, const uint32_t* sou
         G1_TRY(graph_alloc(g, &p, per));
         g->road_slots.push_back(p);
     }
-    const uint64_t qcap = n;
-    for (uint32_t b0 = 0; b0 < count; b0 += kRoadSlots) {
-        const uint32_t c = std::min<uint32_t>(kRoadSlots, count - b0);
-        std::vector<RoadQuery> hq(c);
-        std::vector<uint32_t*> hout(c);
-        for (uint32_t i = 0; i < c; ++i) {
-            uint8_t* base = static_cast<uint8_t*>(g->road_slots[i]);
-            RoadQuery& Q = hq[i];
-            memset(&Q, 0, sizeof(Q));
-            Q.sssp = kinds[b0 + i] ? 1u : 0u;
-            Q.dstamp = reinterpret_cast<unsigned long long*>(base);
-            uint32_t* u32 = reinterpret_cast<uint32_t*>(base + n * sizeof(unsigned long long));
-            Q.q[0] = u32;
-            Q.q[1] = u32 + n;
-            Q.far[0] = u32 + 2 * n;
-            Q.far[1] = u32 + 2 * n + g->road_far_cap;
-            Q.depth = outs[b0 + i];
-            Q.src = sources[b0 + i];
-            hout[i] = outs[b0 + i];
+    const uint32_t qcap = g->n;
+    // Small graphs take the kernel with its distances in LDS first; the queries it hands back (status 2), and
+    // every query of a larger graph, take the global-memory one.
+    std::vector<uint32_t> todo(count);
+    for (uint32_t i = 0; i < count; ++i) todo[i] = i;
+    for (int pass = g->n <= kRoadLdsMaxN ? 0 : 1; pass < 2 && !todo.empty(); ++pass) {
+        std::vector<uint32_t> again;
+        for (size_t b0 = 0; b0 < todo.size(); b0 += kRoadSlots) {
+            const uint32_t c = static_cast<uint32_t>(std::min<size_t>(kRoadSlots, todo.size() - b0));
+            std::vector<RoadQuery> hq(c);
+            std::vector<uint32_t*> hout(c);
+            for (uint32_t i = 0; i < c; ++i) {
+                const uint32_t id = todo[b0 + i];
+                uint8_t* base = static_cast<uint8_t*>(g->road_slots[i]);
+                RoadQuery& Q = hq[i];
+                memset(&Q, 0, sizeof(Q));
+                Q.sssp = kinds[id] ? 1u : 0u;
+                Q.dstamp = reinterpret_cast<unsigned long long*>(base);
+                uint32_t* u32 = reinterpret_cast<uint32_t*>(base + n * sizeof(unsigned long long));
+                Q.q[0] = u32;
+                Q.q[1] = u32 + n;
+                Q.far[0] = u32 + 2 * n;
+                Q.far[1] = u32 + 2 * n + g->road_far_cap;
+                Q.depth = outs[id];
+                Q.src = sources[id];
+                hout[i] = outs[id];
+            }
+            RoadQuery* dq = static_cast<RoadQuery*>(g->road_q);
+            G1_HIP(hipMemcpyAsync(dq, hq.data(), c * sizeof(RoadQuery), hipMemcpyHostToDevice, s));
+            if (pass == 0) {
+                road_lds_kernel<<<c, kRoadThreads, 0, s>>>(g->n, g->row_off, g->col, g->w, dq, road_delta(g, true),
+                                                           g->road_far_cap, qcap, kHistIters);
+                G1_LAUNCHED();
+            } else {
+                uint32_t** douts = g->road_outs;
+                G1_HIP(hipMemcpyAsync(douts, hout.data(), c * sizeof(uint32_t*), hipMemcpyHostToDevice, s));
+                const dim3 all(std::min<uint32_t>(grid_for(g->n, 256, 1024), 1024), c);
+                road_init_kernel<<<all, 256, 0, s>>>(g->n, dq, c);
+                G1_LAUNCHED();
+                road_query_kernel<<<c, kRoadThreads, 0, s>>>(g->row_off, g->col, g->w, dq, road_delta(g, false),
+                                                             g->road_far_cap, qcap, kHistIters);
+                G1_LAUNCHED();
+                road_extract_kernel<<<all, 256, 0, s>>>(g->n, dq, douts, c);
+                G1_LAUNCHED();
+            }
+            G1_HIP(hipMemcpyAsync(hq.data(), dq, c * sizeof(RoadQuery), hipMemcpyDeviceToHost, s));
+            G1_HIP(hipStreamSynchronize(s));
+            for (uint32_t i = 0; i < c; ++i) {
+                const uint32_t id = todo[b0 + i];
+                ok[id] = hq[i].status == 0 ? 1 : 0;
+                if (iters) iters[id] = hq[i].iterations;
+                if (pass == 0 && !ok[id]) again.push_back(id);
+            }
         }
-        RoadQuery* dq = static_cast<RoadQuery*>(g->road_q);
-        G1_HIP(hipMemcpyAsync(dq, hq.data(), c * sizeof(RoadQuery), hipMemcpyHostToDevice, s));
-        uint32_t** douts = g->road_outs;
-        G1_HIP(hipMemcpyAsync(douts, hout.data(), c * sizeof(uint32_t*), hipMemcpyHostToDevice, s));
-        road_init_kernel<<<dim3(std::min<uint32_t>(grid_for(g->n, 256, 1024), 1024), c), 256, 0, s>>>(g->n, dq, c);
-        G1_LAUNCHED();
-        road_query_kernel<<<c, kRoadThreads, 0, s>>>(g->row_off, g->col, g->w, dq, road_delta(g, false), g->road_far_cap,
-                                                     static_cast<uint32_t>(qcap), kHistIters);
-        G1_LAUNCHED();
-        road_extract_kernel<<<dim3(std::min<uint32_t>(grid_for(g->n, 256, 1024), 1024), c), 256, 0, s>>>(g->n, dq, douts, c);
-        G1_LAUNCHED();
-        G1_HIP(hipMemcpyAsync(hq.data(), dq, c * sizeof(RoadQuery), hipMemcpyDeviceToHost, s));
-        G1_HIP(hipStreamSynchronize(s));
-        for (uint32_t i = 0; i < c; ++i) {
-            ok[b0 + i] = hq[i].status == 0 ? 1 : 0;
-            if (iters) iters[b0 + i] = hq[i].iterations;
-        }
+        if (pass == 0) todo.swap(again);
     }
     return G1_OK;
 }
@@ -694,34 +734,13 @@ g1_status run_sssp_push(g1_graph* g, uint32_t src, uint32_t* dist, g1_run_stats*
                         bool allow_road = true);
 
 g1_status run_sssp_road(g1_graph* g, uint32_t src, uint32_t* dist, g1_run_stats* st, hipStream_t s) {
-    G1_TRY(ensure_road_work(g, s));
-    const uint32_t n = g->n;
-    dstamp_init_kernel<<<grid_for(n, 256, kMaxPushBlocks), 256, 0, s>>>(n, src, g->dstamp);
-    G1_LAUNCHED();
-    G1_HIP(hipEventRecord(g->ev[0], s));
     bool ok = false;
-    G1_TRY(run_road<true>(g, src, nullptr, st, s, &ok));
-    if (!ok) return run_sssp_push(g, src, dist, st, s, false);
-    G1_HIP(hipEventRecord(g->ev[1], s));
-    G1_TRY(elapsed(g, st));
-    G1_TRY(prof_flush(g));
-    dstamp_extract_kernel<<<grid_for(n, 256, kMaxPushBlocks), 256, 0, s>>>(n, g->dstamp, dist);
-    G1_LAUNCHED();
-    return finish_stats(g, dist, st, s);
+    G1_TRY(run_road<true>(g, src, dist, st, s, &ok));
+    return ok ? G1_OK : run_sssp_push(g, src, dist, st, s, false);
 }
 
 g1_status run_bfs_road(g1_graph* g, uint32_t src, uint32_t* depth, g1_run_stats* st, hipStream_t s, bool* ok) {
-    G1_TRY(ensure_road_work(g, s));
-    G1_TRY(g1_fill_u32(depth, kInf, g->n, s));
-    set_u32_kernel<<<1, 64, 0, s>>>(depth, src, 0u);
-    G1_LAUNCHED();
-    G1_HIP(hipEventRecord(g->ev[0], s));
-    G1_TRY(run_road<false>(g, src, depth, st, s, ok));
-    if (!*ok) return G1_OK;
-    G1_HIP(hipEventRecord(g->ev[1], s));
-    G1_TRY(elapsed(g, st));
-    G1_TRY(prof_flush(g));
-    return finish_stats(g, depth, st, s);
+    return run_road<false>(g, src, depth, st, s, ok);
 }
 
 // The push iterations of the SSSP advance engine from iteration it0, whose input frontier is in the

@@ -335,6 +335,37 @@ def test_road_sssp_past_16_bit_distances(gpu):
         assert np.array_equal(got.values, want), hi
 
 
+@pytest.mark.parametrize("n, deg", [(1, 0), (2, 1), (300, 16), (46080, 5), (46081, 7), (120000, 16)])
+def test_road_engine_shapes(gpu, n, deg):
+    """The one-workgroup engine around its own limits: 46,080 vertices (the last size with distances in LDS) and
+    one more, rows of more than four edges (four lanes a row) up to the engine's sixteen, frontiers past the
+    2048 and 4096 entries kept in LDS (a random graph of this degree reaches tens of thousands of vertices in
+    one level), a vertex alone; single runs and one batch, weighted and, for BFS, without weights. Also
+    weights whose distances pass 16 bits, which the batch hands from one kernel to the other."""
+    import graphone_amd as g1
+    rng = np.random.default_rng(n + deg)
+    src = np.repeat(np.arange(n), deg)
+    dst = (src + rng.integers(1, n, size=src.size)) % n if n > 1 else src
+    for hi in ((30,) if n > 46081 else (30, 40000)):
+        w = rng.integers(1, hi + 1, size=src.size).astype(np.uint32)
+        h = g1.HostGraph.from_edges(n, src, dst, w)
+        g = g1.Graph(h)
+        assert int(h.out_degrees().max(initial=0)) <= 16
+        s0 = n // 2
+        dj, bf = oracle.dijkstra(h.row_offsets, h.col_indices, h.weights, s0), oracle.bfs_queue(h.row_offsets, h.col_indices, s0)
+        for _ in range(2):
+            got = g.sssp(s0, "advance")
+            assert np.array_equal(got.values, dj)
+            assert got.stats["reached"] == int((dj != g1.INF).sum())
+        assert np.array_equal(g.bfs(s0, "advance").values, bf)
+        batch = g.road_batch([s0, s0, n - 1], ["sssp", "bfs", "sssp"])
+        last = oracle.dijkstra(h.row_offsets, h.col_indices, h.weights, n - 1)
+        for row, want in zip(batch.values, (dj, bf, last)):
+            assert np.array_equal(row, want)
+    unweighted = g1.Graph(g1.HostGraph.from_edges(n, src, dst))
+    assert np.array_equal(unweighted.bfs(s0, "advance").values, bf)
+
+
 def test_pagerank_rmat20_l1(gpu):
     """PageRank on unweighted RMAT scale 20 (16.1M edges) within L1 1e-5 of the FP64 oracle."""
     import graphone_amd as g1
