@@ -370,7 +370,7 @@ def dropin_sssp_adv(h, src: int) -> dict | None:
 
 def pagerank_benchmark(g1, scale: int, seed: int, cpu: bool) -> dict:
     """PageRank (apps/pagerank_blas.cu formula) on an unweighted RMAT graph (edge factor 16, the main a/b/c/d):
-    damping 0.85, FP32 ranks with Kahan row sums, FP64 L1 stop at 1e-7 or 50 iterations, both SpMV engines.
+    damping 0.85, FP32 ranks with 64-bit row sums, FP64 L1 stop at 1e-7 or 50 iterations, both SpMV engines.
     Per iteration the algorithmic bytes are 4(n+1) + 4m + 4m (x gather) + 4n (y) for the SpMV and 20n for
     the apply. The two engines' ranks are compared with each other, and (with `cpu`) with the oracle's FP64
     power iteration under the same stop rule on the same graph: L1 and max-abs per engine. The FP64 run is

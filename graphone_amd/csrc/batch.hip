@@ -1,5 +1,5 @@
 // Batched multi-source engines: k sources run together as k columns of one semiring SpMM over the
-// in-edge CSR (g1/spmm.hpp), min-plus for SSSP/BFS and compensated plus-times for personalized PageRank.
+// in-edge CSR (g1/spmm.hpp), min-plus for SSSP/BFS and plus-times (64-bit sums) for personalized PageRank.
 //
 // A batch of S sources is cut into ceil(S/k) column tiles of k in {8, 16, 32, 64}; k comes from the
 // caller or from the autotuner (g1_batch_autotune), which times one tile of every width on the graph and
@@ -164,7 +164,7 @@ g1_status ensure_batch(g1_graph* g, uint32_t K, bool ppr, BatchWork** out, hipSt
         // (min-plus k = 64 may run on the smallest merge tile: four times the graph's tiles)
         const size_t rb = std::max(static_cast<size_t>(merge_num_tiles_for(g->n, g->m, kWaveTileItems[0])) *
                                        sizeof(SpmmTileRec<MinPlusU32, 64>),
-                                   spmm_records_bytes<PlusTimesKahanF32, 64>(g->n, g->m));
+                                   spmm_records_bytes<PlusTimesF32, 64>(g->n, g->m));
         void* v = nullptr;
         G1_TRY(graph_alloc(g, &v, rb + 256));
         b->recs = v;
@@ -264,13 +264,13 @@ bool ppr_wave() {
     return on;
 }
 
-// One plus-times SpMM iteration: Y = A^T (x) X over the in-edges (k columns, Kahan sums in the fold order
+// One plus-times SpMM iteration: Y = A^T (x) X over the in-edges (k columns, 64-bit sums in the fold order
 // of the single-source SpMV), then the fixup of rows that cross tiles.
 template <int K>
 g1_status launch_plustimes(g1_graph* g, const float* X, float* Y, void* recs_v, hipStream_t s) {
     const uint32_t tiles = merge_num_tiles(g->n, g->m);
     PlusTimesBatchPolicy<K> pol{X, Y};
-    auto* recs = static_cast<SpmmTileRec<PlusTimesKahanF32, K>*>(recs_v);
+    auto* recs = static_cast<SpmmTileRec<PlusTimesF32, K>*>(recs_v);
     const MergeCoord* coords = merge_coords(g->t_ws);
     const float* vals = g->t_wf;
     bool done = false;
@@ -288,13 +288,13 @@ g1_status launch_plustimes(g1_graph* g, const float* X, float* Y, void* recs_v, 
         }
     }
     if (!done) {
-        spmm_tile_kernel<PlusTimesKahanF32, K, PlusTimesBatchPolicy<K>><<<tiles, 256, 0, s>>>(
+        spmm_tile_kernel<PlusTimesF32, K, PlusTimesBatchPolicy<K>><<<tiles, 256, 0, s>>>(
             g->n, g->m, g->t_row_off, g->t_col, vals, coords, recs, pol, nullptr);
         G1_LAUNCHED();
     }
     if (tiles > 1) {
         const uint32_t blocks = static_cast<uint32_t>((static_cast<uint64_t>(tiles) * K + 255) / 256);
-        spmm_fixup_kernel<PlusTimesKahanF32, K, PlusTimesBatchPolicy<K>><<<blocks, 256, 0, s>>>(tiles, coords, recs,
+        spmm_fixup_kernel<PlusTimesF32, K, PlusTimesBatchPolicy<K>><<<blocks, 256, 0, s>>>(tiles, coords, recs,
                                                                                               pol, nullptr);
         G1_LAUNCHED();
     }
@@ -767,7 +767,7 @@ namespace {
 size_t records_bytes(const g1_graph* g, int kind, uint32_t k) {
     auto pick = [&](auto tag) -> size_t {
         constexpr int KK = decltype(tag)::value;
-        return kind == kSessPpr ? spmm_records_bytes<PlusTimesKahanF32, KK>(g->n, g->m)
+        return kind == kSessPpr ? spmm_records_bytes<PlusTimesF32, KK>(g->n, g->m)
                                 : spmm_records_bytes<MinPlusU32, KK>(g->n, g->m);
     };
     switch (k) {

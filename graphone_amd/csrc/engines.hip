@@ -1339,10 +1339,10 @@ g1_status run_pagerank(g1_graph* g, float alpha, uint32_t seed, float restart, u
             delta = g->h_scalar[0];
             if (delta <= tol || it >= max_iter) break;
             if (engine == G1_ENGINE_BLAS_CSRVEC)
-                G1_TRY(launch_spmv_csrvec<PlusTimesKahanF32>(n, t_ro, t_ci, vals, g->xf, g->yf, lanes, s, lrows, nlong,
+                G1_TRY(launch_spmv_csrvec<PlusTimesF32>(n, t_ro, t_ci, vals, g->xf, g->yf, lanes, s, lrows, nlong,
                                                               g->long_min));
             else
-                G1_TRY(launch_spmv_merge<PlusTimesKahanF32>(n, g->m, t_ro, t_ci, vals, g->xf, g->yf, ws, s));
+                G1_TRY(launch_spmv_merge<PlusTimesF32>(n, g->m, t_ro, t_ci, vals, g->xf, g->yf, ws, s));
             // In place on ranks[idx] as apply_each does; the partials of this call are unused.
             pr_apply_kernel<1><<<blocks, 256, 0, s>>>(n, g->yf, base_all, seed, base_seed, g->iw, g->r[idx ^ 1],
                                                       g->r[idx], g->xf, g->partials);
@@ -1361,11 +1361,11 @@ g1_status run_pagerank(g1_graph* g, float alpha, uint32_t seed, float restart, u
             int tok;
             if (engine == G1_ENGINE_BLAS_CSRVEC) {
                 tok = prof_begin(g, "spmv_csrvec_plustimes", s);
-                G1_TRY(launch_spmv_csrvec<PlusTimesKahanF32>(n, t_ro, t_ci, vals, g->xf, g->yf, lanes, s, lrows, nlong,
+                G1_TRY(launch_spmv_csrvec<PlusTimesF32>(n, t_ro, t_ci, vals, g->xf, g->yf, lanes, s, lrows, nlong,
                                                               g->long_min));
             } else {
                 tok = prof_begin(g, "spmv_merge_plustimes", s);
-                G1_TRY(launch_spmv_merge<PlusTimesKahanF32>(n, g->m, t_ro, t_ci, vals, g->xf, g->yf, ws, s));
+                G1_TRY(launch_spmv_merge<PlusTimesF32>(n, g->m, t_ro, t_ci, vals, g->xf, g->yf, ws, s));
             }
             prof_end(g, tok, s, spmv_bytes);
             tok = prof_begin(g, "pr_apply", s);

@@ -1,5 +1,5 @@
 // C-ABI exports of the semiring SpMV kernels (merge-path and CSR-vector) for the two fixed semirings
-// of the hot path: min-plus over uint32 (SSSP/BFS) and compensated plus-times over float (PageRank).
+// of the hot path: min-plus over uint32 (SSSP/BFS) and plus-times over float with 64-bit sums (PageRank).
 #include <hip/hip_runtime.h>
 
 #include <mutex>
@@ -119,7 +119,7 @@ g1_status g1_spmv_merge_minplus_u32(uint32_t n_rows, uint32_t n_cols, uint32_t n
 g1_status g1_spmv_merge_plustimes_f32(uint32_t n_rows, uint32_t n_cols, uint32_t nnz, const uint32_t* row_offsets,
                                       const uint32_t* col, const float* vals, const float* x, float* y,
                                       void* ws, size_t ws_bytes, g1_stream_t stream) {
-    return g1::spmv_merge_exported<g1::PlusTimesKahanF32>(n_rows, n_cols, nnz, row_offsets, col, vals, x, y,
+    return g1::spmv_merge_exported<g1::PlusTimesF32>(n_rows, n_cols, nnz, row_offsets, col, vals, x, y,
                                                           ws, ws_bytes, stream);
 }
 
@@ -135,7 +135,7 @@ g1_status g1_spmv_csrvec_minplus_u32(uint32_t n_rows, uint32_t n_cols, uint32_t 
 g1_status g1_spmv_csrvec_plustimes_f32(uint32_t n_rows, uint32_t n_cols, uint32_t nnz, const uint32_t* row_offsets,
                                        const uint32_t* col, const float* vals, const float* x, float* y,
                                        uint32_t lanes, g1_stream_t stream) {
-    return g1::spmv_csrvec_exported<g1::PlusTimesKahanF32>(n_rows, n_cols, nnz, row_offsets, col, vals, x, y,
+    return g1::spmv_csrvec_exported<g1::PlusTimesF32>(n_rows, n_cols, nnz, row_offsets, col, vals, x, y,
                                                            lanes, stream);
 }
 

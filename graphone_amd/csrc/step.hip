@@ -107,10 +107,10 @@ g1_status advance(uint32_t n, const uint32_t* row_off, const uint32_t* col, cons
 }
 
 // SpMM workspace: the merge-path partition of the matrix, then the tile records of one 64-column pass
-// (sized for the larger record, the compensated plus-times one).
+// (sized for the larger record, the plus-times one).
 size_t spmm_ws_bytes(uint32_t n_rows, uint32_t nnz) {
     const size_t t = merge_num_tiles(n_rows, nnz);
-    return al((t + 1) * sizeof(MergeCoord)) + t * sizeof(SpmmTileRec<PlusTimesKahanF32, 64>) + 256;
+    return al((t + 1) * sizeof(MergeCoord)) + t * sizeof(SpmmTileRec<PlusTimesF32, 64>) + 256;
 }
 
 template <typename S>
@@ -284,7 +284,7 @@ g1_status g1_spmm_minplus_u32(uint32_t n_rows, uint32_t n_cols, uint32_t nnz, ui
 g1_status g1_spmm_plustimes_f32(uint32_t n_rows, uint32_t n_cols, uint32_t nnz, uint32_t k, const uint32_t* row_offsets,
                                 const uint32_t* col_indices, const float* values, const float* X, float* Y,
                                 const uint64_t* col_mask, void* ws, size_t ws_bytes, g1_stream_t stream) {
-    return spmm<PlusTimesKahanF32>(n_rows, n_cols, nnz, k, row_offsets, col_indices, values, X, Y,
+    return spmm<PlusTimesF32>(n_rows, n_cols, nnz, k, row_offsets, col_indices, values, X, Y,
                                    reinterpret_cast<const unsigned long long*>(col_mask), ws, ws_bytes,
                                    as_stream(stream), "g1_spmm_plustimes_f32");
 }

@@ -918,7 +918,7 @@ struct PlusTimesBatchPolicy {
 };
 
 // ------------------------------------------------------------------------------------------------
-// Batched plus-times (Kahan) at k = 64 with one wavefront per merge-path tile, lane j = column j, the
+// Batched plus-times at k = 64 with one wavefront per merge-path tile, lane j = column j, the
 // walk on the scalar unit. It reproduces the fold of spmv_merge_tile_kernel exactly, per column: the
 // tile's 2048 merge steps are cut into the same 256 runs of 8 ("virtual threads"); inside a run a row's
 // products are added left to right; a run that closes a row finishes its first closed row by merging,
@@ -937,9 +937,9 @@ __global__ void __launch_bounds__(256)
 spmm_plustimes_wave_kernel(uint32_t n_rows, uint32_t num_tiles, const uint32_t* __restrict__ row_offsets,
                            const uint32_t* __restrict__ col, const float* __restrict__ vals,
                            const MergeCoord* __restrict__ coords,
-                           SpmmTileRec<PlusTimesKahanF32, 64>* __restrict__ recs, const float* __restrict__ X,
+                           SpmmTileRec<PlusTimesF32, 64>* __restrict__ recs, const float* __restrict__ X,
                            float* __restrict__ Y) {
-    using S = PlusTimesKahanF32;
+    using S = PlusTimesF32;
     using acc_t = S::acc_t;
     __shared__ float s_x[4][kPprChunk][64];
     const uint32_t lane = threadIdx.x & 63u;

@@ -268,7 +268,7 @@ step_pr_apply_kernel(uint32_t n, const float* __restrict__ y, float base, const 
 // instead of one wave. This policy reads and writes the 64-column chunk starting at column c0 of the
 // caller's arrays (row stride ld = k); lanes past the chunk's kc columns, and columns whose bit is clear in
 // the device mask (bit j of word j / 64; null: every column), read nothing and write nothing, so their Y
-// values stay. Plus-times folds in the single-source merge-path SpMV's order (Kahan-Babuska), min-plus is
+// values stay. Plus-times folds in the single-source merge-path SpMV's order (64-bit sums), min-plus is
 // order-free.
 template <typename T>
 struct StridedColumnsPolicy {

@@ -77,7 +77,7 @@ g1_status g1_event_elapsed_ms(float* ms, g1_event_t start, g1_event_t stop);
  * Semiring SpMV  y = A (x) x  on a CSR matrix A (n_rows x n_cols, nnz nonzeros).
  *   min-plus u32 : y[r] = min_j ( x[c_j] == INF ? INF : A[r,c_j] + x[c_j] ), empty row -> INF
  *                  (the SSSP semiring of apps/sssp_blas.cu:55-73 with initialize = default_result)
- *   plus-times f32: y[r] = sum_j A[r,c_j] * x[c_j] with compensated (Kahan-Babuska) accumulation,
+ *   plus-times f32: y[r] = sum_j A[r,c_j] * x[c_j] of 32-bit products summed in 64 bits,
  *                  empty row -> 0 (the PageRank semiring of apps/pagerank_blas.cu:82-111)
  * `values_dev` may be NULL: every nonzero then has value 1 (an unweighted graph).
  * Results are deterministic: the plus-times fold order is a function of the matrix only.
@@ -206,7 +206,7 @@ g1_status g1_l1_delta_f64(uint32_t n, const float* a_dev, const float* b_dev, do
  * of include/GraphOne/engine/blas_gnn.h:18-122) and serving batched multi-source steps:
  *   min-plus u32 : Y[r][j] = min over the nonzeros (r, c) of (X[c][j] == G1_INF ? G1_INF : A[r,c] + X[c][j])
  *   plus-times f32: Y[r][j] = sum over the nonzeros of A[r,c] * X[c][j], left to right per row with the
- *                  compensated sum of the SpMV kernels
+ *                  64-bit sum of the SpMV kernels
  * col_mask_dev (device, ceil(k / 64) words; NULL = every column): only the columns whose bit is set are
  * computed, the others keep their Y values. values_dev NULL: unit values. The rows and nonzeros are
  * cut into merge-path tiles of equal size (a row of any length spreads over tiles), 64 columns per pass;
@@ -384,7 +384,7 @@ g1_status g1_sssp(g1_graph* graph, uint32_t src, uint32_t* dist_dev, int32_t eng
 
 /* PageRank (apps/pagerank_blas.cu:16-125): iw[u] = alpha / sum_out w (0 if none), r0 = 1/N,
  * r' = (1-alpha)/N + sum_{u->v} w * r[u] * iw[u]; no dangling redistribution.
- * FP32 values, Kahan row sums. converge_mode:
+ * FP32 values, 64-bit row sums. converge_mode:
  *   G1_PR_L1_F64   stop when the FP64 L1 norm of r'-r is < tol or after max_iter iterations
  *   G1_PR_MAX_ABS  the reference's test: before each iteration stop if max|r_cur - r_pre| <= tol
  *                  (the first test compares r0 with a zero vector, as apps/pagerank_blas.cu:63-78)
