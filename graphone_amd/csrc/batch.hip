@@ -276,13 +276,8 @@ g1_status launch_plustimes(g1_graph* g, const float* X, float* Y, void* recs_v, 
     bool done = false;
     if constexpr (K == 64) {
         if (ppr_wave()) {
-            const uint32_t blocks = (tiles + 3) / 4;
-            if (vals)
-                spmm_plustimes_wave_kernel<true><<<blocks, 256, 0, s>>>(g->n, tiles, g->t_row_off, g->t_col, vals,
-                                                                        coords, recs, X, Y);
-            else
-                spmm_plustimes_wave_kernel<false><<<blocks, 256, 0, s>>>(g->n, tiles, g->t_row_off, g->t_col, vals,
-                                                                         coords, recs, X, Y);
+            launch_spmm_wave<PlusTimesF32>(g->n, tiles, g->t_row_off, g->t_col, vals, coords, recs, pol,
+                                           static_cast<uint64_t>(g->n) * K * sizeof(float), s);
             G1_LAUNCHED();
             done = true;
         }

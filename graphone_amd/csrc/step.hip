@@ -133,8 +133,8 @@ g1_status spmm(uint32_t n_rows, uint32_t n_cols, uint32_t nnz, uint32_t k, const
     const T neutral = std::is_same_v<S, MinPlusU32> ? static_cast<T>(kInf) : T(0);
     for (uint32_t c0 = 0; c0 < k; c0 += 64) {
         StridedColumnsPolicy<T> pol{X, Y, k, c0, std::min<uint32_t>(64u, k - c0), mask, neutral};
-        spmm_tile_kernel<S, 64, StridedColumnsPolicy<T>><<<tiles, 256, 0, s>>>(n_rows, nnz, row_off, col, vals, coords,
-                                                                             recs, pol, nullptr);
+        launch_spmm_wave<S>(n_rows, tiles, row_off, col, vals, coords, recs, pol, static_cast<uint64_t>(n_cols) * k * sizeof(T),
+                            s);
         G1_LAUNCHED();
         if (tiles > 1) {
             spmm_fixup_kernel<S, 64, StridedColumnsPolicy<T>><<<(tiles * 64u + 255) / 256, 256, 0, s>>>(

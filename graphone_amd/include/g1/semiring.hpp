@@ -5,6 +5,7 @@
 // accumulator, so that a sum keeps more bits than a y value across threads and tiles:
 //   identity()      the accumulator of an empty fold (initialize())
 //   combine(w, x)   the per-nonzero product
+//   nothing()       a product that add() leaves acc unchanged by
 //   add(acc, p)     acc = reduce(acc, p), p to the right of everything already in acc
 //   merge(a, b)     the fold of a followed by b (a holds the lower nonzero positions)
 //   finalize(acc)   the y value
@@ -28,6 +29,7 @@ struct MinPlusU32 {
     static constexpr bool kOrderFree = true;
 
     __device__ __forceinline__ static acc_t identity() { return acc_t{kInf}; }
+    __device__ __forceinline__ static uint32_t nothing() { return kInf; }
     __device__ __forceinline__ static uint32_t combine(uint32_t w, uint32_t x) {
         return x == kInf ? kInf : w + x;
     }
@@ -78,6 +80,7 @@ struct PlusTimesF32 {
     static constexpr bool kOrderFree = false;
 
     __device__ __forceinline__ static acc_t identity() { return acc_t{0.0}; }
+    __device__ __forceinline__ static float nothing() { return 0.0f; }
     __device__ __forceinline__ static float combine(float w, float x) { return x * w; }
     __device__ __forceinline__ static void add(acc_t& a, float p) { a.s += static_cast<double>(p); }
     __device__ __forceinline__ static acc_t merge(acc_t a, acc_t b) { return acc_t{a.s + b.s}; }

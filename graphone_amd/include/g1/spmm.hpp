@@ -65,7 +65,7 @@ spmm_tile_kernel(uint32_t n_rows, uint32_t nnz, const uint32_t* __restrict__ row
     using x_t = typename S::x_t;
     using aux_t = typename P::aux_t;
     constexpr int G = 256 / K;                  // virtual threads per round
-    constexpr int kRounds = kMergeThreads / G;  // = K
+    constexpr int kRounds = kMergeThreads / G;  // = K: a quarter of the virtual threads is K / 4 rounds
     constexpr int kWavesG = kWave / K;          // groups per wave
     __shared__ uint32_t s_rowend[kMergeTile + 1];
     __shared__ uint32_t s_col[kMergeTile];
@@ -74,7 +74,8 @@ spmm_tile_kernel(uint32_t n_rows, uint32_t nnz, const uint32_t* __restrict__ row
     __shared__ uint32_t s_vi[kMergeThreads + 1];  // first row (tile-relative) of each virtual thread
     __shared__ uint32_t s_vj[kMergeThreads + 1];  // first nonzero (tile-relative) of each virtual thread
     __shared__ acc_t s_tail[2][G][K];
-    __shared__ acc_t s_carry[2][K];
+    __shared__ acc_t s_carry[2][K];  // the open row since the quarter's start (a quarter: 64 virtual threads)
+    __shared__ acc_t s_outer[2][K];  // ... and in the quarters before it
     __shared__ uint32_t s_hm[2][256 / kWave];  // closing groups of the round, one word per wave
     __shared__ unsigned long long s_or;
 
@@ -139,7 +140,7 @@ spmm_tile_kernel(uint32_t n_rows, uint32_t nnz, const uint32_t* __restrict__ row
             s_vi[kMergeThreads] = rows;
             s_vj[kMergeThreads] = nzs;
         }
-        if (tid < static_cast<uint32_t>(K)) s_carry[0][tid] = S::identity();
+        if (tid < static_cast<uint32_t>(K)) s_carry[0][tid] = s_outer[0][tid] = S::identity();
     }
     __syncthreads();
 
@@ -149,6 +150,7 @@ spmm_tile_kernel(uint32_t n_rows, uint32_t nnz, const uint32_t* __restrict__ row
     // The tile's first closed row is deferred to the fixup when it began in an earlier tile.
     const bool first_started_before = (rows > 0) && (row_offsets[c0.x] < c0.y);
     bool seen = false;     // some row closed in an earlier round
+    bool seen_q = false;   // ... of this quarter
     uint64_t counted = 0;  // OR of the changed-column masks this lane's policy calls reported
 
     // Loads of round r: x values of its nonzeros, old values of the rows it closes (fixed count).
@@ -236,6 +238,7 @@ spmm_tile_kernel(uint32_t n_rows, uint32_t nnz, const uint32_t* __restrict__ row
 #pragma unroll
         for (int q = 0; q < 256 / kWave; ++q) hm |= s_hm[par][q];
         const acc_t open = s_carry[par][j];
+        const acc_t outer = s_outer[par][j];
         if (hasend) {
             const uint32_t below = hm & ((g == 31) ? 0x7fffffffu : ((1u << g) - 1u));
             acc_t chain;
@@ -248,13 +251,15 @@ spmm_tile_kernel(uint32_t n_rows, uint32_t nnz, const uint32_t* __restrict__ row
                 chain = open;
             }
             for (uint32_t v = v0; v < g; ++v) chain = S::merge(chain, s_tail[par][v][j]);
-            const acc_t whole = S::merge(chain, head);
+            acc_t whole = S::merge(chain, head);
+            if (!below && !seen_q) whole = S::merge(outer, whole);  // the quarter's first closed row
             if (!below && !seen && first_started_before) {
                 recs[tile].head[j] = whole;
             } else {
                 counted |= pol.row_done(first_row, j, S::finalize(whole), head_old);
             }
         }
+        const bool quarter_end = (r + 1) % (kRounds / 4) == 0;
         if (g == static_cast<uint32_t>(G - 1)) {
             acc_t c;
             uint32_t v0;
@@ -266,9 +271,15 @@ spmm_tile_kernel(uint32_t n_rows, uint32_t nnz, const uint32_t* __restrict__ row
                 c = open;
             }
             for (uint32_t v = v0; v < static_cast<uint32_t>(G); ++v) c = S::merge(c, s_tail[par][v][j]);
+            acc_t o = outer;
+            if (quarter_end) {
+                o = (seen_q || hm != 0) ? S::merge(S::identity(), c) : S::merge(outer, c);
+                c = S::identity();
+            }
             s_carry[par ^ 1][j] = c;
+            s_outer[par ^ 1][j] = o;
             if (r + 1 == kRounds) {
-                recs[tile].carry[j] = c;
+                recs[tile].carry[j] = o;
                 if (j == 0) {
                     const bool any = seen || hm != 0;
                     uint32_t flags = any ? kTileHasEnd : 0u;
@@ -277,6 +288,7 @@ spmm_tile_kernel(uint32_t n_rows, uint32_t nnz, const uint32_t* __restrict__ row
                 }
             }
         }
+        seen_q = !quarter_end && (seen_q || hm != 0);
         seen = seen || hm != 0;
     };
 
@@ -906,6 +918,15 @@ struct PlusTimesBatchPolicy {
     static constexpr bool kRowOld = false;
     const float* X;
     float* Y;
+    __device__ __forceinline__ void init(uint32_t) {}
+    template <bool kWide>
+    __device__ __forceinline__ float x(uint32_t u, uint32_t j) const {
+        if constexpr (kWide) return X[static_cast<size_t>(u) * K + j];
+        return *reinterpret_cast<const float*>(reinterpret_cast<const char*>(X) + (u * (K * 4u) + j * 4u));
+    }
+    __device__ __forceinline__ void store(uint32_t row, uint32_t j, float y) const {
+        Y[static_cast<size_t>(row) * K + j] = y;
+    }
     __device__ __forceinline__ aux_t aux(uint32_t) const { return 0u; }
     __device__ __forceinline__ float x(uint32_t u, aux_t, uint32_t j, bool) const {
         return X[static_cast<size_t>(u) * K + j];
@@ -918,37 +939,85 @@ struct PlusTimesBatchPolicy {
 };
 
 // ------------------------------------------------------------------------------------------------
-// Batched plus-times at k = 64 with one wavefront per merge-path tile, lane j = column j, the
-// walk on the scalar unit. It reproduces the fold of spmv_merge_tile_kernel exactly, per column: the
-// tile's 2048 merge steps are cut into the same 256 runs of 8 ("virtual threads"); inside a run a row's
-// products are added left to right; a run that closes a row finishes its first closed row by merging,
-// left to right, the tails of the runs since the last run that closed a row and then its own head; the
-// tile's open row leaves as the carry, a first row that began before the tile as the deferred head
-// (finished by spmm_fixup_kernel). Batched personalized PageRank columns therefore stay bit-identical
-// to the single-source runs.
+// SpMM over 64 columns: a workgroup of four waves takes a merge-path tile, a wave a quarter of its merge
+// steps, lane j = column j, the walk on the scalar unit. It reproduces the fold of spmv_merge_tile_kernel
+// exactly, per column: a quarter's 512 steps are cut into the same 64 runs of 8 that the threads of one of
+// its waves take; inside a run a row's products are added left to right; a run that closes a row finishes
+// its first closed row by merging, left to right, the tails of the runs since the last run that closed a
+// row and then its own head; the quarters' carries are merged in front of the first row a quarter closes,
+// the tile's open row leaves as the carry, a first row that began before the tile as the deferred head
+// (finished by spmm_fixup_kernel). Batched personalized PageRank columns therefore stay bit-identical to the
+// single-source runs.
 //
-// The x rows of 32 nonzeros are loaded at a time (one 256-byte access per source, issued a chunk ahead)
-// and parked in LDS, so the walk indexes them at run time; weights and column indices come with one
-// coalesced load per chunk and are read out of their lanes.
-constexpr uint32_t kPprChunk = 32;
+// Quarters, because a wave per tile left too few waves: 11 M rows and nonzeros are 5,300 tiles for 8,192
+// resident waves, and each wave's chain of loads is then as long as the launch.
+// What bounds it is the x rows, 256 bytes per nonzero, as long as the walk keeps out of their way; the walk is
+// one wave-uniform stream, so its scalar instructions are what it is made of. The x rows go to registers
+// kWaveChunk at a time: a chunk's products are formed from the rows loaded during the chunk before, the next
+// chunk's loads are issued, and the products are folded while those fly. The fold is unrolled over the chunk
+// and its next event (a row's end or a run's end, whichever comes first) is kept as a position in the chunk,
+// so a nonzero without an event costs a compare, a branch and its add; a source's row is a 32-bit offset
+// (kWide: 64-bit, for x arrays of 4 GB and more), one vector instruction. Column indices and values come 64 at
+// a time, a block ahead, and are read out of their lanes. Measured: 16 M nonzeros x 64 columns
+// 1.03 ms with the round-based tile kernel, 0.66 ms here (6.5 TB/s of x rows; 0.88 ms with a wave per tile, 0.85 ms
+// with the run counter and the 64-bit row addresses on the scalar unit as well, 19 scalar instructions a
+// nonzero against 8); 11 M nonzeros of a PPR batch 0.70 ms with x parked in LDS and a wave per tile, 0.40 ms.
+constexpr uint32_t kWaveChunk = 16;
+static_assert(64 % kWaveChunk == 0, "a block of 64 indices holds whole chunks");
 
-template <bool kWeighted>
+// The number of rows of [lo, hi) that end before merge step `diag`: row r does when row_offsets[r + 1] + r + 1 <=
+// diag (merge_path_search with 64 rows tested at a time). Every lane of the wave calls it and gets lo plus that.
+__device__ __forceinline__ uint32_t wave_merge_search(const uint32_t* __restrict__ row_offsets, uint32_t lo, uint32_t hi,
+                                                      uint64_t diag) {
+    const uint32_t lane = lane_id();
+    while (lo < hi) {
+        const uint32_t stride = (hi - lo + kWave - 1) / kWave;
+        const uint32_t r = lo + lane * stride;
+        const bool ended = r < hi && static_cast<uint64_t>(row_offsets[r + 1]) + r + 1 <= diag;
+        const uint32_t k = static_cast<uint32_t>(__popcll(ballot(ended)));  // the first k lanes
+        if (k == 0) break;
+        const uint32_t next = lo + (k - 1) * stride + 1;  // row next - 1 ended
+        const uint32_t top = next - 1 + stride;           // row top, if tested, did not
+        lo = next;
+        if (top < hi) hi = top;
+    }
+    return __builtin_amdgcn_readfirstlane(lo);
+}
+
+// P: init(lane) once per wave; x<kWide>(u, lane) the lane's value of source u, loaded unconditionally (a
+// column the policy leaves out may read any valid element: its products are never stored); store(row, lane, y).
+template <typename S, bool kValues, bool kWide, typename P>
 __global__ void __launch_bounds__(256)
-spmm_plustimes_wave_kernel(uint32_t n_rows, uint32_t num_tiles, const uint32_t* __restrict__ row_offsets,
-                           const uint32_t* __restrict__ col, const float* __restrict__ vals,
-                           const MergeCoord* __restrict__ coords,
-                           SpmmTileRec<PlusTimesF32, 64>* __restrict__ recs, const float* __restrict__ X,
-                           float* __restrict__ Y) {
-    using S = PlusTimesF32;
-    using acc_t = S::acc_t;
-    __shared__ float s_x[4][kPprChunk][64];
+spmm_wave_kernel(uint32_t n_rows, const uint32_t* __restrict__ row_offsets,
+                 const uint32_t* __restrict__ col, const typename S::value_t* __restrict__ vals,
+                 const MergeCoord* __restrict__ coords, SpmmTileRec<S, 64>* __restrict__ recs, P pol) {
+    using acc_t = typename S::acc_t;
+    using value_t = typename S::value_t;
+    using x_t = typename S::x_t;
+    using y_t = typename S::y_t;
+    static_assert(sizeof(value_t) == 4, "values travel through readlane");
+    __shared__ acc_t s_carry[kMergeWaves][64];
+    __shared__ uint32_t s_ends[kMergeWaves];
+    __shared__ uint32_t s_row[kMergeWaves + 1];
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const uint32_t tile = blockIdx.x * 4u + wave;
-    if (tile >= num_tiles) return;
-    const uint32_t r0 = coords[tile].x, r_last = coords[tile + 1].x;
-    const uint32_t q0 = coords[tile].y, q1 = coords[tile + 1].y;
+    const uint32_t tile = blockIdx.x;
+    const MergeCoord c0 = coords[tile], c1 = coords[tile + 1];
+    pol.init(lane);
 
+    // the quarters' bounds: the merge-path search of the wave's first step, 64 rows at a time
+    const uint64_t step0 = static_cast<uint64_t>(c0.x) + c0.y, step1 = static_cast<uint64_t>(c1.x) + c1.y;
+    auto quarter = [&](uint32_t w) { return step0 + w * (kMergeTile / 4) < step1 ? step0 + w * (kMergeTile / 4) : step1; };
+    const uint32_t first = wave_merge_search(row_offsets, c0.x, c1.x, quarter(wave));
+    if (lane == 0) {
+        s_row[wave] = first;
+        if (wave == 0) s_row[kMergeWaves] = c1.x;
+    }
+    __syncthreads();
+    const uint32_t r0 = first, r_last = __builtin_amdgcn_readfirstlane(s_row[wave + 1]);
+    const uint32_t q0 = static_cast<uint32_t>(quarter(wave) - r0), q1 = static_cast<uint32_t>(quarter(wave + 1) - r_last);
+
+    // row ends of 64 consecutive rows, one per lane, read out with readlane
     uint32_t rbase = r0;
     uint32_t rwin = row_offsets[rbase + 1 + lane <= n_rows ? rbase + 1 + lane : n_rows];
     auto row_end = [&](uint32_t r) -> uint32_t {
@@ -959,101 +1028,166 @@ spmm_plustimes_wave_kernel(uint32_t n_rows, uint32_t num_tiles, const uint32_t* 
         return __builtin_amdgcn_readlane(rwin, r - rbase);
     };
 
-    uint32_t r = r0;                                    // next row to close
-    uint32_t re = r0 < r_last ? row_end(r0) : kInf;     // its end (kInf: no further row end in the tile)
-    uint32_t d = 0;                                     // merge steps done in the tile
+    uint32_t r = r0;                                 // next row to close
+    uint32_t re = r0 < r_last ? row_end(r0) : kInf;  // its end (kInf: no further row end in the tile)
+    // The nonzero before which the run ends unless a row closes first (each row closed is a step too).
+    uint32_t run = q0 + kMergeItems;
     acc_t acc = S::identity(), head = S::identity(), chain = S::identity();
     bool hasend = false, any_end = false;
     uint32_t first_row = 0;
+
+    acc_t part = S::identity();  // the first row the quarter closes, as far as the quarter holds it
+    uint32_t part_row = 0;
 
     // End of a run of 8 steps (the same folds as merge_walk's, per column).
     auto run_end = [&]() {
         if (hasend) {
             const acc_t whole = S::merge(chain, head);
-            if (!any_end && row_offsets[first_row] < q0) {
-                recs[tile].head[lane] = whole;
+            if (any_end) {
+                pol.store(first_row, lane, S::finalize(whole));
             } else {
-                Y[static_cast<size_t>(first_row) * 64 + lane] = S::finalize(whole);
+                part = whole;
+                part_row = first_row;
             }
-            chain = S::merge(S::identity(), acc);
+            chain = acc;
             any_end = true;
+            hasend = false;
         } else {
             chain = S::merge(chain, acc);
         }
         acc = S::identity();
-        head = S::identity();
-        hasend = false;
     };
-    auto step = [&]() {
-        ++d;
-        if ((d & (kMergeItems - 1)) == 0) run_end();
-    };
-    auto close_row = [&]() {
-        if (!hasend) {
-            head = acc;
-            hasend = true;
-            first_row = r;
-        } else {
-            Y[static_cast<size_t>(r) * 64 + lane] = S::finalize(acc);
+    // Every run and row that ends before nonzero q is added.
+    auto events = [&](uint32_t q) {
+        if (run == q) {
+            run_end();
+            run = q + kMergeItems;
         }
-        acc = S::identity();
-        ++r;
-        re = r < r_last ? row_end(r) : kInf;
-        step();
+        while (re <= q) {
+            if (!hasend) {
+                head = acc;
+                hasend = true;
+                first_row = r;
+            } else {
+                pol.store(r, lane, S::finalize(acc));
+            }
+            acc = S::identity();
+            ++r;
+            re = r < r_last ? row_end(r) : kInf;
+            if (--run == q) {
+                run_end();
+                run = q + kMergeItems;
+            }
+        }
     };
 
     if (q0 < q1) {
-        const uint32_t c_first = q0 / kPprChunk, c_end = (q1 + kPprChunk - 1) / kPprChunk;
-        auto load_cw = [&](uint32_t c, uint32_t& cv, uint32_t& wv) {
+        constexpr uint32_t kPer = 64 / kWaveChunk;  // chunks per block of indices
+        const uint32_t c_end = (q1 + kWaveChunk - 1) / kWaveChunk;
+        uint32_t c = q0 / kWaveChunk;
+        // a lane outside the tile's nonzeros holds source 0 (never folded)
+        auto load_block = [&](uint32_t b, uint32_t& cv, uint32_t& wv) {
+            const uint32_t q = b * 64u + lane;
             cv = 0;
-            wv = __float_as_uint(1.0f);
-            const uint32_t q = c * kPprChunk + lane;
-            if (lane < kPprChunk && q >= q0 && q < q1) {
-                cv = col[q];
-                if (kWeighted) wv = __float_as_uint(vals[q]);
+            wv = 0;
+            if (q >= q0 && q < q1) {
+                cv = __builtin_nontemporal_load(col + q);
+                if (kValues) wv = __builtin_bit_cast(uint32_t, __builtin_nontemporal_load(vals + q));
             }
         };
-        float xr[kPprChunk];
-        auto load_x = [&](uint32_t cv) {
+        x_t xn[kWaveChunk];
+        auto load_x = [&](uint32_t cv, uint32_t at) {
 #pragma unroll
-            for (uint32_t t = 0; t < kPprChunk; ++t) {
-                const uint32_t u = __builtin_amdgcn_readlane(cv, t);  // inactive lanes hold source 0
-                xr[t] = X[static_cast<size_t>(u) * 64 + lane];
-            }
+            for (uint32_t t = 0; t < kWaveChunk; ++t)
+                xn[t] = pol.template x<kWide>(__builtin_amdgcn_readlane(cv, at + t), lane);
         };
-        uint32_t colA, wA, colB = 0, wB = 0;
-        load_cw(c_first, colA, wA);
-        load_x(colA);
-        if (c_first + 1 < c_end) load_cw(c_first + 1, colB, wB);
-        for (uint32_t c = c_first; c < c_end; ++c) {
+        uint32_t cA, wA, cB, wB;
+        load_block(c / kPer, cA, wA);
+        load_block(c / kPer + 1, cB, wB);
+        load_x(cA, (c % kPer) * kWaveChunk);
+        for (; c < c_end; ++c) {
+            const uint32_t at = (c % kPer) * kWaveChunk;
+            y_t p[kWaveChunk];
 #pragma unroll
-            for (uint32_t t = 0; t < kPprChunk; ++t) s_x[wave][t][lane] = xr[t];
-            if (c + 1 < c_end) load_x(colB);
-            uint32_t colC = 0, wC = 0;
-            if (c + 2 < c_end) load_cw(c + 2, colC, wC);
-            const uint32_t qa = (q0 > c * kPprChunk) ? q0 : c * kPprChunk;
-            const uint32_t qb = (q1 < (c + 1) * kPprChunk) ? q1 : (c + 1) * kPprChunk;
-            for (uint32_t q = qa; q < qb; ++q) {
-                while (re <= q) close_row();
-                const uint32_t t = q - c * kPprChunk;
-                const float w = kWeighted ? __uint_as_float(__builtin_amdgcn_readlane(wA, t)) : 1.0f;
-                S::add(acc, S::combine(w, s_x[wave][t][lane]));
-                step();
+            for (uint32_t t = 0; t < kWaveChunk; ++t) {
+                value_t w = value_t(1);
+                if (kValues) w = __builtin_bit_cast(value_t, static_cast<uint32_t>(__builtin_amdgcn_readlane(wA, at + t)));
+                p[t] = S::combine(w, xn[t]);
             }
-            wA = wB;
-            colB = colC;
-            wB = wC;
+            if (at + kWaveChunk == 64u) {
+                cA = cB;
+                wA = wB;
+                load_x(cA, 0);
+                load_block((c + 1) / kPer + 1, cB, wB);
+            } else {
+                load_x(cA, at + kWaveChunk);  // past the tile's end: source 0's row, unused
+            }
+            const uint32_t qc = c * kWaveChunk;
+            if (qc < q0 || q1 - qc < kWaveChunk) {
+                // the tile's first or last chunk: products outside the tile fold as nothing
+                const uint32_t ta = q0 > qc ? q0 - qc : 0u;
+#pragma unroll
+                for (uint32_t t = 0; t < kWaveChunk; ++t)
+                    if (t < ta || qc + t >= q1) p[t] = S::nothing();
+            }
+            // next: the position of the first event in the chunk (none before q0; past q1 only ends of runs that
+            // add nothing)
+            auto upcoming = [&]() { return (re < run ? re : run) - qc; };
+            uint32_t next = upcoming();
+#pragma unroll
+            for (uint32_t t = 0; t < kWaveChunk; ++t) {
+                if (next <= t) {
+                    events(qc + t);
+                    next = upcoming();
+                }
+                S::add(acc, p[t]);
+            }
         }
     }
-    while (r < r_last) close_row();
-    // The runs after the tile's last step (the last tile only) are empty: their tails still join the chain.
-    if ((d & (kMergeItems - 1)) != 0) run_end();
-    for (uint32_t v = (d + kMergeItems - 1) / kMergeItems; v < static_cast<uint32_t>(kMergeThreads); ++v) run_end();
-    recs[tile].carry[lane] = chain;
-    if (lane == 0) {
-        uint32_t flags = any_end ? kTileHasEnd : 0u;
-        if (any_end && row_offsets[r0] < q0) flags |= kTileDeferred;
-        recs[tile].flags = flags;
+    events(q1);  // the rows left end at q1
+    run_end();
+
+    s_carry[wave][lane] = chain;
+    if (lane == 0) s_ends[wave] = any_end;
+    __syncthreads();
+    // The carries of the quarters before w since the last one that closed a row (merge_wave_chain).
+    auto outer = [&](int w, bool& any) {
+        int u = w - 1;
+        while (u > 0 && !s_ends[u]) --u;
+        any = u >= 0 && s_ends[u] != 0u;
+        acc_t sum = S::identity();
+        for (int v = u > 0 ? u : 0; v < w; ++v) sum = S::merge(sum, s_carry[v][lane]);
+        return sum;
+    };
+    bool before;
+    if (any_end) {
+        const acc_t whole = S::merge(outer(static_cast<int>(wave), before), part);
+        if (!before && row_offsets[part_row] < c0.y) recs[tile].head[lane] = whole;
+        else pol.store(part_row, lane, S::finalize(whole));
+    }
+    if (wave == kMergeWaves - 1) {
+        recs[tile].carry[lane] = outer(kMergeWaves, before);
+        if (lane == 0) {
+            uint32_t flags = before ? kTileHasEnd : 0u;
+            if (before && row_offsets[c0.x] < c0.y) flags |= kTileDeferred;
+            recs[tile].flags = flags;
+        }
+    }
+}
+
+// One pass of the wave kernel; x_bytes is the size of the x array the policy reads.
+template <typename S, typename P>
+inline void launch_spmm_wave(uint32_t n_rows, uint32_t tiles, const uint32_t* row_off, const uint32_t* col,
+                             const typename S::value_t* vals, const MergeCoord* coords, SpmmTileRec<S, 64>* recs,
+                             const P& pol, uint64_t x_bytes, hipStream_t s) {
+    const bool wide = x_bytes >= (1ull << 32);
+    auto go = [&](auto kernel) { kernel<<<tiles, 256, 0, s>>>(n_rows, row_off, col, vals, coords, recs, pol); };
+    if (vals) {
+        if (wide) go(spmm_wave_kernel<S, true, true, P>);
+        else go(spmm_wave_kernel<S, true, false, P>);
+    } else {
+        if (wide) go(spmm_wave_kernel<S, false, true, P>);
+        else go(spmm_wave_kernel<S, false, false, P>);
     }
 }
 

@@ -9,13 +9,15 @@
 // once per matrix (merge_partition_kernel, the reference's SegmentSearch run once in the dispatcher
 // constructor, include/GraphOne/archi/blas/spmv/cuda/cuda.cuh:89-91) and reused by every multiply.
 //
-// Fold order (what makes plus-times results reproducible): inside a thread a row's products are
-// added left to right; a row that crosses thread boundaries is finished by the thread that closes it
-// by merging, left to right, the tails of the threads before it back to the last thread that closed
-// a row; a row that crosses tiles is finished by the fixup kernel, which merges the carries of the
-// tiles it crosses, left to right, followed by the closing tile's head. The order therefore depends
-// only on the matrix and the constants below, never on scheduling, so repeated runs and the batched
-// SpMM (which uses the same partition) give the same bits.
+// Fold order (what makes plus-times results reproducible): inside a thread a row's products are added left
+// to right; the thread that first closes a row in its wave merges, left to right, the tails of the threads
+// before it back to the wave's start (or to the last thread that closed a row, for the later closers) and
+// then its own part; a row that crosses waves merges the carries of the waves it crosses, left to right, in
+// front of that; a row that crosses tiles is finished by the fixup kernel, which merges the carries of
+// the tiles it crosses, left to right, followed by the closing tile's head. The order therefore depends only
+// on the matrix and the constants below, never on scheduling, so repeated runs and the batched SpMM
+// (which folds a quarter of a tile where this folds a wave) give the same bits. Waves are a level of their
+// own because a quarter of a tile is then a piece of work that the SpMM can give to a wave.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -165,18 +167,6 @@ __device__ __forceinline__ void merge_to_lds(const MergeStage<S>& st, uint32_t* 
     if (tid == 0) s_rowend[rows] = kInf;  // no further row end inside this tile
 }
 
-// The last thread below t that closed a row (-1 if none), from the waves' ballots of the closing threads
-// (masks[2w], masks[2w + 1]: the 64 flags of wave w): at most kMergeThreads / 64 words read.
-__device__ __forceinline__ int merge_last_end_before(const uint32_t* masks, uint32_t t) {
-    for (int w = static_cast<int>((t - 1) / kWave); t > 0 && w >= 0; --w) {
-        uint64_t m = (static_cast<uint64_t>(masks[2 * w + 1]) << 32) | masks[2 * w];
-        const uint32_t below = t - static_cast<uint32_t>(w) * kWave;  // flags of lanes < below count
-        if (below < static_cast<uint32_t>(kWave)) m &= (1ull << below) - 1ull;
-        if (m) return w * kWave + 63 - __clzll(m);
-    }
-    return -1;
-}
-
 // The left-to-right fold of the tails of threads [v0, v1): the loads issued eight at a time ahead of their
 // merges, so a fold across a long row does not wait on each LDS read in turn (same order, same result).
 template <typename S>
@@ -195,6 +185,21 @@ __device__ __forceinline__ typename S::acc_t merge_fold_tails(const typename S::
     return chain;
 }
 
+constexpr int kMergeWaves = kMergeThreads / kWave;
+
+// The carry into wave w from the waves before it in the tile: their carries since the last wave below w
+// that closed a row (carries begin there), left to right.
+template <typename S>
+__device__ __forceinline__ typename S::acc_t merge_wave_chain(const typename S::acc_t* s_carry, const uint32_t* s_ends,
+                                                              int w, bool& any) {
+    int u = w - 1;
+    while (u > 0 && !s_ends[u]) --u;
+    any = u >= 0 && s_ends[u] != 0u;
+    typename S::acc_t chain = S::identity();
+    for (int v = u > 0 ? u : 0; v < w; ++v) chain = S::merge(chain, s_carry[v]);
+    return chain;
+}
+
 // The walk of one staged tile (LDS filled, after a barrier): each thread's kMergeItems steps, the rows
 // it closes, the tails chain, and the tile record. Contains one barrier; every thread must call it.
 template <typename S>
@@ -202,7 +207,7 @@ __device__ __forceinline__ void merge_walk(uint32_t tile, MergeCoord c0, MergeCo
                                            const uint32_t* __restrict__ row_offsets, typename S::y_t* __restrict__ y,
                                            MergeTileRec<S>* __restrict__ recs, const uint32_t* s_rowend,
                                            const typename S::y_t* s_prod, typename S::acc_t* s_tail,
-                                           uint32_t* s_hasend) {
+                                           typename S::acc_t* s_carry, uint32_t* s_ends) {
     using acc_t = typename S::acc_t;
     const uint32_t tid = threadIdx.x;
     const uint32_t rows = c1.x - c0.x;
@@ -245,33 +250,42 @@ __device__ __forceinline__ void merge_walk(uint32_t tile, MergeCoord c0, MergeCo
         }
     }
     s_tail[tid] = acc;
-    // which threads closed a row: one 64-bit ballot per wave, as two words (s_hasend[2w], s_hasend[2w + 1])
+    // A wave's tails are read by that wave only: its LDS operations run in program order, which the compiler
+    // must keep too.
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
     const uint64_t ends = ballot(hasend);
-    if (lane_id() == 0) {
-        s_hasend[2 * (tid / kWave)] = static_cast<uint32_t>(ends);
-        s_hasend[2 * (tid / kWave) + 1] = static_cast<uint32_t>(ends >> 32);
+    const uint32_t lane = lane_id();
+    const int w = static_cast<int>(tid / kWave);
+    const uint32_t w0 = static_cast<uint32_t>(w) * kWave;
+    const uint64_t below = ends & ((1ull << lane) - 1ull);
+    acc_t part = S::identity();  // the row a thread closes first, as far as this wave holds it
+    if (hasend) {
+        const acc_t chain = merge_fold_tails<S>(s_tail, below ? w0 + 63u - __clzll(below) : w0, tid);
+        part = S::merge(chain, head);
+        if (below) y[first_row] = S::finalize(part);
+    }
+    if (lane == kWave - 1) {
+        s_carry[w] = merge_fold_tails<S>(s_tail, ends ? w0 + 63u - __clzll(ends) : w0, w0 + kWave);
+        s_ends[w] = ends != 0ull;
     }
     __syncthreads();
 
-    if (hasend) {
-        const int u = merge_last_end_before(s_hasend, tid);
-        const acc_t chain = merge_fold_tails<S>(s_tail, u >= 0 ? static_cast<uint32_t>(u) : 0u, tid);
-        const acc_t whole = S::merge(chain, head);
+    if (hasend && !below) {
+        bool any;
+        const acc_t chain = merge_wave_chain<S>(s_carry, s_ends, w, any);
+        const acc_t whole = S::merge(chain, part);
         // The tile's first closed row began in an earlier tile: leave it for the fixup kernel.
-        if (u < 0 && row_offsets[first_row] < c0.y) {
-            recs[tile].head = whole;
-        } else {
-            y[first_row] = S::finalize(whole);
-        }
+        if (!any && row_offsets[first_row] < c0.y) recs[tile].head = whole;
+        else y[first_row] = S::finalize(whole);
     }
     if (tid == kMergeThreads - 1) {
-        const int u = merge_last_end_before(s_hasend, kMergeThreads);
-        const acc_t carry = merge_fold_tails<S>(s_tail, u >= 0 ? static_cast<uint32_t>(u) : 0u, kMergeThreads);
-        recs[tile].carry = carry;
-        uint32_t flags = (u >= 0) ? kTileHasEnd : 0u;
+        bool any;
+        recs[tile].carry = merge_wave_chain<S>(s_carry, s_ends, kMergeWaves, any);
+        uint32_t flags = any ? kTileHasEnd : 0u;
         // Deferred exactly when the tile's first closed row (row c0.x) began in an earlier tile; the
         // first closing thread made the same test above and stored its head instead of writing y.
-        if (u >= 0 && row_offsets[c0.x] < c0.y) flags |= kTileDeferred;
+        if (any && row_offsets[c0.x] < c0.y) flags |= kTileDeferred;
         recs[tile].flags = flags;
     }
 }
@@ -288,14 +302,15 @@ spmv_merge_tile_kernel(uint32_t n_rows, uint32_t nnz, const uint32_t* __restrict
     __shared__ uint32_t s_rowend[kMergeTile + 1];
     __shared__ y_t s_prod[kMergeTile];
     __shared__ acc_t s_tail[kMergeThreads];
-    __shared__ uint32_t s_hasend[kMergeThreads];
+    __shared__ acc_t s_carry[kMergeWaves];
+    __shared__ uint32_t s_ends[kMergeWaves];
     const uint32_t tile = blockIdx.x;
     MergeStage<S> st;
     merge_load_index<S, kHasValues>(tile, row_offsets, col, vals, coords, st);
     merge_load_x<S>(x, st);
     merge_to_lds<S>(st, s_rowend, s_prod);
     __syncthreads();
-    merge_walk<S>(tile, st.c0, st.c1, row_offsets, y, recs, s_rowend, s_prod, s_tail, s_hasend);
+    merge_walk<S>(tile, st.c0, st.c1, row_offsets, y, recs, s_rowend, s_prod, s_tail, s_carry, s_ends);
 }
 
 // One thread per tile: finish the first closed row of every deferred tile by folding, left to right,

@@ -282,6 +282,20 @@ struct StridedColumnsPolicy {
     uint32_t kc;  // columns in the chunk (<= 64)
     const unsigned long long* mask;
     T neutral;    // what a skipped column reads (the semiring's absorbing x: INF for min-plus, 0 for plus-times)
+    uint32_t jc = 0;    // spmm_wave_kernel: the column this lane reads (its own, or 0 when it stores nothing)
+    bool mine = false;
+    __device__ __forceinline__ void init(uint32_t j) {
+        mine = on(j);
+        jc = mine ? c0 + j : 0u;
+    }
+    template <bool kWide>
+    __device__ __forceinline__ T x(uint32_t u, uint32_t) const {
+        if constexpr (kWide) return X[static_cast<size_t>(u) * ld + jc];
+        return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(X) + (u * (ld * 4u) + jc * 4u));
+    }
+    __device__ __forceinline__ void store(uint32_t row, uint32_t, T y) const {
+        if (mine) Y[static_cast<size_t>(row) * ld + jc] = y;
+    }
     __device__ __forceinline__ bool on(uint32_t j) const {
         return j < kc && (!mask || ((mask[(c0 + j) >> 6] >> ((c0 + j) & 63u)) & 1ull));
     }

@@ -278,3 +278,71 @@ def test_spmm_minplus_and_plustimes(gpu, k):
     for j in range(0, k, max(1, k // 8)):
         want = oracle.spmv_plustimes_f64(t.row_offsets, t.col_indices, wf.astype(np.float64), Xf[:, j].astype(np.float64))
         assert np.allclose(Yf[:, j], want, rtol=2e-6, atol=1e-30), j
+
+
+@pytest.mark.parametrize("degs, k", [
+    ([0], 3), ([1], 64), ([511], 64), ([255, 255], 65), ([512, 0, 0], 64), ([0] * 700, 5), ([2047], 64), ([2048], 64),
+    ([0, 0, 5000, 0, 1, 700, 3], 64), ([7] * 900, 64), ([0, 1] * 1500, 128), ([16] * 31 + [0], 64)])
+def test_spmm_tile_edges(gpu, degs, k):
+    """Rows and nonzeros around the steps that the SpMM is cut at (runs of 8, chunks of 16, quarters of 512, tiles of
+    2048 steps): rows that end on a cut, span several, or hold nothing, columns past one pass of 64, with and
+    without values. Min-plus is exact. Plus-times products are rounded to 32 bits and so is the sum: at most
+    2^-24 of the terms' magnitudes and of the result, so 2^-23 of the magnitudes. Source 0 holds an infinity that
+    no row but its own readers may see."""
+    g1 = _g1()
+    rng = np.random.default_rng(len(degs) + k)
+    n_rows, n_cols = len(degs), 6000
+    rp = np.concatenate([[0], np.cumsum(degs)]).astype(np.uint32)
+    m = int(rp[-1])
+    ci = rng.integers(1, n_cols, m).astype(np.uint32)
+    w = rng.integers(1, 90, m).astype(np.uint32)
+    rows = np.repeat(np.arange(n_rows), degs)
+    wsb = g1._lib.lib().g1_spmm_workspace_bytes(n_rows, m)
+    ws = g1.DeviceArray((wsb + 3) // 4 + 1, np.uint32)
+    drp, dci, dw, dwf = _dev(rp), _dev(np.append(ci, 0).astype(np.uint32)), _dev(np.append(w, 0).astype(np.uint32)), _dev(np.append(w, 0).astype(np.float32))
+    X = rng.integers(0, 1000, (n_cols, k)).astype(np.uint32)
+    X[rng.random((n_cols, k)) < 0.3] = INF
+    Xf = rng.standard_normal((n_cols, k)).astype(np.float32)
+    Xf[0] = np.inf
+    dX, dXf = _dev(X), _dev(Xf)
+    for values in (True, False):
+        dY, dYf = g1.DeviceArray(n_rows * k, np.uint32), g1.DeviceArray(n_rows * k, np.float32)
+        _call("g1_spmm_minplus_u32", n_rows, n_cols, m, k, _p(drp), _p(dci), _p(dw) if values else None, _p(dX), _p(dY),
+              None, _p(ws), C.c_size_t(wsb), None)
+        _call("g1_spmm_plustimes_f32", n_rows, n_cols, m, k, _p(drp), _p(dci), _p(dwf) if values else None, _p(dXf),
+              _p(dYf), None, _p(ws), C.c_size_t(wsb), None)
+        wv = w.astype(np.int64) if values else np.ones(m, np.int64)
+        far = 1 << 40
+        want = np.full((n_rows, k), far, np.int64)
+        np.minimum.at(want, rows, np.where(X[ci] == INF, far, X[ci].astype(np.int64) + wv[:, None]))
+        assert np.array_equal(dY.numpy().reshape(n_rows, k), np.where(want >= far, INF, want).astype(np.uint32))
+        p = Xf[ci].astype(np.float64) * wv[:, None]
+        sums, sizes = np.zeros((n_rows, k)), np.zeros((n_rows, k))
+        np.add.at(sums, rows, p)
+        np.add.at(sizes, rows, np.abs(p))
+        assert np.all(np.abs(dYf.numpy().reshape(n_rows, k) - sums) <= sizes * 2.0 ** -23)
+
+
+def test_spmm_x_past_4_gib(gpu):
+    """An X of more than 2^32 bytes: the sources' rows are reached with 64-bit offsets."""
+    g1 = _g1()
+    n_cols, k = (1 << 24) + 3, 64
+    ci = np.array([0, n_cols - 1, 5, (1 << 24) + 1, n_cols - 1], np.uint32)
+    rp = np.array([0, 2, 2, 5], np.uint32)
+    w = np.arange(1, 6, dtype=np.float32)
+    dX = g1.DeviceArray(n_cols * k, np.float32)
+    dX.fill(0.0)
+    L = g1._lib
+    for c in set(ci.tolist()):
+        row = (np.arange(k, dtype=np.float32) + 1) * (1 + c % 7)
+        L.call("g1_memcpy_h2d", C.c_void_p(dX.ptr + c * k * 4), row.ctypes.data_as(C.c_void_p), C.c_size_t(k * 4), None)
+    dY = g1.DeviceArray(3 * k, np.float32)
+    wsb = L.lib().g1_spmm_workspace_bytes(3, 5)
+    ws = g1.DeviceArray((wsb + 3) // 4, np.uint32)
+    drp, dci, dw = _dev(rp), _dev(ci), _dev(w)
+    _call("g1_spmm_plustimes_f32", 3, n_cols, 5, k, _p(drp), _p(dci), _p(dw), _p(dX), _p(dY), None, _p(ws),
+          C.c_size_t(wsb), None)
+    base = np.arange(k) + 1.0
+    f = [1 + int(c) % 7 for c in ci]
+    want = np.stack([base * (f[0] + 2 * f[1]), 0 * base, base * (3 * f[2] + 4 * f[3] + 5 * f[4])])
+    assert np.array_equal(dY.numpy().reshape(3, k), want.astype(np.float32))  # small whole numbers: exact
