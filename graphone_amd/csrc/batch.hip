@@ -477,7 +477,7 @@ g1_status ppr_tile_run(g1_graph* g, BatchWork* b, const uint32_t* seeds_host, ui
     // An iteration after every column froze changes nothing (frozen columns copy R into the other buffer).
     auto iteration = [&](int cur, hipStream_t st) -> g1_status {
         G1_TRY(launch_plustimes<K>(g, b->X, b->Y, b->recs, st));
-        rank_apply_batch_kernel<K><<<(nb + 256 / K - 1) / (256 / K), 256, 0, st>>>(
+        rank_apply_batch_kernel<K><<<rank_apply_grid<K>(nb), 256, 0, st>>>(
             n, b->Y, 0.0f, g->seeds_dev, restart, g->iw, b->R[cur], b->R[cur ^ 1], b->X, g->rpart, nb, 0ull, state);
         G1_LAUNCHED();
         reduce_partials_kernel<0><<<dim3(1, K), 256, 0, st>>>(g->rpart, nb, g->rpart + static_cast<size_t>(nb) * kBatchCols);
@@ -814,7 +814,7 @@ g1_status session_step_ppr(Session* ss, uint64_t* done) {
     const hipStream_t s = ss->s;
     G1_TRY(launch_plustimes<K>(g, ss->X, ss->Y, ss->recs, s));
     const unsigned long long live = ss->active & ~ss->converged;
-    rank_apply_batch_kernel<K><<<(nb + 256 / K - 1) / (256 / K), 256, 0, s>>>(
+    rank_apply_batch_kernel<K><<<rank_apply_grid<K>(nb), 256, 0, s>>>(
         n, ss->Y, 0.0f, ss->seeds_dev, ss->restart, ss->iw, ss->R[ss->rcur], ss->R[ss->rcur ^ 1], ss->X, ss->part, nb,
         ~live, nullptr);
     G1_LAUNCHED();

@@ -961,7 +961,7 @@ struct PlusTimesBatchPolicy {
 // a time, a block ahead, and are read out of their lanes. Measured: 16 M nonzeros x 64 columns
 // 1.03 ms with the round-based tile kernel, 0.66 ms here (6.5 TB/s of x rows; 0.88 ms with a wave per tile, 0.85 ms
 // with the run counter and the 64-bit row addresses on the scalar unit as well, 19 scalar instructions a
-// nonzero against 8); 11 M nonzeros of a PPR batch 0.70 ms with x parked in LDS and a wave per tile, 0.40 ms.
+// nonzero against 8); 11 M nonzeros of a PPR batch 0.72 ms with x parked in LDS and a wave per tile, 0.38 ms.
 constexpr uint32_t kWaveChunk = 16;
 static_assert(64 % kWaveChunk == 0, "a block of 64 indices holds whole chunks");
 
