@@ -112,22 +112,7 @@ uint32_t fill_blocks(size_t items) {
 // Words of the k = 64 activity bitmap (act_bits_kernel): two per 64 vertices.
 size_t act_words(size_t n) { return 2 * ((n + 63) / 64) + 2; }
 
-// The row-start bitmap of the in-edge CSR used by the k = 64 min-plus kernel; built once per graph
-// (caller holds g->mu), finished before it returns so any stream may use it.
-g1_status ensure_row_starts(g1_graph* g, hipStream_t s) {
-    if (g->t_starts || !g->has_t) return G1_OK;
-    const size_t words = (static_cast<size_t>(g->m) >> 6) + 2;
-    G1_TRY(alloc_n(g, &g->t_starts, words));
-    G1_TRY(g1_fill_u32(reinterpret_cast<uint32_t*>(g->t_starts), 0u, 2 * words, reinterpret_cast<g1_stream_t>(s)));
-    if (g->n) {
-        row_starts_kernel<<<fill_blocks(g->n), 256, 0, s>>>(g->n, g->t_row_off, g->t_starts);
-        G1_LAUNCHED();
-    }
-    G1_HIP(hipStreamSynchronize(s));
-    return G1_OK;
-}
-
-// Merge tiles (rows + nonzeros per wavefront) the autotuner tries for the k = 64 min-plus kernel. Min is
+// Merge tiles (rows + nonzeros per workgroup) the autotuner tries for the k = 64 min-plus kernel. Min is
 // order-free, so every partition gives the same bits; [kWaveTileOwn] is the graph's own partition (t_ws), shared
 // with the single-source SpMV and the plus-times kernels, whose fold order it fixes.
 constexpr uint32_t kWaveTileItems[kWaveTileCount] = {kMergeTile / 4, kMergeTile / 2, kMergeTile, kMergeTile * 2};
@@ -170,7 +155,6 @@ g1_status ensure_batch(g1_graph* g, uint32_t K, bool ppr, BatchWork** out, hipSt
         b->recs = v;
         G1_TRY(alloc_n(g, &b->changed, 64));
     }
-    if (!ppr && K == 64) G1_TRY(ensure_row_starts(g, s));
     if (!ppr && !b->D) {
         G1_TRY(alloc_n(g, &b->D, (n + 1) * K));  // row n: all unreached (read for inactive sources)
         G1_TRY(alloc_n(g, &b->mask[0], n));
@@ -319,21 +303,17 @@ g1_status launch_minplus(g1_graph* g, DT* D, unsigned long long* mask_prev, unsi
                 coords = static_cast<const MergeCoord*>(g->wave_coords[tile_idx]);
                 fix_blocks = static_cast<uint32_t>((static_cast<uint64_t>(tiles) * K + 255) / 256);
             }
-            const uint32_t blocks = (tiles + 3) / 4;
-            G1_CHECK(g->t_starts != nullptr && act != nullptr, G1_ERR_INTERNAL,
-                     "min-plus k = 64: row-start or activity bitmap missing");
+            G1_CHECK(act != nullptr, G1_ERR_INTERNAL, "min-plus k = 64: activity bitmap missing");
             // The wavefront kernel writes only non-zero change masks, and reads activity as a bitmap.
             G1_TRY(g1_fill_u32(reinterpret_cast<uint32_t*>(mask_next), 0u, 2ull * g->n, reinterpret_cast<g1_stream_t>(s)));
             act_bits_kernel<<<fill_blocks(static_cast<size_t>(g->n) / 4 + 64), 256, 0, s>>>(g->n, mask_prev, act);
             G1_LAUNCHED();
-            if (weighted)
-                spmm_minplus_wave_kernel<true, DT><<<blocks, 256, 0, s>>>(g->n, tiles, g->t_row_off, g->t_col, vals,
-                                                                          g->t_starts, coords, recs, D, act,
-                                                                          mask_next, flag, overflow);
-            else
-                spmm_minplus_wave_kernel<false, DT><<<blocks, 256, 0, s>>>(g->n, tiles, g->t_row_off, g->t_col, vals,
-                                                                           g->t_starts, coords, recs, D, act,
-                                                                           mask_next, flag, overflow);
+            auto go = [&](auto kernel) {
+                kernel<<<tiles, 256, 0, s>>>(g->n, kWaveTileItems[tile_idx], g->t_row_off, g->t_col, vals, coords, recs, D,
+                                             act, mask_next, flag, overflow);
+            };
+            if (weighted) go(spmm_minplus_wave_kernel<true, DT>);
+            else go(spmm_minplus_wave_kernel<false, DT>);
             G1_LAUNCHED();
             if (tiles > 1) {
                 if constexpr (sizeof(DT) == 2) {
@@ -890,7 +870,6 @@ g1_status session_create(g1_graph* g, int kind, uint32_t k, float restart, hipSt
     {
         std::lock_guard<std::mutex> lock(g->mu);  // lazily built graph arrays
         if (kind == kSessPpr) G1_TRY(ensure_pull_work(g, true));  // float weights, out-weight sums
-        else if (k == 64) G1_TRY(ensure_row_starts(g, stream));
     }
     Session* ss = new Session();
     ss->g = g;

@@ -30,7 +30,6 @@ struct g1_graph {
     bool t_alias = false;
     void* t_ws = nullptr;  // merge-path partition of the in-edge CSR
     size_t t_ws_bytes = 0;
-    unsigned long long* t_starts = nullptr;  // bitmap of in-edge CSR row starts (lazy, batched min-plus)
 
     // plain PageRank over the vertices relabelled hub first (lazy, ensure_pr_relabel): new id i is old id
     // pr_perm[i]; the in-edge CSR, its weights, the out-weight sums and the merge partition in the new ids

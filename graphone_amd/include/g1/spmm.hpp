@@ -574,40 +574,56 @@ __global__ void __launch_bounds__(256) spmm_fixup_kernel(uint32_t num_tiles, con
 }
 
 // ------------------------------------------------------------------------------------------------
-// Min-plus SpMM at k = 64 with one wavefront per merge-path tile: lane j owns column j.
+// x rows that a wave of the 64-column kernels below keeps in flight.
+constexpr uint32_t kWaveChunk = 16;
+static_assert(64 % kWaveChunk == 0, "a block of 64 indices holds whole chunks");
+
+// The number of rows of [lo, hi) that end before merge step `diag`: row r does when row_offsets[r + 1] + r + 1 <=
+// diag (merge_path_search with 64 rows tested at a time). Every lane of the wave calls it and gets lo plus that.
+__device__ __forceinline__ uint32_t wave_merge_search(const uint32_t* __restrict__ row_offsets, uint32_t lo, uint32_t hi,
+                                                      uint64_t diag) {
+    const uint32_t lane = lane_id();
+    while (lo < hi) {
+        const uint32_t stride = (hi - lo + kWave - 1) / kWave;
+        const uint32_t r = lo + lane * stride;
+        const bool ended = r < hi && static_cast<uint64_t>(row_offsets[r + 1]) + r + 1 <= diag;
+        const uint32_t k = static_cast<uint32_t>(__popcll(ballot(ended)));  // the first k lanes
+        if (k == 0) break;
+        const uint32_t next = lo + (k - 1) * stride + 1;  // row next - 1 ended
+        const uint32_t top = next - 1 + stride;           // row top, if tested, did not
+        lo = next;
+        if (top < hi) hi = top;
+    }
+    return __builtin_amdgcn_readfirstlane(lo);
+}
+
+// Min-plus SpMM at k = 64: a workgroup of four waves takes a merge-path tile, a wave a quarter of its merge
+// steps, lane j owns column j.
 //
-// The tile's nonzeros are taken in chunks of 64 aligned to multiples of 64 (lane t <-> nonzero
-// 64c + t): one coalesced load brings the chunk's column indices and weights, one gather the change
-// masks of their sources. A source whose mask is empty costs nothing more; for an active one the wave
-// reads its index and mask out of the lane that holds them (readlane) and loads the source's 64
-// distances with one 256-byte access, the lanes of the unchanged columns masked off. The loads of chunk
-// c + 1 (masks) and c + 2 (indices) are issued before those of chunk c, so they are in flight while
-// chunk c is folded. Row boundaries inside a chunk come from a per-graph bitmap of row starts (bit q:
-// a non-empty row begins at nonzero q): the fold keeps one running minimum and, at each boundary, parks
-// the finished row's 64 values in LDS; the rows are then applied in order (d = min(d, y), the columns
-// that improved go to mask_next). A chunk with more boundaries than the LDS slots is folded in parts.
+// A wave takes its merge steps (nonzeros and row ends, in merge order) 64 at a time, a lane each: the lane of a
+// nonzero holds its source and weight, the lane of a row end holds the row. The steps that are row ends are one
+// 64-bit mask: the ends of the next 64 rows, loaded a lane each, say which lanes they fall on. A source that
+// did not change last iteration is replaced by row n, which is never reached, and so is a row none of whose
+// nonzeros in the block can lower it; a block without any is stepped over. The distances of a nonzero's
+// source and the old distances of a row end are then the same load of 64 columns, sixteen in flight while the
+// sixteen before them fold: a nonzero adds its weight and takes the minimum, a row end (weight 0) compares the
+// minimum with its old distances, stores what improved and starts the next row. So a step costs two reads of
+// a lane, an address, an add and a minimum, and two scalar instructions; what bounds it is the 128 bytes of
+// distances it loads. Activity and indices of the next block load while a block folds.
+// Measured on 2.1 M vertices, 33 M edges, 16-bit distances: a dense iteration 1.25 -> 0.69 ms (6.6 TB/s of
+// distance rows, the old ones with them), the batch 15.9 -> 9.2 ms, against a wave per tile that loaded 64
+// sources' rows, folded them around a bitmap of row starts and then loaded the old rows of what it closed. An
+// iteration with next to no active source takes 0.15 ms for its indices and activity (0.11 ms before).
 //
-// The column and weight arrays must be readable up to the next multiple of 64 past the last nonzero
-// (the graph keeps kCsrPad = 64 padding entries).
-//
-// Min is order-free, so the result does not depend on how rows are cut into tiles or chunks; rows that
+// Min is order-free, so the result does not depend on how rows are cut into tiles, quarters or blocks; rows that
 // cross tiles leave head / carry records in the SpmmTileRec layout and are finished by spmm_fixup_kernel
 // with MinPlusBatchPolicy<64>, as for the other min-plus kernels. Distances are updated in place (a
 // source row read during the iteration may already hold this iteration's smaller value): each column
 // still decreases monotonically to the same fixed point, and an iteration with no change ends the run.
-constexpr uint32_t kWaveStage = 16;  // finished rows parked per fold part
-constexpr uint32_t kCloseBatch = 4;  // rows applied together (their old distances loaded together)
-
-// Bit q of starts[q >> 6]: a non-empty row of the CSR begins at nonzero q. starts has (nnz >> 6) + 2
-// words and must be zero on entry.
-static __global__ void __launch_bounds__(256) row_starts_kernel(uint32_t n_rows, const uint32_t* __restrict__ row_offsets,
-                                                         unsigned long long* __restrict__ starts) {
-    for (uint32_t r = blockIdx.x * 256 + threadIdx.x; r < n_rows; r += gridDim.x * 256) {
-        const uint32_t b = row_offsets[r];
-        if (row_offsets[r + 1] > b) atomicOr(&starts[b >> 6], 1ull << (b & 63u));
-    }
-}
-
+// Every column of an active source is relaxed: a column whose distance did not change last iteration was
+// relaxed through this edge when it last changed, so it cannot improve the row now, and the result (a fixed
+// point of min) is the same.
+//
 // Distances are stored as DT: uint32_t, or int16_t when every finite distance of the run is below
 // kCompactLimit (then a source row is one 128-byte line instead of two). 16-bit storage is exact or
 // void: -1 is the unreached distance, so a sign-extending load yields G1_INF for it and the distance
@@ -637,216 +653,171 @@ static __global__ void __launch_bounds__(256) act_bits_kernel(uint32_t n, const 
 }
 
 template <bool kWeighted, typename DT>
-__global__ void __launch_bounds__(256, 5)  // five waves per SIMD: at most 96 VGPRs
-spmm_minplus_wave_kernel(uint32_t n_rows, uint32_t num_tiles, const uint32_t* __restrict__ row_offsets,
+__global__ void __launch_bounds__(256)
+spmm_minplus_wave_kernel(uint32_t n_rows, uint32_t tile_items, const uint32_t* __restrict__ row_offsets,
                          const uint32_t* __restrict__ col, const uint32_t* __restrict__ vals,
-                         const unsigned long long* __restrict__ starts, const MergeCoord* __restrict__ coords,
-                         SpmmTileRec<MinPlusU32, 64>* __restrict__ recs, DT* __restrict__ D,
-                         const uint32_t* __restrict__ act_prev, unsigned long long* __restrict__ mask_next,
-                         unsigned long long* __restrict__ changed, uint32_t* __restrict__ overflow) {
-    __shared__ uint32_t s_stage[4][kWaveStage][64];
+                         const MergeCoord* __restrict__ coords, SpmmTileRec<MinPlusU32, 64>* __restrict__ recs,
+                         DT* __restrict__ D, const uint32_t* __restrict__ act_prev,
+                         unsigned long long* __restrict__ mask_next, unsigned long long* __restrict__ changed,
+                         uint32_t* __restrict__ overflow) {
+    __shared__ uint32_t s_mark[kMergeWaves][64];
+    __shared__ uint32_t s_carry[kMergeWaves][64];
+    __shared__ uint32_t s_ends[kMergeWaves];
+    __shared__ uint32_t s_row[kMergeWaves + 1];
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const uint32_t tile = blockIdx.x * 4u + wave;
-    if (tile >= num_tiles) return;
-    const uint32_t r0 = coords[tile].x, r_last = coords[tile + 1].x;  // rows [r0, r_last) end in the tile
-    const uint32_t q0 = coords[tile].y, q1 = coords[tile + 1].y;      // nonzeros [q0, q1)
-    const bool deferred = r0 < r_last && row_offsets[r0] < q0;         // the first row began before the tile
-
-    // Row ends of 64 consecutive rows, one per lane, read out with readlane.
-    uint32_t rbase = r0;
-    uint32_t rwin = row_offsets[rbase + 1 + lane <= n_rows ? rbase + 1 + lane : n_rows];
-    auto row_end = [&](uint32_t r) -> uint32_t {
-        if (r - rbase >= 64u) {
-            rbase = r;
-            rwin = row_offsets[rbase + 1 + lane <= n_rows ? rbase + 1 + lane : n_rows];
-        }
-        return __builtin_amdgcn_readlane(rwin, r - rbase);
-    };
-
-    uint32_t r = r0;
-    uint32_t rs = r0 < r_last ? row_offsets[r0] : 0u;  // start of row r
-    uint32_t re = r0 < r_last ? row_end(r0) : kInf;    // end of row r (kInf: the tile's open tail)
-    uint32_t acc = kInf;                               // running minimum of the open row
-    uint64_t counted = 0;
-
-    // Closes every row that ends at or before nonzero position lim, kCloseBatch rows at a time: the old
-    // distances of a batch are loaded together, then the rows are applied in order (d = min(d, y), the
-    // columns that improved go to mask_next; the deferred first row goes to the tile record). A non-empty
-    // row that ends before lim was parked in the next LDS slot; the one that ends at lim is the open
-    // minimum; an empty row (or every row when all_inf) is unreached.
-    auto close_upto = [&](uint32_t lim, bool all_inf) {
-        if (all_inf) {
-            // Every row closing here is unreached: nothing to relax and nothing to record (mask_next is
-            // cleared before the launch), so whole runs of rows are stepped over through the row-end
-            // window; only a deferred first row leaves its (unreached) head.
-            if (r == r0 && deferred && re <= lim) {
-                recs[tile].head[lane] = MinPlusU32::acc_t{kInf};
-                rs = re;
-                ++r;
-                re = r < r_last ? row_end(r) : kInf;
-            }
-            while (re <= lim) {
-                const uint32_t off = r - rbase;  // < 64: row_end(r) refilled the window
-                const uint32_t run = static_cast<uint32_t>(__popcll(ballot(lane >= off && rwin <= lim)));
-                uint32_t last = r + (run ? run : 1u) - 1u;
-                if (last >= r_last) last = r_last - 1u;
-                rs = row_end(last);
-                r = last + 1u;
-                re = r < r_last ? row_end(r) : kInf;
-            }
-            return;
-        }
-        uint32_t k = 0;  // next LDS slot
-        while (re <= lim) {
-            uint32_t rid[kCloseBatch], src[kCloseBatch], slot[kCloseBatch];  // src: 0 none, 1 unreached, 2 slot, 3 open
-            uint32_t open_val = kInf;
-#pragma unroll
-            for (uint32_t b = 0; b < kCloseBatch; ++b) {
-                src[b] = 0;
-                rid[b] = 0;
-                slot[b] = 0;
-                if (re <= lim) {
-                    rid[b] = r;
-                    if (re == rs || all_inf) {
-                        src[b] = 1;
-                    } else if (re < lim) {
-                        src[b] = 2;
-                        slot[b] = k++;
-                    } else {
-                        src[b] = 3;
-                        open_val = acc;
-                        acc = kInf;
-                    }
-                    rs = re;
-                    ++r;
-                    re = r < r_last ? row_end(r) : kInf;
-                }
-            }
-            uint32_t old[kCloseBatch];
-#pragma unroll
-            for (uint32_t b = 0; b < kCloseBatch; ++b) {
-                old[b] = kInf;
-                if (src[b] >= 2 && !(rid[b] == r0 && deferred))
-                    old[b] = widen_dist<DT>(D[static_cast<size_t>(rid[b]) * 64 + lane]);
-            }
-#pragma unroll
-            for (uint32_t b = 0; b < kCloseBatch; ++b) {
-                if (src[b] == 0) continue;
-                const uint32_t val = src[b] == 2 ? s_stage[wave][slot[b]][lane] : (src[b] == 3 ? open_val : kInf);
-                if (rid[b] == r0 && deferred) {
-                    recs[tile].head[lane] = MinPlusU32::acc_t{val};
-                    continue;
-                }
-                const bool improved = val < old[b];
-                if (improved) {
-                    if (sizeof(DT) == 2 && val >= kCompactLimit) *overflow = 1u;
-                    else D[static_cast<size_t>(rid[b]) * 64 + lane] = static_cast<DT>(val);
-                }
-                const uint64_t bits = ballot(improved);
-                if (lane == 0 && bits) mask_next[rid[b]] = bits;  // cleared before the launch
-                counted |= bits;
-            }
-        }
-    };
-
-    close_upto(q0, false);
-    if (q0 < q1) {
-        const uint32_t c_first = q0 >> 6, c_end = (q1 + 63u) >> 6;
-        auto in_tile = [&](uint32_t c) {
-            const uint32_t q = c * 64u + lane;
-            return q >= q0 && q < q1;
-        };
-        // Source activity comes from a bitmap of the vertices that changed last iteration (one bit per
-        // vertex, small enough to stay in L2): the word of each lane's source, tested at use.
-        uint32_t col0 = col[c_first * 64u + lane];
-        uint32_t col1 = 0;
-        if (c_first + 1 < c_end) col1 = col[(c_first + 1) * 64u + lane];
-        uint32_t a0 = in_tile(c_first) ? act_prev[col0 >> 5] : 0u;
-        for (uint32_t c = c_first; c < c_end; ++c) {
-            const uint64_t act = ballot(((a0 >> (col0 & 31u)) & 1u) != 0u);
-            // Prefetch, in this order (vector loads complete in order): activity of chunk c + 1, indices
-            // of chunk c + 2; both finish before this chunk's distance loads.
-            uint32_t a1 = 0;
-            if (c + 1 < c_end && in_tile(c + 1)) a1 = act_prev[col1 >> 5];
-            uint32_t col2 = 0;
-            if (c + 2 < c_end) col2 = col[(c + 2) * 64u + lane];
-            const unsigned long long bnd = starts[c];
-            const uint32_t lo = (q0 > c * 64u ? q0 - c * 64u : 0u);
-            const uint32_t hi = (q1 - c * 64u < 64u ? q1 - c * 64u : 64u);
-            if (act == 0ull && ballot(acc != kInf) == 0ull) {
-                close_upto(c * 64u + hi, true);  // nothing to fold: every row closing here is unreached
-            } else {
-                // The 64 sources' distance rows: an active source's row, or for an inactive one the
-                // all-unreached row n_rows (kept in cache), so every entry folds without a test. Every
-                // column of an active source is relaxed: a column whose distance did not change last
-                // iteration was relaxed through this edge when it last changed, so it cannot improve
-                // the row now, and the result (a fixed point of min) is the same.
-                const uint32_t w0 = kWeighted ? vals[c * 64u + lane] : 1u;  // weights: active chunks only
-                uint32_t x[64];
-                const uint32_t lane_off = lane * static_cast<uint32_t>(sizeof(DT));
-#pragma unroll
-                for (uint32_t t = 0; t < 64; ++t) {
-                    uint32_t cu = __builtin_amdgcn_readlane(col0, t);
-                    asm volatile("" : "+s"(cu));  // keep the readlane out of a branch: select, not jump
-                    const uint32_t u = ((act >> t) & 1ull) ? cu : n_rows;
-                    if constexpr (sizeof(DT) == 2) {
-                        // 32-bit byte offsets: the caller keeps (n_rows + 1) * 128 below 2^32
-                        x[t] = widen_dist<DT>(*reinterpret_cast<const DT*>(reinterpret_cast<const char*>(D) +
-                                                                          (u << 7) + lane_off));
-                    } else {
-                        x[t] = D[static_cast<size_t>(u) * 64 + lane];
-                    }
-                }
-                uint32_t lo_p = lo;
-                while (lo_p < hi) {
-                    // A fresh copy of the boundary bits for this part's fold, so the bits are tested
-                    // where they are used instead of 64 saved predicates being kept alive.
-                    uint64_t bnd_f = bnd;
-                    asm volatile("" : "+s"(bnd_f));
-                    // Boundaries strictly inside the part; at most kWaveStage of them.
-                    uint64_t inner = (lo_p + 1 < 64u) ? (bnd >> (lo_p + 1)) << (lo_p + 1) : 0ull;
-                    if (hi < 64u) inner &= (1ull << hi) - 1ull;
-                    uint32_t hi_p = hi;
-                    if (static_cast<uint32_t>(__popcll(inner)) > kWaveStage) {
-#pragma unroll
-                        for (uint32_t k = 0; k < kWaveStage; ++k) inner &= inner - 1ull;
-                        hi_p = static_cast<uint32_t>(__builtin_ctzll(inner));
-                    }
-                    uint32_t ns = 0;
-                    auto fold = [&](uint32_t t, bool first) {
-                        if (!first && ((bnd_f >> t) & 1ull)) {
-                            s_stage[wave][ns][lane] = acc;
-                            ++ns;
-                            acc = kInf;
-                        }
-                        const uint32_t wt = kWeighted ? __builtin_amdgcn_readlane(w0, t) : 1u;
-                        const uint32_t p = sizeof(DT) == 2 ? __builtin_elementwise_add_sat(x[t], wt)
-                                                           : MinPlusU32::combine(wt, x[t]);
-                        acc = p < acc ? p : acc;
-                    };
-                    if (lo_p == 0 && hi_p == 64) {  // the whole chunk in one part: no range tests
-#pragma unroll
-                        for (uint32_t t = 0; t < 64; ++t) fold(t, t == 0);
-                    } else {
-#pragma unroll
-                        for (uint32_t t = 0; t < 64; ++t)
-                            if (t >= lo_p && t < hi_p) fold(t, t == lo_p);
-                    }
-                    close_upto(c * 64u + hi_p, false);
-                    lo_p = hi_p;
-                }
-            }
-            col0 = col1;
-            a0 = a1;
-            col1 = col2;
-        }
+    const uint32_t tile = blockIdx.x;
+    const MergeCoord c0 = coords[tile], c1 = coords[tile + 1];
+    const uint64_t step0 = static_cast<uint64_t>(c0.x) + c0.y, step1 = static_cast<uint64_t>(c1.x) + c1.y;
+    auto quarter = [&](uint32_t w) { return step0 + w * (tile_items / 4) < step1 ? step0 + w * (tile_items / 4) : step1; };
+    const uint32_t r0 = wave_merge_search(row_offsets, c0.x, c1.x, quarter(wave));
+    if (lane == 0) {
+        s_row[wave] = r0;
+        if (wave == 0) s_row[kMergeWaves] = c1.x;
     }
-    recs[tile].carry[lane] = MinPlusU32::acc_t{acc};
-    if (lane == 0) recs[tile].flags = (r_last > r0 ? kTileHasEnd : 0u) | (deferred ? kTileDeferred : 0u);
+    __syncthreads();
+    const uint32_t r_last = __builtin_amdgcn_readfirstlane(s_row[wave + 1]);
+    const uint32_t q0 = static_cast<uint32_t>(quarter(wave) - r0);
+    const uint32_t steps = static_cast<uint32_t>(quarter(wave + 1) - quarter(wave));
+    const bool continued = r0 < r_last && row_offsets[r0] < q0;  // its first row end closes an earlier quarter's row
+
+    uint32_t acc = kInf;   // running minimum of the open row
+    uint32_t part = kInf;  // the continued row's, once closed
+    uint64_t counted = 0;
+    // Row r's distances become min(old, val); the columns that improved go to mask_next (cleared before the launch).
+    auto apply = [&](uint32_t r, uint32_t val, uint32_t old) {
+        const bool improved = val < old;
+        if (improved) {
+            if (sizeof(DT) == 2 && val >= kCompactLimit) *overflow = 1u;
+            else D[static_cast<size_t>(r) * 64 + lane] = static_cast<DT>(val);
+        }
+        const uint64_t bits = ballot(improved);
+        if (lane == 0 && bits) mask_next[r] = bits;
+        counted |= bits;
+    };
+    auto dist = [&](uint32_t u) -> uint32_t {
+        // 16-bit storage: 32-bit byte offsets, the caller keeps (n_rows + 1) * 128 below 2^32
+        if constexpr (sizeof(DT) == 2)
+            return widen_dist<DT>(*reinterpret_cast<const DT*>(reinterpret_cast<const char*>(D) + ((u << 7) + (lane << 1))));
+        return D[static_cast<size_t>(u) * 64 + lane];
+    };
+
+    // One block of 64 merge steps from row i, nonzero j on: the row-end mask, and the lane's row (a row end) or
+    // source and weight (a nonzero; a lane past the last step is a nonzero that `live` leaves out).
+    struct Block {
+        uint64_t ends;
+        uint32_t id, w;
+        uint64_t live;
+    };
+    uint32_t* mark = s_mark[wave];
+    auto load_block = [&](uint32_t i, uint32_t j, uint32_t left) -> Block {
+        Block b;
+        const uint32_t row = i + lane;
+        uint32_t at = 64;
+        if (row < r_last) at = row_offsets[row + 1] - j + lane;  // the step its end falls on
+        // (a wave's LDS operations run in program order, which the compiler must keep too)
+        mark[lane] = 0u;
+        asm volatile("" ::: "memory");
+        if (at < 64) mark[at] = 1u;
+        asm volatile("" ::: "memory");
+        const bool is_end = mark[lane] != 0u;
+        b.ends = ballot(is_end);
+        const uint32_t before = mask_prefix(b.ends);
+        b.live = ballot(lane < left && !is_end);
+        b.id = i + before;
+        b.w = 0;
+        if (lane < left && !is_end) {
+            const uint32_t q = j + lane - before;
+            b.id = __builtin_nontemporal_load(col + q);
+            b.w = kWeighted ? __builtin_nontemporal_load(vals + q) : 1u;
+        }
+        return b;
+    };
+    auto activity = [&](const Block& b) -> uint32_t { return (b.live >> lane) & 1ull ? act_prev[b.id >> 5] : 0u; };
+
+    uint64_t pending = 0;  // 1: the open row has an active nonzero in an earlier block
+    Block cur = load_block(r0, q0, steps);
+    uint32_t word = activity(cur);
+    uint32_t i = r0, j = q0;
+    for (uint32_t s = 0; s < steps; s += 64) {
+        const uint32_t rows = static_cast<uint32_t>(__popcll(cur.ends));
+        i += rows;
+        j += 64 - rows;
+        Block next{0, 0, 0, 0};
+        uint32_t next_word = 0;
+        const bool more = s + 64 < steps;
+        if (more) next = load_block(i, j, steps - s - 64);
+        const uint64_t active = ballot((word >> (cur.id & 31u)) & 1u) & cur.live;
+        // A row end needs its row when a nonzero since the row end before it is active (or the row is pending):
+        // adding the active bits to the runs of ones between the row ends carries into exactly those.
+        const uint64_t runs = ~cur.ends;
+        const uint64_t sum = runs + active;
+        const uint64_t all = sum + pending;
+        const uint64_t need = all & cur.ends;
+        pending = (sum < runs ? 1u : 0u) | (all < sum ? 1u : 0u);
+        const bool idle = (active | need) == 0ull;
+        const uint32_t id = ((active | need) >> lane) & 1ull ? cur.id : n_rows;
+        const uint32_t w = cur.w;
+        if (more) next_word = activity(next);
+        if (!idle) {
+            uint32_t x[kWaveChunk];
+#pragma unroll
+            for (uint32_t t = 0; t < kWaveChunk; ++t) x[t] = dist(__builtin_amdgcn_readlane(id, t));
+            for (uint32_t c = 0; c < 64; c += kWaveChunk) {
+                uint32_t p[kWaveChunk];
+#pragma unroll
+                for (uint32_t t = 0; t < kWaveChunk; ++t) {
+                    const uint32_t wt = __builtin_amdgcn_readlane(w, c + t);
+                    p[t] = sizeof(DT) == 2 ? __builtin_elementwise_add_sat(x[t], wt) : MinPlusU32::combine(wt, x[t]);
+                }
+                if (c + kWaveChunk < 64) {
+#pragma unroll
+                    for (uint32_t t = 0; t < kWaveChunk; ++t) x[t] = dist(__builtin_amdgcn_readlane(id, c + kWaveChunk + t));
+                }
+                const uint32_t ends = static_cast<uint32_t>(need >> c);
+#pragma unroll
+                for (uint32_t t = 0; t < kWaveChunk; ++t) {
+                    if ((ends >> t) & 1u) {
+                        const uint32_t r = __builtin_amdgcn_readlane(id, c + t);
+                        if (continued && r == r0) part = acc;
+                        else apply(r, acc, p[t]);
+                        acc = kInf;
+                    } else {
+                        acc = p[t] < acc ? p[t] : acc;
+                    }
+                }
+            }
+        }
+        cur = next;
+        word = next_word;
+    }
+
+    s_carry[wave][lane] = acc;
+    if (lane == 0) s_ends[wave] = r_last > r0;
+    __syncthreads();
+    // The minimum of the quarters' open rows before w since the last one that closed a row.
+    auto outer = [&](int w, bool& any) {
+        int u = w - 1;
+        while (u > 0 && !s_ends[u]) --u;
+        any = u >= 0 && s_ends[u] != 0u;
+        uint32_t m = kInf;
+        for (int v = u > 0 ? u : 0; v < w; ++v) m = s_carry[v][lane] < m ? s_carry[v][lane] : m;
+        return m;
+    };
+    bool before;
+    if (continued) {
+        const uint32_t o = outer(static_cast<int>(wave), before);
+        const uint32_t whole = part < o ? part : o;
+        if (!before && row_offsets[r0] < c0.y) recs[tile].head[lane] = MinPlusU32::acc_t{whole};
+        else if (ballot(whole != kInf)) apply(r0, whole, dist(r0));
+    }
+    if (wave == kMergeWaves - 1) {
+        recs[tile].carry[lane] = MinPlusU32::acc_t{outer(kMergeWaves, before)};
+        if (lane == 0) recs[tile].flags = (before ? kTileHasEnd : 0u) | (before && row_offsets[c0.x] < c0.y ? kTileDeferred : 0u);
+    }
     if (counted && lane == 0) {
-        const unsigned long long cur = *reinterpret_cast<volatile unsigned long long*>(changed);
-        if (counted & ~cur) atomicOr(changed, static_cast<unsigned long long>(counted));
+        const unsigned long long seen = *reinterpret_cast<volatile unsigned long long*>(changed);
+        if (counted & ~seen) atomicOr(changed, static_cast<unsigned long long>(counted));
     }
 }
 
@@ -962,27 +933,6 @@ struct PlusTimesBatchPolicy {
 // 1.03 ms with the round-based tile kernel, 0.66 ms here (6.5 TB/s of x rows; 0.88 ms with a wave per tile, 0.85 ms
 // with the run counter and the 64-bit row addresses on the scalar unit as well, 19 scalar instructions a
 // nonzero against 8); 11 M nonzeros of a PPR batch 0.72 ms with x parked in LDS and a wave per tile, 0.38 ms.
-constexpr uint32_t kWaveChunk = 16;
-static_assert(64 % kWaveChunk == 0, "a block of 64 indices holds whole chunks");
-
-// The number of rows of [lo, hi) that end before merge step `diag`: row r does when row_offsets[r + 1] + r + 1 <=
-// diag (merge_path_search with 64 rows tested at a time). Every lane of the wave calls it and gets lo plus that.
-__device__ __forceinline__ uint32_t wave_merge_search(const uint32_t* __restrict__ row_offsets, uint32_t lo, uint32_t hi,
-                                                      uint64_t diag) {
-    const uint32_t lane = lane_id();
-    while (lo < hi) {
-        const uint32_t stride = (hi - lo + kWave - 1) / kWave;
-        const uint32_t r = lo + lane * stride;
-        const bool ended = r < hi && static_cast<uint64_t>(row_offsets[r + 1]) + r + 1 <= diag;
-        const uint32_t k = static_cast<uint32_t>(__popcll(ballot(ended)));  // the first k lanes
-        if (k == 0) break;
-        const uint32_t next = lo + (k - 1) * stride + 1;  // row next - 1 ended
-        const uint32_t top = next - 1 + stride;           // row top, if tested, did not
-        lo = next;
-        if (top < hi) hi = top;
-    }
-    return __builtin_amdgcn_readfirstlane(lo);
-}
 
 // P: init(lane) once per wave; x<kWide>(u, lane) the lane's value of source u, loaded unconditionally (a
 // column the policy leaves out may read any valid element: its products are never stored); store(row, lane, y).

@@ -198,3 +198,43 @@ def test_sssp_batch_distances_past_16_bits(gpu):
             assert np.array_equal(got.values[c], want), (wv, c, s)
         if wv == 250:
             assert int(got.values.max()) > 0xFFFF
+
+
+@pytest.mark.parametrize("shape", ["alone", "chain", "hub", "sparse", "dense"])
+def test_batch64_row_shapes(gpu, shape):
+    """The k = 64 min-plus kernel takes 64 merge steps (nonzeros and row ends) at a time, a quarter of a merge tile
+    a wave: a vertex alone, one in-edge a row (every other step an end), a row across several tiles, blocks
+    that are nothing but row ends, and rows of about a block; on every merge tile, weighted (16-bit storage, and
+    with long edges the 32-bit rerun) and as BFS, against Dijkstra and the queue BFS."""
+    import graphone_amd as g1
+    rng = np.random.default_rng(len(shape))
+    if shape == "alone":
+        n, src, dst = 1, [], []
+    elif shape == "chain":
+        n = 300
+        src, dst = np.arange(n - 1), np.arange(1, n)
+    elif shape == "hub":
+        n = 6001  # everything leads to vertex 6000, which leads back to a third of it
+        src = np.concatenate([np.arange(6000), np.full(2000, 6000)])
+        dst = np.concatenate([np.full(6000, 6000), rng.choice(6000, 2000, replace=False)])
+    elif shape == "sparse":
+        n = 20000
+        src, dst = rng.integers(0, 40, 900) * 500, rng.integers(0, n, 900)
+    else:
+        n = 257
+        src, dst = np.repeat(np.arange(n), 63), rng.integers(0, n, 63 * n)
+    srcs = rng.integers(0, n, size=64 if n > 1 else 3)
+    for hi in (200, 70000):
+        w = rng.integers(1, hi + 1, size=len(src)).astype(np.uint32)
+        h = g1.HostGraph.from_edges(n, src, dst, w)
+        g = g1.Graph(h)
+        few = sorted(set(int(s) for s in srcs))[:4]
+        want = {s: (oracle.dijkstra(h.row_offsets, h.col_indices, h.weights, s),
+                    oracle.bfs_queue(h.row_offsets, h.col_indices, s)) for s in few}
+        for tile in (512, 1024, 2048, 4096):
+            g.set_merge_tile(tile)
+            for weighted in (True, False):
+                got = g.sssp_batch(srcs, k=64, weighted=weighted).values
+                for c, s in enumerate(srcs):
+                    if int(s) in want:
+                        assert np.array_equal(got[c], want[int(s)][0 if weighted else 1]), (tile, weighted, c)
