@@ -206,37 +206,69 @@ __global__ void __launch_bounds__(64) frontier_post_kernel(const unsigned long l
     }
 }
 
-// Returns (E << 32) | nf of the frontier in counter set `set`, once the work enqueued on s before it is
-// done. The host spins on the mailbox, yielding its core between polls after the first 2048 (a dense
-// iteration runs for hundreds of microseconds, and the query server polls from many threads at once);
-// every 1024 polls it asks the stream, and a stream that has drained (or failed) without the post showing
-// is an error.
-g1_status read_frontier(g1_graph* g, uint32_t set, hipStream_t s, unsigned long long* packed,
-                        const uint32_t* mins = nullptr, uint32_t nmins = 0, uint32_t* min_out = nullptr) {
-    const unsigned long long seq = ++g->post_seq;
-    frontier_post_kernel<<<1, 64, 0, s>>>(g->qcnt + set * kSegments, g->h_mbox, seq, mins, nmins);
-    G1_LAUNCHED();
+// Waits until `*word` (in the graph's mailbox) is seq. The host spins on it, yielding its core between polls
+// after the first 2048 (a dense iteration runs for hundreds of microseconds, and the query server polls from many
+// threads at once); every 1024 polls it asks the stream, and a stream that has drained (or failed) without the
+// post showing is an error.
+g1_status wait_post(const unsigned long long* word, unsigned long long seq, hipStream_t s) {
     uint32_t polls = 0;
-    while (__atomic_load_n(g->h_mbox, __ATOMIC_ACQUIRE) != seq) {
+    while (__atomic_load_n(word, __ATOMIC_ACQUIRE) != seq) {
         if ((++polls & 1023u) == 0) {
             const hipError_t q = hipStreamQuery(s);
             if (q != hipErrorNotReady) {
-                if (__atomic_load_n(g->h_mbox, __ATOMIC_ACQUIRE) == seq) break;
+                if (__atomic_load_n(word, __ATOMIC_ACQUIRE) == seq) break;
                 G1_HIP(q);
                 G1_HIP(hipStreamSynchronize(s));
-                G1_CHECK(__atomic_load_n(g->h_mbox, __ATOMIC_ACQUIRE) == seq, G1_ERR_INTERNAL,
-                         "frontier post missing after the stream drained");
+                G1_CHECK(__atomic_load_n(word, __ATOMIC_ACQUIRE) == seq, G1_ERR_INTERNAL,
+                         "post missing after the stream drained");
                 break;
             }
         }
         if (polls < 2048) _mm_pause();
         else std::this_thread::yield();
     }
+    return G1_OK;
+}
+
+// Returns (E << 32) | nf of the frontier in counter set `set`, once the work enqueued on s before it is done.
+g1_status read_frontier(g1_graph* g, uint32_t set, hipStream_t s, unsigned long long* packed,
+                        const uint32_t* mins = nullptr, uint32_t nmins = 0, uint32_t* min_out = nullptr) {
+    const unsigned long long seq = ++g->post_seq;
+    frontier_post_kernel<<<1, 64, 0, s>>>(g->qcnt + set * kSegments, g->h_mbox, seq, mins, nmins);
+    G1_LAUNCHED();
+    G1_TRY(wait_post(g->h_mbox, seq, s));
     const unsigned long long nf = __atomic_load_n(g->h_mbox + 1, __ATOMIC_ACQUIRE);
     const unsigned long long E = __atomic_load_n(g->h_mbox + 2, __ATOMIC_ACQUIRE);
     G1_CHECK(E < 0xFFFFFFFFull && nf <= 0xFFFFFFFFull, G1_ERR_INTERNAL, "frontier edge count overflow");
     *packed = (E << 32) | nf;
     if (min_out) *min_out = static_cast<uint32_t>(__atomic_load_n(g->h_mbox + 3, __ATOMIC_ACQUIRE));
+    return G1_OK;
+}
+
+// The loop of the SpMV engines. launch(i, post, seq) enqueues iteration i, which posts one value; ended(value)
+// says whether the run ends with it and sure(value) whether the iteration after the next one is needed whatever
+// the next one posts (a guess: a wrong one costs an iteration that changes nothing the run returns). While it is,
+// the host enqueues that iteration before it reads the next post, so that the GPU does not wait for the host
+// between iterations. *iterations gets the number of iterations up to the one that ended the run, at most
+// max_iter.
+template <typename Launch, typename Ended, typename Sure>
+g1_status drive_pull(g1_graph* g, hipStream_t s, uint32_t max_iter, Launch&& launch, Ended&& ended, Sure&& sure,
+                     uint32_t* iterations) {
+    unsigned long long seqs[2] = {0, 0};
+    uint32_t launched = 0, it = 0, ahead = 2;
+    while (it < max_iter) {
+        for (; launched < max_iter && launched - it < ahead; ++launched) {
+            seqs[launched & 1] = ++g->post_seq;
+            G1_TRY(launch(launched, g->h_mbox + 8 + 4 * (launched & 1), seqs[launched & 1]));
+        }
+        const unsigned long long* post = g->h_mbox + 8 + 4 * (it & 1);
+        G1_TRY(wait_post(post, seqs[it & 1], s));
+        const unsigned long long value = __atomic_load_n(post + 1, __ATOMIC_ACQUIRE);
+        ++it;
+        if (ended(value)) break;
+        ahead = sure(value) ? 2 : 1;
+    }
+    *iterations = it;
     return G1_OK;
 }
 
@@ -1229,15 +1261,13 @@ g1_status run_minplus_pull(g1_graph* g, uint32_t src, uint32_t* d, bool weighted
     const uint32_t cap = std::min<uint32_t>(persistent_cap(), kMaxPushBlocks);
     minplus_seed_kernel<<<grid_for(n, 256, cap), 256, 0, s>>>(n, src, d, g->xu);
     G1_LAUNCHED();
-    clear_u64_kernel<<<1, 64, 0, s>>>(g->ctr + 6, 1);
-    G1_LAUNCHED();
     const uint32_t* vals = weighted ? g->t_w : nullptr;
     const uint32_t lanes = csrvec_lanes(n, g->m);
     G1_HIP(hipEventRecord(g->ev[0], s));
-    uint64_t prev = 0, frontier_sum = 1;
+    uint64_t frontier_sum = 1;
     uint32_t it = 0;
     const double spmv_bytes = 4.0 * (n + 1.0) + 4.0 * g->m * (weighted ? 2.0 : 1.0) + 8.0 * n;
-    for (;;) {
+    auto launch = [&](uint32_t, unsigned long long* post, unsigned long long seq) -> g1_status {
         if (engine == G1_ENGINE_BLAS_CSRVEC) {
             const int tok = prof_begin(g, "spmv_csrvec_minplus", s);
             G1_TRY(launch_spmv_csrvec<MinPlusU32>(n, g->t_row_off, g->t_col, vals, g->xu, g->yu, lanes, s, g->t_long,
@@ -1252,17 +1282,21 @@ g1_status run_minplus_pull(g1_graph* g, uint32_t src, uint32_t* d, bool weighted
         apply_minplus_kernel<<<grid_for(n, 256, cap), 256, 0, s>>>(n, g->yu, d, g->xu, g->slots);
         G1_LAUNCHED();
         prof_end(g, tok, s, 12.0 * n);
-        sum_slots_kernel<<<1, 256, 0, s>>>(g->slots, kMaxPushBlocks, g->ctr + 6);
+        applied_post_kernel<<<1, 256, 0, s>>>(g->slots, kMaxPushBlocks, post, seq);
         G1_LAUNCHED();
-        ++it;
-        st->edges_sum += g->m;
-        G1_TRY(read_ctr(g, s, 6, 1));
-        const uint64_t c = g->h_ctr[6];
-        const uint64_t delta = c - prev;
-        prev = c;
-        if (delta == 0 || it >= kMaxIterations) break;
-        frontier_sum += delta;
-    }
+        return G1_OK;
+    };
+    // An iteration that applied at least this many vertices is hardly ever the last but one; one launched after
+    // the last has no finite x and changes nothing.
+    constexpr uint64_t kSureApplied = 32;
+    G1_TRY(drive_pull(
+        g, s, kMaxIterations, launch,
+        [&](unsigned long long applied) {
+            frontier_sum += applied;
+            return applied == 0;
+        },
+        [&](unsigned long long applied) { return applied >= kSureApplied; }, &it));
+    st->edges_sum = static_cast<uint64_t>(it) * g->m;
     G1_HIP(hipEventRecord(g->ev[1], s));
     G1_TRY(elapsed(g, st));
     G1_TRY(prof_flush(g));
@@ -1356,33 +1390,44 @@ g1_status run_pagerank(g1_graph* g, float alpha, uint32_t seed, float restart, u
         G1_TRY(ensure_rank_partials(g));
         const uint32_t nb = rank_blocks(n);
         G1_HIP(hipMemcpyAsync(g->seeds_dev, &seed, sizeof(uint32_t), hipMemcpyHostToDevice, s));
-        for (;;) {
-            if (it >= max_iter) break;
+        double* const sum = g->rpart + static_cast<size_t>(nb) * kBatchCols;
+        auto launch = [&](uint32_t i, unsigned long long* post, unsigned long long seq) -> g1_status {
             int tok;
             if (engine == G1_ENGINE_BLAS_CSRVEC) {
                 tok = prof_begin(g, "spmv_csrvec_plustimes", s);
                 G1_TRY(launch_spmv_csrvec<PlusTimesF32>(n, t_ro, t_ci, vals, g->xf, g->yf, lanes, s, lrows, nlong,
-                                                              g->long_min));
+                                                        g->long_min));
             } else {
                 tok = prof_begin(g, "spmv_merge_plustimes", s);
                 G1_TRY(launch_spmv_merge<PlusTimesF32>(n, g->m, t_ro, t_ci, vals, g->xf, g->yf, ws, s));
             }
             prof_end(g, tok, s, spmv_bytes);
             tok = prof_begin(g, "pr_apply", s);
-            rank_apply_kernel<<<nb, 256, 0, s>>>(n, g->yf, base_all, g->seeds_dev, base_seed, g->iw, g->r[cur],
-                                                 g->r[cur ^ 1], g->xf, g->rpart);
+            rank_apply_kernel<<<nb, 256, 0, s>>>(n, g->yf, base_all, g->seeds_dev, base_seed, g->iw, g->r[i & 1],
+                                                 g->r[(i & 1) ^ 1], g->xf, g->rpart);
             G1_LAUNCHED();
             prof_end(g, tok, s, 20.0 * n);
-            reduce_partials_kernel<0><<<dim3(1, 1), 256, 0, s>>>(g->rpart, nb, g->rpart + static_cast<size_t>(nb) * kBatchCols);
+            if (nb >= kRunsMin) {  // (one column: the partials' other columns are free)
+                partial_runs_kernel<<<16, 256, 0, s>>>(g->rpart, nb, g->rpart + nb);
+                G1_LAUNCHED();
+                reduce_partials_kernel<0><<<1, 256, 0, s>>>(g->rpart + nb, 256, sum, post, seq);
+            } else {
+                reduce_partials_kernel<0><<<1, 256, 0, s>>>(g->rpart, nb, sum, post, seq);
+            }
             G1_LAUNCHED();
-            cur ^= 1;
-            ++it;
-            G1_HIP(hipMemcpyAsync(g->h_scalar, g->rpart + static_cast<size_t>(nb) * kBatchCols, sizeof(double),
-                                  hipMemcpyDeviceToHost, s));
-            G1_HIP(hipStreamSynchronize(s));
-            delta = g->h_scalar[0];
-            if (delta < tol) break;
-        }
+            return G1_OK;
+        };
+        // The change falls by at most a factor of two or so an iteration (a seed's first iterations aside), so
+        // one far above the tolerance means at least one more iteration after the next. An iteration launched
+        // after the last one writes the other rank vector.
+        G1_TRY(drive_pull(
+            g, s, max_iter, launch,
+            [&](unsigned long long bits) {
+                delta = __builtin_bit_cast(double, bits);
+                return delta < tol;
+            },
+            [&](unsigned long long) { return delta > 8.0 * tol; }, &it));
+        cur = static_cast<int>(it & 1);
     }
     G1_HIP(hipEventRecord(g->ev[1], s));
     G1_TRY(elapsed(g, st));

@@ -271,10 +271,10 @@ static g1_status graph_common(g1_graph* g, const char* what) {
     G1_TRY(alloc_n(g, &g->partials, kPartials + 8));
     G1_CHECK(hipHostMalloc(reinterpret_cast<void**>(&g->h_ctr), 256 * sizeof(unsigned long long)) == hipSuccess &&
                  hipHostMalloc(reinterpret_cast<void**>(&g->h_scalar), 8 * sizeof(double)) == hipSuccess &&
-                 hipHostMalloc(reinterpret_cast<void**>(&g->h_mbox), 4 * sizeof(unsigned long long),
+                 hipHostMalloc(reinterpret_cast<void**>(&g->h_mbox), 16 * sizeof(unsigned long long),
                                hipHostMallocCoherent) == hipSuccess,
              G1_ERR_HIP, "%s: pinned host allocation failed", what);
-    memset(g->h_mbox, 0, 4 * sizeof(unsigned long long));
+    memset(g->h_mbox, 0, 16 * sizeof(unsigned long long));
     G1_CHECK(hipEventCreate(&g->ev[0]) == hipSuccess && hipEventCreate(&g->ev[1]) == hipSuccess, G1_ERR_HIP,
              "%s: event creation failed", what);
     return G1_OK;
