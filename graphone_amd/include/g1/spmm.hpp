@@ -627,8 +627,8 @@ __device__ __forceinline__ uint32_t wave_merge_search(const uint32_t* __restrict
 // Distances are stored as DT: uint32_t, or int16_t when every finite distance of the run is below
 // kCompactLimit (then a source row is one 128-byte line instead of two). 16-bit storage is exact or
 // void: -1 is the unreached distance, so a sign-extending load yields G1_INF for it and the distance
-// itself otherwise; a relaxation that would store a finite value >= kCompactLimit sets *overflow instead
-// (the caller then reruns the batch with 32-bit storage). With 16-bit storage the weight is added with
+// itself otherwise; a relaxation that would store a finite value >= kCompactLimit sets *overflow instead and
+// counts as no change (the run then still ends, and the caller reruns the batch with 32-bit storage). With 16-bit storage the weight is added with
 // unsigned saturation, which equals the semiring's combine because x + w cannot wrap (the caller only
 // picks 16-bit storage when every weight is <= 0xFFFF0000).
 constexpr uint32_t kCompactLimit = 0x7FFFu;
@@ -686,11 +686,12 @@ spmm_minplus_wave_kernel(uint32_t n_rows, uint32_t tile_items, const uint32_t* _
     uint64_t counted = 0;
     // Row r's distances become min(old, val); the columns that improved go to mask_next (cleared before the launch).
     auto apply = [&](uint32_t r, uint32_t val, uint32_t old) {
-        const bool improved = val < old;
-        if (improved) {
-            if (sizeof(DT) == 2 && val >= kCompactLimit) *overflow = 1u;
-            else D[static_cast<size_t>(r) * 64 + lane] = static_cast<DT>(val);
+        bool improved = val < old;
+        if (sizeof(DT) == 2 && improved && val >= kCompactLimit) {
+            *overflow = 1u;
+            improved = false;  // nothing is stored: a change reported here would be reported again for ever
         }
+        if (improved) D[static_cast<size_t>(r) * 64 + lane] = static_cast<DT>(val);
         const uint64_t bits = ballot(improved);
         if (lane == 0 && bits) mask_next[r] = bits;
         counted |= bits;
@@ -870,11 +871,12 @@ struct MinPlusBatchPolicy16 {
         return widen_dist<int16_t>(D[static_cast<size_t>(row) * 64 + j]);
     }
     __device__ __forceinline__ uint64_t row_done(uint32_t row, uint32_t j, uint32_t y, uint32_t old) const {
-        const bool improved = y < old;
-        if (improved) {
-            if (y >= kCompactLimit) *overflow = 1u;
-            else D[static_cast<size_t>(row) * 64 + j] = static_cast<int16_t>(y);
+        bool improved = y < old;
+        if (improved && y >= kCompactLimit) {
+            *overflow = 1u;
+            improved = false;  // as in the kernel
         }
+        if (improved) D[static_cast<size_t>(row) * 64 + j] = static_cast<int16_t>(y);
         const uint64_t bits = ballot(improved);
         if (j == 0) mask_next[row] = bits;
         return (j == 0) ? bits : 0ull;
