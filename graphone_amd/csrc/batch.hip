@@ -260,7 +260,8 @@ g1_status launch_plustimes(g1_graph* g, const float* X, float* Y, void* recs_v, 
     bool done = false;
     if constexpr (K == 64) {
         if (ppr_wave()) {
-            launch_spmm_wave<PlusTimesF32>(g->n, tiles, g->t_row_off, g->t_col, vals, coords, recs, pol,
+            launch_spmm_wave<PlusTimesF32>(g->n, g->m, tiles, kMergeTile, false, g->t_row_off, g->t_col, vals,
+                                           merge_coords(g->t_ws), recs, pol,
                                            static_cast<uint64_t>(g->n) * K * sizeof(float), s);
             G1_LAUNCHED();
             done = true;

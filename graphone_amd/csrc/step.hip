@@ -106,10 +106,21 @@ g1_status advance(uint32_t n, const uint32_t* row_off, const uint32_t* col, cons
     return G1_OK;
 }
 
-// SpMM workspace: the merge-path partition of the matrix, then the tile records of one 64-column pass
-// (sized for the larger record, the plus-times one).
+// Merge steps of an SpMM tile (a workgroup; a wave takes a quarter): 2048, halved down to 256 while the matrix
+// gives the chip fewer than 8,192 waves, all that it holds at once. A wave's steps are a chain of loads, sixteen
+// sources at a time: 330 K rows and nonzeros x 8 columns take 25 us at 256 (86 at 2048), 1.3 M x 100 columns 121 us
+// (240 at 2048).
+uint32_t spmm_tile_items(uint32_t n_rows, uint32_t nnz) {
+    const uint64_t total = static_cast<uint64_t>(n_rows) + nnz;
+    uint32_t items = kMergeTile;
+    while (items > kMergeTile / 8 && total / (items / 4) < 8192) items /= 2;
+    return items;
+}
+
+// SpMM workspace: the tiles' starts, then their records of one 64-column pass (sized for the larger record, the
+// plus-times one).
 size_t spmm_ws_bytes(uint32_t n_rows, uint32_t nnz) {
-    const size_t t = merge_num_tiles(n_rows, nnz);
+    const size_t t = merge_num_tiles_for(n_rows, nnz, spmm_tile_items(n_rows, nnz));
     return al((t + 1) * sizeof(MergeCoord)) + t * sizeof(SpmmTileRec<PlusTimesF32, 64>) + 256;
 }
 
@@ -125,16 +136,23 @@ g1_status spmm(uint32_t n_rows, uint32_t n_cols, uint32_t nnz, uint32_t k, const
     G1_CHECK(ws != nullptr && ws_bytes >= spmm_ws_bytes(n_rows, nnz), G1_ERR_INVALID_ARG,
              "%s: workspace of %zu bytes, %zu needed (g1_spmm_workspace_bytes)", what, ws_bytes,
              spmm_ws_bytes(n_rows, nnz));
-    const uint32_t tiles = merge_num_tiles(n_rows, nnz);
-    G1_TRY(launch_merge_partition(n_rows, nnz, row_off, ws, s));
-    const MergeCoord* coords = merge_coords(ws);
+    const uint32_t items = spmm_tile_items(n_rows, nnz);
+    const uint32_t tiles = merge_num_tiles_for(n_rows, nnz, items);
+    MergeCoord* coords = merge_coords(ws);
     auto* recs = reinterpret_cast<SpmmTileRec<S, 64>*>(static_cast<char*>(ws) + al((tiles + 1ull) * sizeof(MergeCoord)));
+    // While every tile is resident at once, a search over all the rows in each wave (three or four loads) costs less
+    // than a launch that partitions the matrix (10 us); beyond, the searches would add up.
+    const bool find = tiles <= 2048;
+    if (!find) {
+        merge_partition_kernel<<<(tiles + 1 + 255) / 256, 256, 0, s>>>(row_off, n_rows, nnz, tiles, coords, items);
+        G1_LAUNCHED();
+    }
     using T = typename S::x_t;
     const T neutral = std::is_same_v<S, MinPlusU32> ? static_cast<T>(kInf) : T(0);
     for (uint32_t c0 = 0; c0 < k; c0 += 64) {
         StridedColumnsPolicy<T> pol{X, Y, k, c0, std::min<uint32_t>(64u, k - c0), mask, neutral};
-        launch_spmm_wave<S>(n_rows, tiles, row_off, col, vals, coords, recs, pol, static_cast<uint64_t>(n_cols) * k * sizeof(T),
-                            s);
+        launch_spmm_wave<S>(n_rows, nnz, tiles, items, find && c0 == 0, row_off, col, vals, coords, recs, pol,
+                            static_cast<uint64_t>(n_cols) * k * sizeof(T), s);
         G1_LAUNCHED();
         if (tiles > 1) {
             spmm_fixup_kernel<S, 64, StridedColumnsPolicy<T>><<<(tiles * 64u + 255) / 256, 256, 0, s>>>(

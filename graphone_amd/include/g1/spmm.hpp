@@ -940,9 +940,10 @@ struct PlusTimesBatchPolicy {
 // column the policy leaves out may read any valid element: its products are never stored); store(row, lane, y).
 template <typename S, bool kValues, bool kWide, typename P>
 __global__ void __launch_bounds__(256)
-spmm_wave_kernel(uint32_t n_rows, const uint32_t* __restrict__ row_offsets,
-                 const uint32_t* __restrict__ col, const typename S::value_t* __restrict__ vals,
-                 const MergeCoord* __restrict__ coords, SpmmTileRec<S, 64>* __restrict__ recs, P pol) {
+spmm_wave_kernel(uint32_t n_rows, uint32_t nnz, uint32_t quarter_steps, bool find,
+                 const uint32_t* __restrict__ row_offsets, const uint32_t* __restrict__ col,
+                 const typename S::value_t* __restrict__ vals, MergeCoord* __restrict__ coords,
+                 SpmmTileRec<S, 64>* __restrict__ recs, P pol) {
     using acc_t = typename S::acc_t;
     using value_t = typename S::value_t;
     using x_t = typename S::x_t;
@@ -954,18 +955,34 @@ spmm_wave_kernel(uint32_t n_rows, const uint32_t* __restrict__ row_offsets,
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t tile = blockIdx.x;
-    const MergeCoord c0 = coords[tile], c1 = coords[tile + 1];
     pol.init(lane);
 
-    // the quarters' bounds: the merge-path search of the wave's first step, 64 rows at a time
-    const uint64_t step0 = static_cast<uint64_t>(c0.x) + c0.y, step1 = static_cast<uint64_t>(c1.x) + c1.y;
-    auto quarter = [&](uint32_t w) { return step0 + w * (kMergeTile / 4) < step1 ? step0 + w * (kMergeTile / 4) : step1; };
+    // The quarters' bounds: the merge-path search of the wave's first step, 64 rows at a time, within the tile's rows
+    // or, when the caller has no partition, in all of them (the tile's start then goes to coords for the fixup).
+    MergeCoord c0{0, 0}, c1{n_rows, nnz};
+    const uint64_t total = static_cast<uint64_t>(n_rows) + nnz;
+    const uint64_t step0 = static_cast<uint64_t>(tile) * (4ull * quarter_steps);
+    const uint64_t step1 = step0 + 4ull * quarter_steps < total ? step0 + 4ull * quarter_steps : total;
+    auto quarter = [&](uint32_t w) { return step0 + w * static_cast<uint64_t>(quarter_steps) < step1 ? step0 + w * static_cast<uint64_t>(quarter_steps) : step1; };
+    if (!find) {
+        c0 = coords[tile];
+        c1 = coords[tile + 1];
+    }
     const uint32_t first = wave_merge_search(row_offsets, c0.x, c1.x, quarter(wave));
+    if (find && wave == kMergeWaves - 1) c1.x = wave_merge_search(row_offsets, first, n_rows, step1);
     if (lane == 0) {
         s_row[wave] = first;
-        if (wave == 0) s_row[kMergeWaves] = c1.x;
+        if (wave == kMergeWaves - 1) s_row[kMergeWaves] = c1.x;
     }
     __syncthreads();
+    if (find) {
+        c0.x = __builtin_amdgcn_readfirstlane(s_row[0]);
+        c0.y = static_cast<uint32_t>(step0 - c0.x);
+        if (threadIdx.x == 0) {
+            coords[tile] = c0;
+            if (tile == gridDim.x - 1) coords[tile + 1] = MergeCoord{n_rows, nnz};
+        }
+    }
     const uint32_t r0 = first, r_last = __builtin_amdgcn_readfirstlane(s_row[wave + 1]);
     const uint32_t q0 = static_cast<uint32_t>(quarter(wave) - r0), q1 = static_cast<uint32_t>(quarter(wave + 1) - r_last);
 
@@ -1127,13 +1144,18 @@ spmm_wave_kernel(uint32_t n_rows, const uint32_t* __restrict__ row_offsets,
     }
 }
 
-// One pass of the wave kernel; x_bytes is the size of the x array the policy reads.
+// One pass of the wave kernel over `tiles` tiles of tile_items merge steps; x_bytes is the size of the x array the
+// policy reads. With `find` the waves search the whole matrix for their bounds and leave the tiles' starts in
+// coords, otherwise coords holds the partition.
 template <typename S, typename P>
-inline void launch_spmm_wave(uint32_t n_rows, uint32_t tiles, const uint32_t* row_off, const uint32_t* col,
-                             const typename S::value_t* vals, const MergeCoord* coords, SpmmTileRec<S, 64>* recs,
-                             const P& pol, uint64_t x_bytes, hipStream_t s) {
+inline void launch_spmm_wave(uint32_t n_rows, uint32_t nnz, uint32_t tiles, uint32_t tile_items, bool find,
+                             const uint32_t* row_off, const uint32_t* col, const typename S::value_t* vals,
+                             MergeCoord* coords, SpmmTileRec<S, 64>* recs, const P& pol, uint64_t x_bytes,
+                             hipStream_t s) {
     const bool wide = x_bytes >= (1ull << 32);
-    auto go = [&](auto kernel) { kernel<<<tiles, 256, 0, s>>>(n_rows, row_off, col, vals, coords, recs, pol); };
+    auto go = [&](auto kernel) {
+        kernel<<<tiles, 256, 0, s>>>(n_rows, nnz, tile_items / 4, find, row_off, col, vals, coords, recs, pol);
+    };
     if (vals) {
         if (wide) go(spmm_wave_kernel<S, true, true, P>);
         else go(spmm_wave_kernel<S, true, false, P>);
