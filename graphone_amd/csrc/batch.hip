@@ -40,11 +40,12 @@ struct BatchWork {
 namespace g1 {
 namespace {
 
-// state[0] = frozen, state[1] = 0 (the batched PPR's device-side stop-rule state)
+// state[0] = state[2] = frozen, state[1] = 0 (the batched PPR's device-side stop-rule state)
 __global__ void set_state_kernel(unsigned long long* state, unsigned long long frozen) {
     if (threadIdx.x == 0) {
         state[0] = frozen;
         state[1] = 0ull;
+        state[2] = frozen;
     }
 }
 
@@ -134,6 +135,15 @@ g1_status ensure_wave_coords(g1_graph* g, uint32_t idx, hipStream_t s) {
     return G1_OK;
 }
 
+// k = 64 plus-times SpMM on the wavefront kernel unless G1_PPR_WAVE=0 (same bits either way).
+bool ppr_wave() {
+    static const bool on = [] {
+        const char* e = getenv("G1_PPR_WAVE");
+        return !(e && e[0] == '0');
+    }();
+    return on;
+}
+
 g1_status ensure_batch(g1_graph* g, uint32_t K, bool ppr, BatchWork** out, hipStream_t s) {
     const int slot = k_slot(K);
     G1_CHECK(slot >= 0, G1_ERR_INVALID_ARG, "column tile k must be 8, 16, 32 or 64 (got %u)", K);
@@ -165,11 +175,13 @@ g1_status ensure_batch(g1_graph* g, uint32_t K, bool ppr, BatchWork** out, hipSt
             G1_TRY(alloc_n(g, &b->overflow, 64));
         }
     }
-    if (ppr && !b->X) {
-        G1_TRY(alloc_n(g, &b->R[0], n * K));
+    if (ppr && !b->R[1]) {
+        if (!b->R[0]) G1_TRY(alloc_n(g, &b->R[0], n * K));
+        if (K != 64 || !ppr_wave()) {  // (the wavefront kernel needs neither, see RankBatchPolicy)
+            if (!b->X) G1_TRY(alloc_n(g, &b->X, n * K));
+            if (!b->Y) G1_TRY(alloc_n(g, &b->Y, n * K));
+        }
         G1_TRY(alloc_n(g, &b->R[1], n * K));
-        G1_TRY(alloc_n(g, &b->X, n * K));
-        G1_TRY(alloc_n(g, &b->Y, n * K));
         G1_TRY(ensure_rank_partials(g));
         G1_TRY(ensure_pull_work(g, true));  // iw
     }
@@ -201,11 +213,11 @@ __global__ void minplus_batch_seed_kernel(DT* __restrict__ D, unsigned long long
     }
 }
 
-// R0 = e_seed per column and X0 = R0 * iw (pr_init_kernel's seed variant, per column); padding columns
-// (seed kInf) start at zero.
+// R0 = e_seed per column and X0 = R0 * iw (pr_init_kernel's seed variant, per column; X may be null); padding
+// columns (seed kInf) start at zero, in the other rank vector R1 too.
 template <int K>
 __global__ void ppr_batch_init_kernel(uint32_t n, const float* __restrict__ iw, const uint32_t* __restrict__ seeds,
-                                      float* __restrict__ R, float* __restrict__ X) {
+                                      float* __restrict__ R, float* __restrict__ R1, float* __restrict__ X) {
     const size_t total = static_cast<size_t>(n) * K;
     const size_t stride = static_cast<size_t>(gridDim.x) * blockDim.x;
     for (size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < total; i += stride) {
@@ -213,7 +225,8 @@ __global__ void ppr_batch_init_kernel(uint32_t n, const float* __restrict__ iw, 
         const uint32_t j = static_cast<uint32_t>(i % K);
         const float rv = (v == seeds[j]) ? 1.0f : 0.0f;
         R[i] = rv;
-        X[i] = rv * iw[v];
+        if (seeds[j] == kInf) R1[i] = 0.0f;
+        if (X) X[i] = rv * iw[v];
     }
 }
 
@@ -237,15 +250,6 @@ __global__ void __launch_bounds__(256) batch_columns_out_kernel(uint32_t n, cons
         const uint32_t c = f / 64, r = f % 64;
         if (v0 + r < n) out[static_cast<size_t>(c) * n + v0 + r] = s[c][r];
     }
-}
-
-// k = 64 plus-times SpMM on the wavefront kernel unless G1_PPR_WAVE=0 (same bits either way).
-bool ppr_wave() {
-    static const bool on = [] {
-        const char* e = getenv("G1_PPR_WAVE");
-        return !(e && e[0] == '0');
-    }();
-    return on;
 }
 
 // One plus-times SpMM iteration: Y = A^T (x) X over the in-edges (k columns, 64-bit sums in the fold order
@@ -276,6 +280,23 @@ g1_status launch_plustimes(g1_graph* g, const float* X, float* Y, void* recs_v, 
         const uint32_t blocks = static_cast<uint32_t>((static_cast<uint64_t>(tiles) * K + 255) / 256);
         spmm_fixup_kernel<PlusTimesF32, K, PlusTimesBatchPolicy<K>><<<blocks, 256, 0, s>>>(tiles, coords, recs,
                                                                                               pol, nullptr);
+        G1_LAUNCHED();
+    }
+    return G1_OK;
+}
+
+// One iteration of batched personalized PageRank over 64 columns: the product and the new ranks (RankBatchPolicy).
+g1_status launch_rank64(g1_graph* g, const float* R_old, float* R_new, float restart, const unsigned long long* state,
+                        void* recs_v, hipStream_t s) {
+    const uint32_t tiles = merge_num_tiles(g->n, g->m);
+    RankBatchPolicy pol{R_old, R_new, g->iw, g->seeds_dev, restart, state};
+    auto* recs = static_cast<SpmmTileRec<PlusTimesF32, 64>*>(recs_v);
+    launch_spmm_wave<PlusTimesF32>(g->n, g->m, tiles, kMergeTile, false, g->t_row_off, g->t_col, g->t_wf,
+                                   merge_coords(g->t_ws), recs, pol, static_cast<uint64_t>(g->n) * 256, s);
+    G1_LAUNCHED();
+    if (tiles > 1) {
+        spmm_fixup_kernel<PlusTimesF32, 64, RankBatchPolicy><<<(tiles + 3) / 4, 256, 0, s>>>(
+            tiles, merge_coords(g->t_ws), recs, pol, nullptr);
         G1_LAUNCHED();
     }
     return G1_OK;
@@ -444,7 +465,7 @@ g1_status ppr_tile_run(g1_graph* g, BatchWork* b, const uint32_t* seeds_host, ui
     pr_init_kernel<<<fill_blocks(n), 256, 0, s>>>(n, g->osum, 1.0f - restart, g->iw, g->r[0], 0.0f, g->xf, kInf);
     G1_LAUNCHED();
     ppr_batch_init_kernel<K><<<fill_blocks(static_cast<size_t>(n) * K), 256, 0, s>>>(n, g->iw, g->seeds_dev, b->R[0],
-                                                                                      b->X);
+                                                                                      b->R[1], b->X);
     G1_LAUNCHED();
     // Device state of the stop rule: state[0] frozen columns (padding columns never run), state[1] the
     // iteration count; written with the seeds' stream order, by a kernel (no memset in the captured work).
@@ -457,9 +478,20 @@ g1_status ppr_tile_run(g1_graph* g, BatchWork* b, const uint32_t* seeds_host, ui
     // One iteration: SpMM, apply (frozen columns keep their ranks), the canonical L1 per column, the freeze.
     // An iteration after every column froze changes nothing (frozen columns copy R into the other buffer).
     auto iteration = [&](int cur, hipStream_t st) -> g1_status {
-        G1_TRY(launch_plustimes<K>(g, b->X, b->Y, b->recs, st));
-        rank_apply_batch_kernel<K><<<rank_apply_grid<K>(nb), 256, 0, st>>>(
-            n, b->Y, 0.0f, g->seeds_dev, restart, g->iw, b->R[cur], b->R[cur ^ 1], b->X, g->rpart, nb, 0ull, state);
+        bool fused = false;
+        if constexpr (K == 64) {
+            if (ppr_wave()) {
+                G1_TRY(launch_rank64(g, b->R[cur], b->R[cur ^ 1], restart, state, b->recs, st));
+                rank_delta_batch_kernel<K><<<rank_apply_grid<K>(nb), 256, 0, st>>>(n, b->R[cur], b->R[cur ^ 1], g->rpart,
+                                                                                 nb, state);
+                fused = true;
+            }
+        }
+        if (!fused) {
+            G1_TRY(launch_plustimes<K>(g, b->X, b->Y, b->recs, st));
+            rank_apply_batch_kernel<K><<<rank_apply_grid<K>(nb), 256, 0, st>>>(
+                n, b->Y, 0.0f, g->seeds_dev, restart, g->iw, b->R[cur], b->R[cur ^ 1], b->X, g->rpart, nb, 0ull, state);
+        }
         G1_LAUNCHED();
         reduce_partials_kernel<0><<<dim3(1, K), 256, 0, st>>>(g->rpart, nb, g->rpart + static_cast<size_t>(nb) * kBatchCols);
         G1_LAUNCHED();

@@ -223,9 +223,49 @@ __global__ void __launch_bounds__(256) rank_apply_batch_kernel(uint32_t n, const
         partials[static_cast<size_t>(j) * nblocks + blk] = ((s_q[g][j] + s_q[g + 1][j]) + s_q[g + 2][j]) + s_q[g + 3][j];
 }
 
+// The canonical L1 partials of |r' - r| alone, for an iteration whose product kernel wrote r' (RankBatchPolicy);
+// quarters and order as above. A column that is frozen (state[0]) and was running when the iteration before began
+// (not in state[2]) gets its rank copied into r', so that both vectors hold it from then on. Bound by its 8 bytes
+// an element.
+template <int K>
+__global__ void __launch_bounds__(256) rank_delta_batch_kernel(uint32_t n, const float* __restrict__ R_old,
+                                                               float* __restrict__ R_new,
+                                                               double* __restrict__ partials, uint32_t nblocks,
+                                                               const unsigned long long* __restrict__ state) {
+    constexpr uint32_t G = 256 / K;
+    constexpr uint32_t U = 8;
+    __shared__ double s_q[G][K];
+    const uint32_t j = threadIdx.x % K;
+    const uint32_t g = threadIdx.x / K;
+    const uint32_t blk = blockIdx.x * (G / 4) + g / 4;
+    const uint32_t v0 = blk * 256 + (g % 4) * kWave;
+    const bool carry = ((state[0] & ~state[2]) >> j) & 1ull;
+    double acc = 0.0;
+    for (uint32_t k = 0; k < static_cast<uint32_t>(kWave) && v0 + k < n; k += U) {
+        float ro[U], rn[U];
+#pragma unroll
+        for (uint32_t u = 0; u < U; ++u) {
+            const size_t at = static_cast<size_t>(v0 + k + u < n ? v0 + k + u : n - 1) * K + j;
+            ro[u] = R_old[at];
+            rn[u] = R_new[at];
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < U; ++u)
+            if (v0 + k + u < n) {
+                if (carry) R_new[static_cast<size_t>(v0 + k + u) * K + j] = ro[u];
+                else acc += fabs(static_cast<double>(rn[u]) - static_cast<double>(ro[u]));
+            }
+    }
+    s_q[g][j] = acc;
+    __syncthreads();
+    if (g % 4 == 0 && blk < nblocks)
+        partials[static_cast<size_t>(j) * nblocks + blk] = ((s_q[g][j] + s_q[g + 1][j]) + s_q[g + 2][j]) + s_q[g + 3][j];
+}
+
 // The stop rule of the batched personalized PageRank, per column, on the device: a column still running
 // whose FP64 L1 delta (deltas[j]) fell below tol freezes; state[0] is the frozen mask, state[1] counts the
-// iterations that began with a running column. One wave.
+// iterations that began with a running column, state[2] is the mask that this iteration began with (its columns'
+// ranks are in both vectors now). One wave.
 template <int K>
 __global__ void __launch_bounds__(64) ppr_freeze_kernel(const double* __restrict__ deltas, double tol,
                                                         unsigned long long* __restrict__ state) {
@@ -236,6 +276,7 @@ __global__ void __launch_bounds__(64) ppr_freeze_kernel(const double* __restrict
     const unsigned long long nf = f | ballot(stop);
     if (j == 0) {
         if (f != all) state[1] += 1ull;
+        state[2] = f;
         state[0] = nf;
     }
 }

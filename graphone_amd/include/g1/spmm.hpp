@@ -891,6 +891,7 @@ struct PlusTimesBatchPolicy {
     static constexpr bool kRowOld = false;
     const float* X;
     float* Y;
+    static constexpr bool kScale = false;
     __device__ __forceinline__ void init(uint32_t) {}
     template <bool kWide>
     __device__ __forceinline__ float x(uint32_t u, uint32_t j) const {
@@ -912,6 +913,46 @@ struct PlusTimesBatchPolicy {
 };
 
 // ------------------------------------------------------------------------------------------------
+// One iteration of batched personalized PageRank over 64 columns without x and y arrays: a source's x is its old
+// rank times its out-weight's inverse (the product rank_apply_batch_kernel would have stored, so the same bits),
+// and a row's sum goes straight to its new rank. Columns in state[0] (converged, or padding) are not stored:
+// rank_delta_batch_kernel carries their ranks over. Saves y written and read and x written, 12 of 20 bytes an element beside the
+// gathers, for a multiplication a nonzero: 0.7 M vertices x 64 columns 0.38 (product) + 0.17 ms (apply) an
+// iteration before, 0.42 + 0.06 (L1 partials) here; a graph of 20,000 vertices takes 4 % longer (114 us an iteration).
+struct RankBatchPolicy {
+    using aux_t = uint32_t;
+    static constexpr bool kHasAux = false;
+    static constexpr bool kRowOld = false;
+    static constexpr bool kScale = true;
+    const float* R_old;
+    float* R_new;
+    const float* iw;
+    const uint32_t* seeds;
+    float base_seed;
+    const unsigned long long* state;
+    uint32_t seed = 0;
+    bool running = false;
+    __device__ __forceinline__ void init(uint32_t j) {
+        seed = seeds[j];
+        running = !((state[0] >> j) & 1ull);
+    }
+    template <bool kWide>
+    __device__ __forceinline__ float x(uint32_t u, uint32_t j) const {
+        if constexpr (kWide) return R_old[static_cast<size_t>(u) * 64 + j];
+        return *reinterpret_cast<const float*>(reinterpret_cast<const char*>(R_old) + (u * 256u + j * 4u));
+    }
+    __device__ __forceinline__ float scale(uint32_t u) const { return iw[u]; }
+    __device__ __forceinline__ void store(uint32_t row, uint32_t j, float y) const {
+        const float rn = (row == seed ? base_seed : 0.0f) + y;
+        if (running) R_new[static_cast<size_t>(row) * 64 + j] = rn;
+    }
+    __device__ __forceinline__ uint64_t row_done(uint32_t row, uint32_t j, float y, float) {
+        init(j);
+        store(row, j, y);
+        return 0ull;
+    }
+};
+
 // SpMM over 64 columns: a workgroup of four waves takes a merge-path tile, a wave a quarter of its merge
 // steps, lane j = column j, the walk on the scalar unit. It reproduces the fold of spmv_merge_tile_kernel
 // exactly, per column: a quarter's 512 steps are cut into the same 64 runs of 8 that the threads of one of
@@ -937,7 +978,8 @@ struct PlusTimesBatchPolicy {
 // nonzero against 8); 11 M nonzeros of a PPR batch 0.72 ms with x parked in LDS and a wave per tile, 0.38 ms.
 
 // P: init(lane) once per wave; x<kWide>(u, lane) the lane's value of source u, loaded unconditionally (a
-// column the policy leaves out may read any valid element: its products are never stored); store(row, lane, y).
+// column the policy leaves out may read any valid element: its products are never stored), times scale(u) where
+// kScale says so; store(row, lane, y).
 template <typename S, bool kValues, bool kWide, typename P>
 __global__ void __launch_bounds__(256)
 spmm_wave_kernel(uint32_t n_rows, uint32_t nnz, uint32_t quarter_steps, bool find,
@@ -1073,6 +1115,8 @@ spmm_wave_kernel(uint32_t n_rows, uint32_t nnz, uint32_t quarter_steps, bool fin
         uint32_t cA, wA, cB, wB;
         load_block(c / kPer, cA, wA);
         load_block(c / kPer + 1, cB, wB);
+        uint32_t sA = 0;  // the block's scales, a lane each
+        if constexpr (P::kScale) sA = __builtin_bit_cast(uint32_t, pol.scale(cA));
         load_x(cA, (c % kPer) * kWaveChunk);
         for (; c < c_end; ++c) {
             const uint32_t at = (c % kPer) * kWaveChunk;
@@ -1081,11 +1125,14 @@ spmm_wave_kernel(uint32_t n_rows, uint32_t nnz, uint32_t quarter_steps, bool fin
             for (uint32_t t = 0; t < kWaveChunk; ++t) {
                 value_t w = value_t(1);
                 if (kValues) w = __builtin_bit_cast(value_t, static_cast<uint32_t>(__builtin_amdgcn_readlane(wA, at + t)));
-                p[t] = S::combine(w, xn[t]);
+                x_t x = xn[t];
+                if constexpr (P::kScale) x *= __builtin_bit_cast(float, static_cast<uint32_t>(__builtin_amdgcn_readlane(sA, at + t)));
+                p[t] = S::combine(w, x);
             }
             if (at + kWaveChunk == 64u) {
                 cA = cB;
                 wA = wB;
+                if constexpr (P::kScale) sA = __builtin_bit_cast(uint32_t, pol.scale(cA));
                 load_x(cA, 0);
                 load_block((c + 1) / kPer + 1, cB, wB);
             } else {

@@ -275,6 +275,7 @@ struct StridedColumnsPolicy {
     using aux_t = uint32_t;
     static constexpr bool kHasAux = false;
     static constexpr bool kRowOld = false;
+    static constexpr bool kScale = false;
     const T* X;
     T* Y;
     uint32_t ld;  // k
