@@ -54,6 +54,16 @@ struct RoadQuery {
     unsigned long long edges_sum;     // out: relaxations
 };
 
+// A pointer read from a query record, as a pointer to global memory: through a generic one the compiler issues flat
+// accesses, whose completion the LDS counter waits for as well, so that every LDS read after a store to a far list
+// waited for that store.
+template <typename T>
+using road_global = __attribute__((address_space(1))) T*;
+template <typename T>
+__device__ __forceinline__ road_global<T> to_global(T* p) {
+    return (road_global<T>)p;
+}
+
 // The start and end of v's row in one 8-byte load (any u32 alignment).
 struct RoadRow {
     uint32_t beg, end;
@@ -90,10 +100,10 @@ road_query_kernel(const uint32_t* __restrict__ row_off, const uint32_t* __restri
     const uint32_t sub = tid % kRoadLanes, grp = tid / kRoadLanes;
     const bool kSssp = Q.sssp != 0;  // uniform per workgroup
     const uint32_t src = Q.src;
-    unsigned long long* const ds = Q.dstamp;
-    uint32_t* const depth = Q.depth;
-    uint32_t* const gq[2] = {Q.q[0], Q.q[1]};
-    uint32_t* const far[2] = {Q.far[0], Q.far[1]};
+    const road_global<unsigned long long> ds = to_global(Q.dstamp);
+    const road_global<uint32_t> depth = to_global(Q.depth);
+    const road_global<uint32_t> gq[2] = {to_global(Q.q[0]), to_global(Q.q[1])};
+    const road_global<uint32_t> far[2] = {to_global(Q.far[0]), to_global(Q.far[1])};
     // Appends v to near frontier b (counter c): LDS for the first kRoadChunk entries, the query's buffer
     // after them.
     auto push_near = [&](uint32_t b, uint32_t c, uint32_t v, RoadRow r) {
@@ -218,7 +228,7 @@ road_query_kernel(const uint32_t* __restrict__ row_off, const uint32_t* __restri
                     v[r] = col[e];
                     if (kSssp) {
                         w[r] = wts[e];
-                        dw[r] = __hip_atomic_load(&ds[u[r]], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                    dw[r] = __hip_atomic_load(&ds[u[r]], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);  // (BFS: unused)
                     }
                 }
                 RoadRow row[R];
@@ -325,8 +335,12 @@ road_lds_kernel(uint32_t n, const uint32_t* __restrict__ row_off, const uint32_t
     const uint32_t sub = tid % kRoadLanes, grp = tid / kRoadLanes;
     const bool kSssp = Q.sssp != 0;  // uniform per workgroup
     const uint32_t src = Q.src;
-    uint32_t* const gq[2] = {Q.q[0], Q.q[1]};
-    uint32_t* const far[2] = {Q.far[0], Q.far[1]};
+    const road_global<uint32_t> gq[2] = {to_global(Q.q[0]), to_global(Q.q[1])};
+    const road_global<uint32_t> far[2] = {to_global(Q.far[0]), to_global(Q.far[1])};
+    // The second load of an edge: its weight, or (BFS) its target again. Without a branch between them the two are in
+    // flight together (30 sources of a 150x200 grid 642 -> 629 us with the pointers above). road_query_kernel keeps its branch: its
+    // second load comes with the distance, which a BFS has no use for (64 sources of a 610x377 grid: 4.07 against 4.19 ms).
+    const uint32_t* const second = kSssp ? wts : col;
     const uint32_t words = (n + 1) / 2, fwords = (n + 31) / 32;
     for (uint32_t i = tid; i < words; i += kRoadThreads) s_d[i] = 0xFFFFFFFFu;
     for (uint32_t i = tid; i < fwords; i += kRoadThreads) {
@@ -453,11 +467,14 @@ road_lds_kernel(uint32_t n, const uint32_t* __restrict__ row_off, const uint32_t
                 for (uint32_t r = 0; r < R; ++r) {
                     const uint32_t e = on[r] ? k[r] : 0u;
                     v[r] = col[e];
-                    w[r] = kSssp ? wts[e] : 1u;
+                    w[r] = second[e];
                 }
                 RoadRow row[R];
 #pragma unroll
-                for (uint32_t r = 0; r < R; ++r) row[r] = road_row(row_off, v[r]);
+                for (uint32_t r = 0; r < R; ++r) {
+                    row[r] = road_row(row_off, v[r]);
+                    if (!kSssp) w[r] = 1u;
+                }
 #pragma unroll
                 for (uint32_t r = 0; r < R; ++r) {
                     if (!on[r]) continue;
@@ -511,7 +528,7 @@ road_lds_kernel(uint32_t n, const uint32_t* __restrict__ row_off, const uint32_t
     if (!bad) {
         for (uint32_t v = tid; v < n; v += kRoadThreads) {
             const uint32_t d = dist(v);
-            Q.depth[v] = d == 0xFFFFu ? kInf : d;
+            to_global(Q.depth)[v] = d == 0xFFFFu ? kInf : d;
         }
     }
     const unsigned long long edges = road_block_sum(esum, s_sum);
