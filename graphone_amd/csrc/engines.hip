@@ -566,8 +566,6 @@ __global__ void dstamp_extract_kernel(uint32_t n, const unsigned long long* __re
         dist[v] = static_cast<uint32_t>(ds[v] >> 32);
 }
 
-
-
 // ---------------------------------------------------------------- road-like graphs (one workgroup)
 
 // Low-degree graphs (at most kRoadMaxDeg out-edges per vertex: grids, road networks) take the
@@ -577,12 +575,12 @@ constexpr uint32_t kRoadMaxDeg = 16;
 
 bool road_graph(const g1_graph* g) { return g->n > 0 && g->max_out_deg <= kRoadMaxDeg; }
 
-// near-far bucket width: sixteen heaviest edges (a wide bucket: few splits, few extra relaxations)
-// Bucket width of the road engine's near-far split, a multiple of the largest weight: 16 for the LDS kernel
-// (a wider bucket saves iterations, which cost ~3 us each there), 8 for the global-memory kernel (whose
-// extra relaxations cost more). Measured from vertex 1 on p = 0.6 grids: 213 x 213, weights [1, 64], LDS
-// kernel 1.60 ms at 16 (1.67 at 8, 1.63 at 32); 2048 x 2048, weights [1, 255], global kernel 68.3 ms at 8
-// (76.3 at 16, 68.1 at 4). G1_ROAD_DELTA sets one multiple for both.
+// Bucket width of the road engine's near-far split, a multiple of the largest weight: 16 for the LDS kernel (a
+// wider bucket saves iterations, ~1.5 us each there), 8 for the global-memory kernel (whose extra relaxations cost
+// more). Measured on p = 0.6 grids: 213 x 213, weights [1, 64], LDS kernel 0.82 ms at 16 (0.84 at 8, 0.90 at 32),
+// 30 sources of a 150 x 200 one 0.63 ms (0.67 at 8 and at 32); 48 sources of a 610 x 377 one, weights [1, 255],
+// global kernel 4.07 ms at 8 (4.44 at 16, 4.18 at 4); one source of 2048 x 2048 53.0 ms at 8 (61.9 at 16, 51.8 at
+// 4). G1_ROAD_DELTA sets one multiple for both.
 uint32_t road_delta(const g1_graph* g, bool lds) {
     static const int forced = [] {
         const char* e = getenv("G1_ROAD_DELTA");

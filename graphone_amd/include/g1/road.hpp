@@ -339,7 +339,7 @@ road_lds_kernel(uint32_t n, const uint32_t* __restrict__ row_off, const uint32_t
     const road_global<uint32_t> far[2] = {to_global(Q.far[0]), to_global(Q.far[1])};
     // The second load of an edge: its weight, or (BFS) its target again. Without a branch between them the two are in
     // flight together (30 sources of a 150x200 grid 642 -> 629 us with the pointers above). road_query_kernel keeps its branch: its
-    // second load comes with the distance, which a BFS has no use for (64 sources of a 610x377 grid: 4.07 against 4.19 ms).
+    // second load comes with the distance, which a BFS has no use for (48 sources of a 610x377 grid: 4.07 against 4.19 ms).
     const uint32_t* const second = kSssp ? wts : col;
     const uint32_t words = (n + 1) / 2, fwords = (n + 31) / 32;
     for (uint32_t i = tid; i < words; i += kRoadThreads) s_d[i] = 0xFFFFFFFFu;
