@@ -118,9 +118,10 @@ uint32_t spmm_tile_items(uint32_t n_rows, uint32_t nnz) {
 }
 
 // SpMM workspace: the tiles' starts, then their records of one 64-column pass (sized for the larger record, the
-// plus-times one).
-size_t spmm_ws_bytes(uint32_t n_rows, uint32_t nnz) {
-    const size_t t = merge_num_tiles_for(n_rows, nnz, spmm_tile_items(n_rows, nnz));
+// plus-times one). A smaller one, down to that of tiles of 2048 steps, is taken too: the tiles are then the smallest
+// that it holds.
+size_t spmm_ws_bytes(uint32_t n_rows, uint32_t nnz, uint32_t items) {
+    const size_t t = merge_num_tiles_for(n_rows, nnz, items);
     return al((t + 1) * sizeof(MergeCoord)) + t * sizeof(SpmmTileRec<PlusTimesF32, 64>) + 256;
 }
 
@@ -133,10 +134,11 @@ g1_status spmm(uint32_t n_rows, uint32_t n_cols, uint32_t nnz, uint32_t k, const
     G1_CHECK(n_cols > 0 || nnz == 0, G1_ERR_INVALID_ARG, "%s: nnz > 0 with zero columns", what);
     G1_CHECK(nnz < kInf, G1_ERR_INVALID_ARG, "%s: nnz must be below 2^32-1", what);
     if (n_rows == 0 || k == 0) return G1_OK;
-    G1_CHECK(ws != nullptr && ws_bytes >= spmm_ws_bytes(n_rows, nnz), G1_ERR_INVALID_ARG,
+    uint32_t items = spmm_tile_items(n_rows, nnz);
+    while (items < kMergeTile && ws_bytes < spmm_ws_bytes(n_rows, nnz, items)) items *= 2;
+    G1_CHECK(ws != nullptr && ws_bytes >= spmm_ws_bytes(n_rows, nnz, items), G1_ERR_INVALID_ARG,
              "%s: workspace of %zu bytes, %zu needed (g1_spmm_workspace_bytes)", what, ws_bytes,
-             spmm_ws_bytes(n_rows, nnz));
-    const uint32_t items = spmm_tile_items(n_rows, nnz);
+             spmm_ws_bytes(n_rows, nnz, items));
     const uint32_t tiles = merge_num_tiles_for(n_rows, nnz, items);
     MergeCoord* coords = merge_coords(ws);
     auto* recs = reinterpret_cast<SpmmTileRec<S, 64>*>(static_cast<char*>(ws) + al((tiles + 1ull) * sizeof(MergeCoord)));
@@ -289,7 +291,9 @@ g1_status g1_l1_delta_f64(uint32_t n, const float* a, const float* b, double* ou
     return G1_OK;
 }
 
-size_t g1_spmm_workspace_bytes(uint32_t n_rows, uint32_t nnz) { return spmm_ws_bytes(n_rows, nnz); }
+size_t g1_spmm_workspace_bytes(uint32_t n_rows, uint32_t nnz) {
+    return spmm_ws_bytes(n_rows, nnz, spmm_tile_items(n_rows, nnz));
+}
 
 g1_status g1_spmm_minplus_u32(uint32_t n_rows, uint32_t n_cols, uint32_t nnz, uint32_t k, const uint32_t* row_offsets,
                               const uint32_t* col_indices, const uint32_t* values, const uint32_t* X, uint32_t* Y,

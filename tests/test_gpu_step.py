@@ -305,7 +305,13 @@ def test_spmm_tile_edges(gpu, degs, k):
     Xf = rng.standard_normal((n_cols, k)).astype(np.float32)
     Xf[0] = np.inf
     dX, dXf = _dev(X), _dev(Xf)
-    for values in (True, False):
+    # a workspace for tiles of 2048 steps (what as many tiles of 256 need) is enough, and less is refused
+    least = g1._lib.lib().g1_spmm_workspace_bytes(-(-(n_rows + m) // 2048) * 256, 0)
+    with pytest.raises(g1.G1Error):
+        _call("g1_spmm_minplus_u32", n_rows, n_cols, m, k, _p(drp), _p(dci), _p(dw), _p(dX), _p(dX), None, _p(ws),
+              C.c_size_t(least - 1), None)
+    full = wsb
+    for values, wsb in ((True, full), (False, full), (True, least)):
         dY, dYf = g1.DeviceArray(n_rows * k, np.uint32), g1.DeviceArray(n_rows * k, np.float32)
         _call("g1_spmm_minplus_u32", n_rows, n_cols, m, k, _p(drp), _p(dci), _p(dw) if values else None, _p(dX), _p(dY),
               None, _p(ws), C.c_size_t(wsb), None)
