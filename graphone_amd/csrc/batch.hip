@@ -30,6 +30,7 @@ struct BatchWork {
     float* R[2] = {nullptr, nullptr};                      // PPR ranks, n x K
     float* X = nullptr;
     float* Y = nullptr;
+    float* iw_nz = nullptr;                                // k = 64 PPR: iw of each in-edge's source
     hipGraphExec_t minplus_exec[kWaveTileCount][2] = {};   // two captured iterations, [merge tile][weighted]
     int16_t* D16 = nullptr;                                // n x 64 distances, 16-bit storage (k = 64)
     uint32_t* overflow = nullptr;                          // set when a distance does not fit 16 bits
@@ -144,6 +145,13 @@ bool ppr_wave() {
     return on;
 }
 
+// Whether the k = 64 PPR product reads its sources' scales (iw) from an array in the in-edges' order, filled once per
+// call, instead of gathering them. The gather is one of 4 bytes a nonzero beside the 256-byte rows, and past the L2 it
+// costs a line each: RMAT22 x 64 columns 4.0 -> 3.5 ms an iteration (198.6 -> 175.1 ms for 50), 2 M vertices 65.4 ->
+// 61.2 ms, 0.7 M 25.5 -> 24.0. Below 2^18 vertices iw is a small part of the L2 and the array a launch more (20,000
+// vertices 5.74 -> 5.78 ms). Past 128 in-edges a vertex the array would take more memory than a 64-column one.
+bool scales_stream(const g1_graph* g) { return g->n >= (1u << 18) && g->m <= 128ull * g->n && g->m > 0; }
+
 g1_status ensure_batch(g1_graph* g, uint32_t K, bool ppr, BatchWork** out, hipStream_t s) {
     const int slot = k_slot(K);
     G1_CHECK(slot >= 0, G1_ERR_INVALID_ARG, "column tile k must be 8, 16, 32 or 64 (got %u)", K);
@@ -180,6 +188,8 @@ g1_status ensure_batch(g1_graph* g, uint32_t K, bool ppr, BatchWork** out, hipSt
         if (K != 64 || !ppr_wave()) {  // (the wavefront kernel needs neither, see RankBatchPolicy)
             if (!b->X) G1_TRY(alloc_n(g, &b->X, n * K));
             if (!b->Y) G1_TRY(alloc_n(g, &b->Y, n * K));
+        } else if (scales_stream(g) && !b->iw_nz) {
+            G1_TRY(alloc_n(g, &b->iw_nz, g->m));
         }
         G1_TRY(alloc_n(g, &b->R[1], n * K));
         G1_TRY(ensure_rank_partials(g));
@@ -286,10 +296,10 @@ g1_status launch_plustimes(g1_graph* g, const float* X, float* Y, void* recs_v, 
 }
 
 // One iteration of batched personalized PageRank over 64 columns: the product and the new ranks (RankBatchPolicy).
-g1_status launch_rank64(g1_graph* g, const float* R_old, float* R_new, float restart, const unsigned long long* state,
-                        void* recs_v, hipStream_t s) {
+g1_status launch_rank64(g1_graph* g, const float* R_old, float* R_new, const float* iw_nz, float restart,
+                        const unsigned long long* state, void* recs_v, hipStream_t s) {
     const uint32_t tiles = merge_num_tiles(g->n, g->m);
-    RankBatchPolicy pol{R_old, R_new, g->iw, g->seeds_dev, restart, state};
+    RankBatchPolicy pol{R_old, R_new, g->iw, iw_nz, g->seeds_dev, restart, state};
     auto* recs = static_cast<SpmmTileRec<PlusTimesF32, 64>*>(recs_v);
     launch_spmm_wave<PlusTimesF32>(g->n, g->m, tiles, kMergeTile, false, g->t_row_off, g->t_col, g->t_wf,
                                    merge_coords(g->t_ws), recs, pol, static_cast<uint64_t>(g->n) * 256, s);
@@ -453,6 +463,24 @@ g1_status minplus_tile_run(g1_graph* g, BatchWork* b, const uint32_t* srcs_host,
     return G1_OK;
 }
 
+// out[e] = iw[col[e]]: four gathers in flight a thread.
+__global__ void __launch_bounds__(256) edge_scale_kernel(uint32_t m, const uint32_t* __restrict__ col,
+                                                         const float* __restrict__ iw, float* __restrict__ out) {
+    const size_t stride = static_cast<size_t>(gridDim.x) * 256;
+    size_t e = static_cast<size_t>(blockIdx.x) * 256 + threadIdx.x;
+    for (; e + 3 * stride < m; e += 4 * stride) {
+        uint32_t c[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) c[r] = col[e + r * stride];
+        float v[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[r] = iw[c[r]];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) out[e + r * stride] = v[r];
+    }
+    for (; e < m; e += stride) out[e] = iw[col[e]];
+}
+
 template <int K>
 g1_status ppr_tile_run(g1_graph* g, BatchWork* b, const uint32_t* seeds_host, uint32_t cols, float restart,
                        uint32_t max_iter, double tol, float* out, uint32_t* iterations, hipStream_t s) {
@@ -464,6 +492,10 @@ g1_status ppr_tile_run(g1_graph* g, BatchWork* b, const uint32_t* seeds_host, ui
     // iw from the out-edges, then R0 = e_seed per column, X0 = R0 * iw
     pr_init_kernel<<<fill_blocks(n), 256, 0, s>>>(n, g->osum, 1.0f - restart, g->iw, g->r[0], 0.0f, g->xf, kInf);
     G1_LAUNCHED();
+    if (K == 64 && b->iw_nz) {
+        edge_scale_kernel<<<fill_blocks(g->m), 256, 0, s>>>(g->m, g->t_col, g->iw, b->iw_nz);
+        G1_LAUNCHED();
+    }
     ppr_batch_init_kernel<K><<<fill_blocks(static_cast<size_t>(n) * K), 256, 0, s>>>(n, g->iw, g->seeds_dev, b->R[0],
                                                                                       b->R[1], b->X);
     G1_LAUNCHED();
@@ -481,7 +513,7 @@ g1_status ppr_tile_run(g1_graph* g, BatchWork* b, const uint32_t* seeds_host, ui
         bool fused = false;
         if constexpr (K == 64) {
             if (ppr_wave()) {
-                G1_TRY(launch_rank64(g, b->R[cur], b->R[cur ^ 1], restart, state, b->recs, st));
+                G1_TRY(launch_rank64(g, b->R[cur], b->R[cur ^ 1], b->iw_nz, restart, state, b->recs, st));
                 rank_delta_batch_kernel<K><<<rank_apply_grid<K>(nb), 256, 0, st>>>(n, b->R[cur], b->R[cur ^ 1], g->rpart,
                                                                                  nb, state);
                 fused = true;

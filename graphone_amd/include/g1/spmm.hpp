@@ -917,7 +917,8 @@ struct PlusTimesBatchPolicy {
 // rank times its out-weight's inverse (the product rank_apply_batch_kernel would have stored, so the same bits),
 // and a row's sum goes straight to its new rank. Columns in state[0] (converged, or padding) are not stored:
 // rank_delta_batch_kernel carries their ranks over. Saves y written and read and x written, 12 of 20 bytes an element beside the
-// gathers, for a multiplication a nonzero: 0.7 M vertices x 64 columns 0.38 (product) + 0.17 ms (apply) an
+// gathers, for a multiplication a nonzero and its source's scale (which streams beside the weights on large graphs, see
+// scales_stream in batch.hip): 0.7 M vertices x 64 columns 0.38 (product) + 0.17 ms (apply) an
 // iteration before, 0.42 + 0.06 (L1 partials) here; a graph of 20,000 vertices takes 4 % longer (114 us an iteration).
 struct RankBatchPolicy {
     using aux_t = uint32_t;
@@ -927,6 +928,7 @@ struct RankBatchPolicy {
     const float* R_old;
     float* R_new;
     const float* iw;
+    const float* iw_nz;  // iw of each nonzero's source, in the nonzeros' order (null: gathered from iw)
     const uint32_t* seeds;
     float base_seed;
     const unsigned long long* state;
@@ -941,6 +943,8 @@ struct RankBatchPolicy {
         if constexpr (kWide) return R_old[static_cast<size_t>(u) * 64 + j];
         return *reinterpret_cast<const float*>(reinterpret_cast<const char*>(R_old) + (u * 256u + j * 4u));
     }
+    __device__ __forceinline__ bool scale_streams() const { return iw_nz != nullptr; }
+    __device__ __forceinline__ float scale_at(uint32_t e) const { return __builtin_nontemporal_load(iw_nz + e); }
     __device__ __forceinline__ float scale(uint32_t u) const { return iw[u]; }
     __device__ __forceinline__ void store(uint32_t row, uint32_t j, float y) const {
         const float rn = (row == seed ? base_seed : 0.0f) + y;
@@ -979,7 +983,7 @@ struct RankBatchPolicy {
 
 // P: init(lane) once per wave; x<kWide>(u, lane) the lane's value of source u, loaded unconditionally (a
 // column the policy leaves out may read any valid element: its products are never stored), times scale(u) where
-// kScale says so; store(row, lane, y).
+// kScale says so (scale_at(e) of nonzero e instead where scale_streams() does, uniform); store(row, lane, y).
 template <typename S, bool kValues, bool kWide, typename P>
 __global__ void __launch_bounds__(256)
 spmm_wave_kernel(uint32_t n_rows, uint32_t nnz, uint32_t quarter_steps, bool find,
@@ -1097,14 +1101,26 @@ spmm_wave_kernel(uint32_t n_rows, uint32_t nnz, uint32_t quarter_steps, bool fin
         const uint32_t c_end = (q1 + kWaveChunk - 1) / kWaveChunk;
         uint32_t c = q0 / kWaveChunk;
         // a lane outside the tile's nonzeros holds source 0 (never folded)
+        uint32_t sB = 0;  // the scales of the block loaded last, if they stream
         auto load_block = [&](uint32_t b, uint32_t& cv, uint32_t& wv) {
             const uint32_t q = b * 64u + lane;
             cv = 0;
             wv = 0;
+            if constexpr (P::kScale) sB = 0;
             if (q >= q0 && q < q1) {
                 cv = __builtin_nontemporal_load(col + q);
                 if (kValues) wv = __builtin_bit_cast(uint32_t, __builtin_nontemporal_load(vals + q));
+                if constexpr (P::kScale) {
+                    if (pol.scale_streams()) sB = __builtin_bit_cast(uint32_t, pol.scale_at(q));
+                }
             }
+        };
+        // the scales of the block whose sources are cv: s if they stream
+        auto scales = [&](uint32_t cv, uint32_t s) {
+            if constexpr (P::kScale) {
+                if (!pol.scale_streams()) s = __builtin_bit_cast(uint32_t, pol.scale(cv));
+            }
+            return s;
         };
         x_t xn[kWaveChunk];
         auto load_x = [&](uint32_t cv, uint32_t at) {
@@ -1114,9 +1130,8 @@ spmm_wave_kernel(uint32_t n_rows, uint32_t nnz, uint32_t quarter_steps, bool fin
         };
         uint32_t cA, wA, cB, wB;
         load_block(c / kPer, cA, wA);
+        uint32_t sA = scales(cA, sB);  // the block's scales, a lane each
         load_block(c / kPer + 1, cB, wB);
-        uint32_t sA = 0;  // the block's scales, a lane each
-        if constexpr (P::kScale) sA = __builtin_bit_cast(uint32_t, pol.scale(cA));
         load_x(cA, (c % kPer) * kWaveChunk);
         for (; c < c_end; ++c) {
             const uint32_t at = (c % kPer) * kWaveChunk;
@@ -1132,7 +1147,7 @@ spmm_wave_kernel(uint32_t n_rows, uint32_t nnz, uint32_t quarter_steps, bool fin
             if (at + kWaveChunk == 64u) {
                 cA = cB;
                 wA = wB;
-                if constexpr (P::kScale) sA = __builtin_bit_cast(uint32_t, pol.scale(cA));
+                sA = scales(cA, sB);
                 load_x(cA, 0);
                 load_block((c + 1) / kPer + 1, cB, wB);
             } else {

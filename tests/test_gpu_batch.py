@@ -238,3 +238,23 @@ def test_batch64_row_shapes(gpu, shape):
                 for c, s in enumerate(srcs):
                     if int(s) in want:
                         assert np.array_equal(got[c], want[int(s)][0 if weighted else 1]), (tile, weighted, c)
+
+
+@pytest.mark.parametrize("n", [(1 << 18) - 1, 1 << 18])
+def test_ppr_batch64_scale_array(gpu, n):
+    """The 64-column PPR product gathers its sources' scales below 2^18 vertices and streams them in the in-edges'
+    order from there: either way a column has the single-seed run's bits, with another restart (other scales) on the
+    same graph as well. Two thirds of the edges leave 500 hubs; most vertices have neither in- nor out-edges."""
+    import graphone_amd as g1
+    rng = np.random.default_rng(n)
+    m = 400_003
+    src = np.where(rng.random(m) < 0.66, rng.integers(0, 500, m), rng.integers(0, n, m))
+    dst = rng.integers(0, n // 3, m)
+    h = g1.HostGraph.from_edges(n, src, dst, rng.integers(1, 50, m).astype(np.uint32), directed=True)
+    g = g1.Graph(h)
+    seeds = [0, 1, n - 1] + [int(v) for v in src[:64]]  # more than one tile of 64
+    for restart in (0.15, 0.4):
+        got = g.ppr_batch(seeds, restart=restart, max_iter=9, tol=0.0, k=64)
+        for c in (0, 2, 40, 66):
+            single = g.ppr(seeds[c], restart=restart, max_iter=9, tol=0.0)
+            assert np.array_equal(got.values[c].view(np.uint32), single.values.view(np.uint32)), (restart, c)
