@@ -19,8 +19,8 @@
 // Three rotating counters leave one barrier per iteration. The query's state belongs to its workgroup, so
 // its atomics have workgroup scope. Measured against reading the row offsets at the start of an iteration, a
 // prefix sum over the chunk and a binary search per edge: grid 213 x 213 (distances in LDS, 550 iterations)
-// 2.9 -> 1.5 us an iteration, 1.68 -> 0.85 ms a run; 48 queries on a 610 x 377 grid (distances in memory, 1390
-// iterations) 5.8 -> 2.9 us, 8.0 -> 4.1 ms; one SSSP on 2048 x 2048 68 -> 54 ms, BFS 44 -> 34 ms.
+// 2.9 -> 1.5 us an iteration, 1.68 -> 0.83 ms a run; 48 queries on a 610 x 377 grid (distances in memory, 1390
+// iterations) 5.8 -> 2.9 us, 8.0 -> 4.1 ms; one SSSP on 2048 x 2048 68 -> 53 ms, BFS 44 -> 34 ms.
 
 #pragma once
 
