@@ -620,14 +620,16 @@ g1_status ensure_road_work(g1_graph* g, hipStream_t s) {
 // record lives in pinned host memory: the kernel reads the query from it and writes the outcome to it, so a
 // run is three or four launches and one stream synchronization. A small graph's query runs with its distances
 // in LDS (road_lds_kernel); if that reports status 2 (a distance past 16 bits, or a list overflow) the query
-// runs on the global-memory kernel.
+// runs on the global-memory kernel, and the run's time counts both. (The reached counts of the first are then over an
+// array that it left alone; the second's take their place.)
 template <bool kSssp>
 g1_status run_road(g1_graph* g, uint32_t src, uint32_t* out, g1_run_stats* st, hipStream_t s, bool* ok) {
     G1_TRY(ensure_road_work(g, s));
     const uint32_t n = g->n;
     RoadQuery* hq = reinterpret_cast<RoadQuery*>(g->h_ctr + 128);
     const uint64_t qcap = std::min<uint64_t>(static_cast<uint64_t>(g->seg_cap) * kSegments, 0xFFFFFFFFull);
-    for (int pass = n <= kRoadLdsMaxN ? 0 : 1; pass < 2; ++pass) {
+    const int first = n <= kRoadLdsMaxN ? 0 : 1;
+    for (int pass = first; pass < 2; ++pass) {
         memset(hq, 0, sizeof(RoadQuery));
         hq->sssp = kSssp ? 1u : 0u;
         hq->dstamp = g->dstamp;
@@ -644,7 +646,7 @@ g1_status run_road(g1_graph* g, uint32_t src, uint32_t* out, g1_run_stats* st, h
             else depth_init_kernel<<<init_blocks, 256, 0, s>>>(n, src, out);
             G1_LAUNCHED();
         }
-        G1_HIP(hipEventRecord(g->ev[0], s));
+        if (pass == first) G1_HIP(hipEventRecord(g->ev[0], s));
         const int tok = prof_begin(g, kSssp ? "road_sssp" : "road_bfs", s);
         if (pass == 0) {
             road_lds_kernel<<<1, kRoadThreads, 0, s>>>(n, g->row_off, g->col, g->w, hq, road_delta(g, true),

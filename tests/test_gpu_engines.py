@@ -335,6 +335,24 @@ def test_road_sssp_past_16_bit_distances(gpu):
         assert np.array_equal(got.values, want), hi
 
 
+def test_road_hand_back_counts_both_kernels(gpu):
+    """A query that the on-chip road kernel hands back (a distance past 16 bits) reports the time of both kernels:
+    elapsed_ms covers the two launches that the profile names."""
+    import graphone_amd as g1
+    h = g1.HostGraph.grid(60, 60, 0.7, seed=11).assign_weights(1, 4000, seed=12, symmetric=True)
+    want = oracle.dijkstra(h.row_offsets, h.col_indices, h.weights, 5)
+    assert int(want[want != 0xFFFFFFFF].max()) > 0xFFFF
+    g = g1.Graph(h, symmetric=True)
+    g.sssp(5, "advance")
+    g.profile(True)
+    g.read_profile()
+    got = g.sssp(5, "advance")
+    road = [e for e in g.read_profile() if e["name"] == "road_sssp"]
+    assert np.array_equal(got.values, want)
+    assert len(road) == 1 and road[0]["launches"] == 2
+    assert got.stats["elapsed_ms"] >= 0.99 * road[0]["total_ms"]
+
+
 @pytest.mark.parametrize("n, deg", [(1, 0), (2, 1), (300, 16), (46080, 5), (46081, 7), (120000, 16)])
 def test_road_engine_shapes(gpu, n, deg):
     """The one-workgroup engine around its own limits: 46,080 vertices (the last size with distances in LDS) and
