@@ -586,13 +586,11 @@ __device__ __forceinline__ uint32_t wave_merge_search(const uint32_t* __restrict
     while (lo < hi) {
         const uint32_t stride = (hi - lo + kWave - 1) / kWave;
         const uint32_t r = lo + lane * stride;
-        const bool ended = r < hi && static_cast<uint64_t>(row_offsets[r + 1]) + r + 1 <= diag;
+        const bool ended = lane * stride < hi - lo && static_cast<uint64_t>(row_offsets[r + 1]) + r + 1 <= diag;
         const uint32_t k = static_cast<uint32_t>(__popcll(ballot(ended)));  // the first k lanes
         if (k == 0) break;
-        const uint32_t next = lo + (k - 1) * stride + 1;  // row next - 1 ended
-        const uint32_t top = next - 1 + stride;           // row top, if tested, did not
-        lo = next;
-        if (top < hi) hi = top;
+        lo += (k - 1) * stride + 1;                  // row lo - 1 ended
+        if (hi - lo >= stride) hi = lo + stride - 1;  // and row lo - 1 + stride, if tested, did not
     }
     return __builtin_amdgcn_readfirstlane(lo);
 }
@@ -1030,15 +1028,21 @@ spmm_wave_kernel(uint32_t n_rows, uint32_t nnz, uint32_t quarter_steps, bool fin
         }
     }
     const uint32_t r0 = first, r_last = __builtin_amdgcn_readfirstlane(s_row[wave + 1]);
-    const uint32_t q0 = static_cast<uint32_t>(quarter(wave) - r0), q1 = static_cast<uint32_t>(quarter(wave + 1) - r_last);
+    // Nonzeros are counted from `base` on, the block of 64 that holds the quarter's first one, so that no sum of a
+    // position and a chunk or a run passes 32 bits, however many nonzeros the matrix has (up to 2^32 - 2).
+    const uint32_t first_nz = static_cast<uint32_t>(quarter(wave) - r0);
+    const uint32_t base = first_nz & ~63u;
+    col += base;
+    if (kValues) vals += base;
+    const uint32_t q0 = first_nz - base, q1 = static_cast<uint32_t>(quarter(wave + 1) - r_last) - base;
 
     // row ends of 64 consecutive rows, one per lane, read out with readlane
     uint32_t rbase = r0;
-    uint32_t rwin = row_offsets[rbase + 1 + lane <= n_rows ? rbase + 1 + lane : n_rows];
+    uint32_t rwin = row_offsets[lane < n_rows - rbase ? rbase + 1 + lane : n_rows] - base;
     auto row_end = [&](uint32_t r) -> uint32_t {
         if (r - rbase >= 64u) {
             rbase = r;
-            rwin = row_offsets[rbase + 1 + lane <= n_rows ? rbase + 1 + lane : n_rows];
+            rwin = row_offsets[lane < n_rows - rbase ? rbase + 1 + lane : n_rows] - base;
         }
         return __builtin_amdgcn_readlane(rwin, r - rbase);
     };
@@ -1111,7 +1115,7 @@ spmm_wave_kernel(uint32_t n_rows, uint32_t nnz, uint32_t quarter_steps, bool fin
                 cv = __builtin_nontemporal_load(col + q);
                 if (kValues) wv = __builtin_bit_cast(uint32_t, __builtin_nontemporal_load(vals + q));
                 if constexpr (P::kScale) {
-                    if (pol.scale_streams()) sB = __builtin_bit_cast(uint32_t, pol.scale_at(q));
+                    if (pol.scale_streams()) sB = __builtin_bit_cast(uint32_t, pol.scale_at(base + q));
                 }
             }
         };

@@ -352,3 +352,31 @@ def test_spmm_x_past_4_gib(gpu):
     f = [1 + int(c) % 7 for c in ci]
     want = np.stack([base * (f[0] + 2 * f[1]), 0 * base, base * (3 * f[2] + 4 * f[3] + 5 * f[4])])
     assert np.array_equal(dY.numpy().reshape(3, k), want.astype(np.float32))  # small whole numbers: exact
+
+
+@pytest.mark.parametrize("short", [2, 17])
+def test_spmm_nnz_near_2_32(gpu, short):
+    """As many nonzeros as the SpMM takes (2^32 - 2) and the first count that passes no multiple of 16 below 2^32: the
+    last rows' products are added like any others. Row 0 holds source 0 all but 700 times; plus-times sums are
+    whole numbers, exact in 64 bits and rounded to 32 once."""
+    g1 = _g1()
+    m = (1 << 32) - short
+    tail = np.random.default_rng(short).integers(1, 1024, 700).astype(np.uint32)
+    rp = np.array([0, m - 700, m - 300, m - 300, m], np.uint32)
+    ci = g1.DeviceArray(m, np.uint32)
+    ci.fill(0)
+    g1._lib.call("g1_memcpy_h2d", C.c_void_p(ci.ptr + 4 * (m - 700)), tail.ctypes.data_as(C.c_void_p),
+                 C.c_size_t(4 * 700), None)
+    x = np.random.default_rng(1).integers(1, 1000, 1024).astype(np.uint32)
+    x[0] = 1
+    x[tail[-3:]] = [0, 1001, 2000]  # the last nonzeros decide row 3
+    drp, dx, dxf = _dev(rp), _dev(x), _dev(x.astype(np.float32))
+    wsb = g1._lib.lib().g1_spmm_workspace_bytes(4, m)
+    ws = g1.DeviceArray((wsb + 3) // 4, np.uint32)
+    dy, dyf = g1.DeviceArray(4, np.uint32), g1.DeviceArray(4, np.float32)
+    _call("g1_spmm_minplus_u32", 4, 1024, m, 1, _p(drp), _p(ci), None, _p(dx), _p(dy), None, _p(ws), C.c_size_t(wsb), None)
+    _call("g1_spmm_plustimes_f32", 4, 1024, m, 1, _p(drp), _p(ci), None, _p(dxf), _p(dyf), None, _p(ws), C.c_size_t(wsb),
+          None)
+    xt = x[tail].astype(np.int64)
+    assert dy.numpy().tolist() == [2, int(xt[:400].min()) + 1, INF, int(xt[400:].min()) + 1]
+    assert dyf.numpy().tolist() == [float(np.float32(m - 700)), float(xt[:400].sum()), 0.0, float(xt[400:].sum())]
