@@ -274,7 +274,7 @@ g1_status launch_plustimes(g1_graph* g, const float* X, float* Y, void* recs_v, 
     bool done = false;
     if constexpr (K == 64) {
         if (ppr_wave()) {
-            launch_spmm_wave<PlusTimesF32>(g->n, g->m, tiles, kMergeTile, false, g->t_row_off, g->t_col, vals,
+            launch_spmm_wave<PlusTimesF32>(g->n, g->m, false, g->t_row_off, g->t_col, vals,
                                            merge_coords(g->t_ws), recs, pol,
                                            static_cast<uint64_t>(g->n) * K * sizeof(float), s);
             G1_LAUNCHED();
@@ -301,7 +301,7 @@ g1_status launch_rank64(g1_graph* g, const float* R_old, float* R_new, const flo
     const uint32_t tiles = merge_num_tiles(g->n, g->m);
     RankBatchPolicy pol{R_old, R_new, g->iw, iw_nz, g->seeds_dev, restart, state};
     auto* recs = static_cast<SpmmTileRec<PlusTimesF32, 64>*>(recs_v);
-    launch_spmm_wave<PlusTimesF32>(g->n, g->m, tiles, kMergeTile, false, g->t_row_off, g->t_col, g->t_wf,
+    launch_spmm_wave<PlusTimesF32>(g->n, g->m, false, g->t_row_off, g->t_col, g->t_wf,
                                    merge_coords(g->t_ws), recs, pol, static_cast<uint64_t>(g->n) * 256, s);
     G1_LAUNCHED();
     if (tiles > 1) {

@@ -106,20 +106,25 @@ g1_status advance(uint32_t n, const uint32_t* row_off, const uint32_t* col, cons
     return G1_OK;
 }
 
-// Merge steps of an SpMM tile (a workgroup; a wave takes a quarter): 2048, halved down to 256 while the matrix
-// gives the chip fewer than 8,192 waves, all that it holds at once. A wave's steps are a chain of loads, sixteen
-// sources at a time: 330 K rows and nonzeros x 8 columns take 25 us at 256 (86 at 2048), 1.3 M x 100 columns 121 us
-// (240 at 2048).
-uint32_t spmm_tile_items(uint32_t n_rows, uint32_t nnz) {
+// Whether the SpMM splits the quarters of its merge tiles over eight waves each (spmm_wave_kernel): a wave's steps are a
+// chain of loads, sixteen sources at a time, so a matrix whose quarters fill less than half of the 8,192 waves that the
+// chip holds takes shorter chains. Whole quarters against split ones, R-MAT rows: 0.33 M rows and nonzeros x 64 columns
+// 66 and 25 us, 1.1 M x 64 77 and 56, 1.3 M x 100 163 and 119, 2.2 M x 64 93 and 92 (x 8: 91 and 88), 3.1 M x 64 106
+// and 120, 4.0 M x 8 133 and 146.
+constexpr uint32_t kSplitParts = 8;
+bool spmm_split(uint32_t n_rows, uint32_t nnz) { return (static_cast<uint64_t>(n_rows) + nnz) / kQuarter < 4096; }
+
+// The steps per record that g1_spmm_workspace_bytes allows for: 2048, halved down to 256 while the matrix has fewer
+// than 8,192 quarters of that. At least what the split needs (a record per 512 steps).
+uint32_t spmm_ws_items(uint32_t n_rows, uint32_t nnz) {
     const uint64_t total = static_cast<uint64_t>(n_rows) + nnz;
     uint32_t items = kMergeTile;
     while (items > kMergeTile / 8 && total / (items / 4) < 8192) items /= 2;
     return items;
 }
 
-// SpMM workspace: the tiles' starts, then their records of one 64-column pass (sized for the larger record, the
-// plus-times one). A smaller one, down to that of tiles of 2048 steps, is taken too: the tiles are then the smallest
-// that it holds.
+// SpMM workspace for records of `items` merge steps: their starts, then one 64-column pass's records (sized for the
+// larger one, the plus-times record).
 size_t spmm_ws_bytes(uint32_t n_rows, uint32_t nnz, uint32_t items) {
     const size_t t = merge_num_tiles_for(n_rows, nnz, items);
     return al((t + 1) * sizeof(MergeCoord)) + t * sizeof(SpmmTileRec<PlusTimesF32, 64>) + 256;
@@ -134,32 +139,42 @@ g1_status spmm(uint32_t n_rows, uint32_t n_cols, uint32_t nnz, uint32_t k, const
     G1_CHECK(n_cols > 0 || nnz == 0, G1_ERR_INVALID_ARG, "%s: nnz > 0 with zero columns", what);
     G1_CHECK(nnz < kInf, G1_ERR_INVALID_ARG, "%s: nnz must be below 2^32-1", what);
     if (n_rows == 0 || k == 0) return G1_OK;
-    uint32_t items = spmm_tile_items(n_rows, nnz);
-    while (items < kMergeTile && ws_bytes < spmm_ws_bytes(n_rows, nnz, items)) items *= 2;
-    G1_CHECK(ws != nullptr && ws_bytes >= spmm_ws_bytes(n_rows, nnz, items), G1_ERR_INVALID_ARG,
+    G1_CHECK(ws != nullptr && ws_bytes >= spmm_ws_bytes(n_rows, nnz, kMergeTile), G1_ERR_INVALID_ARG,
              "%s: workspace of %zu bytes, %zu needed (g1_spmm_workspace_bytes)", what, ws_bytes,
-             spmm_ws_bytes(n_rows, nnz, items));
+             spmm_ws_bytes(n_rows, nnz, kMergeTile));
+    // (a workspace too small for the quarters' records gets the same sums, from a wave a quarter)
+    const bool split = spmm_split(n_rows, nnz) && ws_bytes >= spmm_ws_bytes(n_rows, nnz, kQuarter);
+    const uint32_t items = split ? kQuarter : kMergeTile;
     const uint32_t tiles = merge_num_tiles_for(n_rows, nnz, items);
     MergeCoord* coords = merge_coords(ws);
     auto* recs = reinterpret_cast<SpmmTileRec<S, 64>*>(static_cast<char*>(ws) + al((tiles + 1ull) * sizeof(MergeCoord)));
-    // While every tile is resident at once, a search over all the rows in each wave (three or four loads) costs less
-    // than a launch that partitions the matrix (10 us); beyond, the searches would add up.
+    // Up to 2048 tiles or quarters a search over all the rows in each wave (three or four loads) costs less than a
+    // launch that partitions the matrix (10 us); beyond, the searches add up (2.2 M rows and nonzeros in split quarters
+    // 93 us with them, 92 with a partition; 3.1 M 124 and 120).
     const bool find = tiles <= 2048;
     if (!find) {
         merge_partition_kernel<<<(tiles + 1 + 255) / 256, 256, 0, s>>>(row_off, n_rows, nnz, tiles, coords, items);
         G1_LAUNCHED();
     }
     using T = typename S::x_t;
-    const T neutral = std::is_same_v<S, MinPlusU32> ? static_cast<T>(kInf) : T(0);
+    using P = StridedColumnsPolicy<T>;
+    const uint64_t x_bytes = static_cast<uint64_t>(n_cols) * k * sizeof(T);
     for (uint32_t c0 = 0; c0 < k; c0 += 64) {
-        StridedColumnsPolicy<T> pol{X, Y, k, c0, std::min<uint32_t>(64u, k - c0), mask, neutral};
-        launch_spmm_wave<S>(n_rows, nnz, tiles, items, find && c0 == 0, row_off, col, vals, coords, recs, pol,
-                            static_cast<uint64_t>(n_cols) * k * sizeof(T), s);
-        G1_LAUNCHED();
-        if (tiles > 1) {
-            spmm_fixup_kernel<S, 64, StridedColumnsPolicy<T>><<<(tiles * 64u + 255) / 256, 256, 0, s>>>(
-                tiles, coords, recs, pol, nullptr);
+        P pol{X, Y, k, c0, std::min<uint32_t>(64u, k - c0), mask};
+        if (split) {
+            launch_spmm_wave<S, kSplitParts>(n_rows, nnz, find && c0 == 0, row_off, col, vals, coords, recs, pol, x_bytes, s);
             G1_LAUNCHED();
+            if (tiles > 1) {
+                spmm_quarter_fixup_kernel<S, P><<<(tiles + 3) / 4, 256, 0, s>>>(tiles, coords, recs, pol);
+                G1_LAUNCHED();
+            }
+        } else {
+            launch_spmm_wave<S>(n_rows, nnz, find && c0 == 0, row_off, col, vals, coords, recs, pol, x_bytes, s);
+            G1_LAUNCHED();
+            if (tiles > 1) {
+                spmm_fixup_kernel<S, 64, P><<<(tiles + 3) / 4, 256, 0, s>>>(tiles, coords, recs, pol, nullptr);
+                G1_LAUNCHED();
+            }
         }
     }
     return G1_OK;
@@ -292,7 +307,7 @@ g1_status g1_l1_delta_f64(uint32_t n, const float* a, const float* b, double* ou
 }
 
 size_t g1_spmm_workspace_bytes(uint32_t n_rows, uint32_t nnz) {
-    return spmm_ws_bytes(n_rows, nnz, spmm_tile_items(n_rows, nnz));
+    return spmm_ws_bytes(n_rows, nnz, spmm_ws_items(n_rows, nnz));
 }
 
 g1_status g1_spmm_minplus_u32(uint32_t n_rows, uint32_t n_cols, uint32_t nnz, uint32_t k, const uint32_t* row_offsets,

@@ -576,6 +576,8 @@ __global__ void __launch_bounds__(256) spmm_fixup_kernel(uint32_t num_tiles, con
 // ------------------------------------------------------------------------------------------------
 // x rows that a wave of the 64-column kernels below keeps in flight.
 constexpr uint32_t kWaveChunk = 16;
+// Merge steps of a quarter of a merge tile: what a wave of spmv_merge_tile_kernel folds.
+constexpr uint32_t kQuarter = kMergeTile / kMergeWaves;
 static_assert(64 % kWaveChunk == 0, "a block of 64 indices holds whole chunks");
 
 // The number of rows of [lo, hi) that end before merge step `diag`: row r does when row_offsets[r + 1] + r + 1 <=
@@ -966,7 +968,12 @@ struct RankBatchPolicy {
 // single-source runs.
 //
 // Quarters, because a wave per tile left too few waves: 11 M rows and nonzeros are 5,300 tiles for 8,192
-// resident waves, and each wave's chain of loads is then as long as the launch.
+// resident waves, and each wave's chain of loads is then as long as the launch. Where quarters are too few as well
+// (small matrices, see spmm_split in step.hip) a workgroup of kParts waves takes one quarter: the order of the sums is
+// that of the quarter's 64 runs, so a wave keeps the tails of its runs in LDS up to the first that closes a row, and
+// what a row holds in the waves before it is folded in front of them once all are done (32 KB of LDS at eight waves
+// of eight runs, 32 waves a CU). The records are then the quarters', and spmm_quarter_fixup_kernel folds them.
+//
 // What bounds it is the x rows, 256 bytes per nonzero, as long as the walk keeps out of their way; the walk is
 // one wave-uniform stream, so its scalar instructions are what it is made of. The x rows go to registers
 // kWaveChunk at a time: a chunk's products are formed from the rows loaded during the chunk before, the next
@@ -982,41 +989,47 @@ struct RankBatchPolicy {
 // P: init(lane) once per wave; x<kWide>(u, lane) the lane's value of source u, loaded unconditionally (a
 // column the policy leaves out may read any valid element: its products are never stored), times scale(u) where
 // kScale says so (scale_at(e) of nonzero e instead where scale_streams() does, uniform); store(row, lane, y).
-template <typename S, bool kValues, bool kWide, typename P>
-__global__ void __launch_bounds__(256)
-spmm_wave_kernel(uint32_t n_rows, uint32_t nnz, uint32_t quarter_steps, bool find,
-                 const uint32_t* __restrict__ row_offsets, const uint32_t* __restrict__ col,
-                 const typename S::value_t* __restrict__ vals, MergeCoord* __restrict__ coords,
-                 SpmmTileRec<S, 64>* __restrict__ recs, P pol) {
+template <typename S, bool kValues, bool kWide, uint32_t kParts, typename P>
+__global__ void __launch_bounds__(kParts == 1 ? 256 : kParts * kWave)
+spmm_wave_kernel(uint32_t n_rows, uint32_t nnz, bool find, const uint32_t* __restrict__ row_offsets,
+                 const uint32_t* __restrict__ col, const typename S::value_t* __restrict__ vals,
+                 MergeCoord* __restrict__ coords, SpmmTileRec<S, 64>* __restrict__ recs, P pol) {
     using acc_t = typename S::acc_t;
     using value_t = typename S::value_t;
     using x_t = typename S::x_t;
     using y_t = typename S::y_t;
     static_assert(sizeof(value_t) == 4, "values travel through readlane");
-    __shared__ acc_t s_carry[kMergeWaves][64];
-    __shared__ uint32_t s_ends[kMergeWaves];
-    __shared__ uint32_t s_row[kMergeWaves + 1];
+    constexpr bool kSplit = kParts > 1;
+    constexpr uint32_t kWaves = kSplit ? kParts : kMergeWaves;
+    constexpr uint32_t kSteps = kQuarter / kParts;      // merge steps of a wave
+    constexpr uint32_t kRuns = kSteps / kMergeItems;
+    constexpr uint64_t kTileSteps = kWaves * kSteps;
+    __shared__ acc_t s_carry[kWaves][64];
+    __shared__ acc_t s_tail[kSplit ? kWaves : 1][kSplit ? kRuns : 1][64];  // the runs before the first that closes a row
+    __shared__ uint32_t s_tails[kWaves];                                   // ... and their number
+    __shared__ uint32_t s_ends[kWaves];
+    __shared__ uint32_t s_row[kWaves + 1];
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t tile = blockIdx.x;
     pol.init(lane);
 
-    // The quarters' bounds: the merge-path search of the wave's first step, 64 rows at a time, within the tile's rows
+    // The waves' bounds: the merge-path search of the wave's first step, 64 rows at a time, within the tile's rows
     // or, when the caller has no partition, in all of them (the tile's start then goes to coords for the fixup).
     MergeCoord c0{0, 0}, c1{n_rows, nnz};
     const uint64_t total = static_cast<uint64_t>(n_rows) + nnz;
-    const uint64_t step0 = static_cast<uint64_t>(tile) * (4ull * quarter_steps);
-    const uint64_t step1 = step0 + 4ull * quarter_steps < total ? step0 + 4ull * quarter_steps : total;
-    auto quarter = [&](uint32_t w) { return step0 + w * static_cast<uint64_t>(quarter_steps) < step1 ? step0 + w * static_cast<uint64_t>(quarter_steps) : step1; };
+    const uint64_t step0 = tile * kTileSteps;
+    const uint64_t step1 = step0 + kTileSteps < total ? step0 + kTileSteps : total;
+    auto part_start = [&](uint32_t w) { return step0 + w * kSteps < step1 ? step0 + w * kSteps : step1; };
     if (!find) {
         c0 = coords[tile];
         c1 = coords[tile + 1];
     }
-    const uint32_t first = wave_merge_search(row_offsets, c0.x, c1.x, quarter(wave));
-    if (find && wave == kMergeWaves - 1) c1.x = wave_merge_search(row_offsets, first, n_rows, step1);
+    const uint32_t first = wave_merge_search(row_offsets, c0.x, c1.x, part_start(wave));
+    if (find && wave == kWaves - 1) c1.x = wave_merge_search(row_offsets, first, n_rows, step1);
     if (lane == 0) {
         s_row[wave] = first;
-        if (wave == kMergeWaves - 1) s_row[kMergeWaves] = c1.x;
+        if (wave == kWaves - 1) s_row[kWaves] = c1.x;
     }
     __syncthreads();
     if (find) {
@@ -1028,13 +1041,13 @@ spmm_wave_kernel(uint32_t n_rows, uint32_t nnz, uint32_t quarter_steps, bool fin
         }
     }
     const uint32_t r0 = first, r_last = __builtin_amdgcn_readfirstlane(s_row[wave + 1]);
-    // Nonzeros are counted from `base` on, the block of 64 that holds the quarter's first one, so that no sum of a
+    // Nonzeros are counted from `base` on, the block of 64 that holds the wave's first one, so that no sum of a
     // position and a chunk or a run passes 32 bits, however many nonzeros the matrix has (up to 2^32 - 2).
-    const uint32_t first_nz = static_cast<uint32_t>(quarter(wave) - r0);
+    const uint32_t first_nz = static_cast<uint32_t>(part_start(wave) - r0);
     const uint32_t base = first_nz & ~63u;
     col += base;
     if (kValues) vals += base;
-    const uint32_t q0 = first_nz - base, q1 = static_cast<uint32_t>(quarter(wave + 1) - r_last) - base;
+    const uint32_t q0 = first_nz - base, q1 = static_cast<uint32_t>(part_start(wave + 1) - r_last) - base;
 
     // row ends of 64 consecutive rows, one per lane, read out with readlane
     uint32_t rbase = r0;
@@ -1055,24 +1068,28 @@ spmm_wave_kernel(uint32_t n_rows, uint32_t nnz, uint32_t quarter_steps, bool fin
     bool hasend = false, any_end = false;
     uint32_t first_row = 0;
 
-    acc_t part = S::identity();  // the first row the quarter closes, as far as the quarter holds it
+    acc_t part = S::identity();  // the first row the wave closes, as far as the wave (kSplit: its run) holds it
     uint32_t part_row = 0;
+    uint32_t tails = 0;
 
-    // End of a run of 8 steps (the same folds as merge_walk's, per column).
+    // End of a run of 8 steps (the same folds as merge_walk's, per column). What is folded in front of a split
+    // quarter's first closed row waits in LDS until the waves before this one are done.
     auto run_end = [&]() {
         if (hasend) {
-            const acc_t whole = S::merge(chain, head);
             if (any_end) {
-                pol.store(first_row, lane, S::finalize(whole));
+                pol.store(first_row, lane, S::finalize(S::merge(chain, head)));
             } else {
-                part = whole;
+                part = kSplit ? head : S::merge(chain, head);
                 part_row = first_row;
             }
             chain = acc;
             any_end = true;
             hasend = false;
-        } else {
+        } else if (!kSplit || any_end) {
             chain = S::merge(chain, acc);
+        } else if (tails < kRuns) {  // (a run past the last step holds nothing)
+            s_tail[kSplit ? wave : 0][kSplit ? tails : 0][lane] = acc;
+            ++tails;
         }
         acc = S::identity();
     };
@@ -1183,25 +1200,39 @@ spmm_wave_kernel(uint32_t n_rows, uint32_t nnz, uint32_t quarter_steps, bool fin
     run_end();
 
     s_carry[wave][lane] = chain;
-    if (lane == 0) s_ends[wave] = any_end;
+    if (lane == 0) {
+        s_ends[wave] = any_end;
+        s_tails[wave] = tails;
+    }
     __syncthreads();
-    // The carries of the quarters before w since the last one that closed a row (merge_wave_chain).
+    // The fold in front of wave w since the last wave before it that closed a row: the quarters' carries
+    // (merge_wave_chain), or in a split quarter that wave's carry and the tails of the runs after it.
     auto outer = [&](int w, bool& any) {
         int u = w - 1;
         while (u > 0 && !s_ends[u]) --u;
         any = u >= 0 && s_ends[u] != 0u;
         acc_t sum = S::identity();
-        for (int v = u > 0 ? u : 0; v < w; ++v) sum = S::merge(sum, s_carry[v][lane]);
+        int v = u > 0 ? u : 0;
+        if constexpr (kSplit) {
+            if (any) sum = s_carry[v++][lane];
+            for (; v < w; ++v)
+                for (uint32_t k = 0; k < s_tails[v]; ++k) sum = S::merge(sum, s_tail[v][k][lane]);
+        } else {
+            for (; v < w; ++v) sum = S::merge(sum, s_carry[v][lane]);
+        }
         return sum;
     };
     bool before;
     if (any_end) {
-        const acc_t whole = S::merge(outer(static_cast<int>(wave), before), part);
+        acc_t chain = outer(static_cast<int>(wave), before);
+        if constexpr (kSplit)
+            for (uint32_t k = 0; k < tails; ++k) chain = S::merge(chain, s_tail[wave][k][lane]);
+        const acc_t whole = S::merge(chain, part);
         if (!before && row_offsets[part_row] < c0.y) recs[tile].head[lane] = whole;
         else pol.store(part_row, lane, S::finalize(whole));
     }
-    if (wave == kMergeWaves - 1) {
-        recs[tile].carry[lane] = outer(kMergeWaves, before);
+    if (wave == kWaves - 1) {
+        recs[tile].carry[lane] = outer(kWaves, before);
         if (lane == 0) {
             uint32_t flags = before ? kTileHasEnd : 0u;
             if (before && row_offsets[c0.x] < c0.y) flags |= kTileDeferred;
@@ -1210,24 +1241,71 @@ spmm_wave_kernel(uint32_t n_rows, uint32_t nnz, uint32_t quarter_steps, bool fin
     }
 }
 
-// One pass of the wave kernel over `tiles` tiles of tile_items merge steps; x_bytes is the size of the x array the
-// policy reads. With `find` the waves search the whole matrix for their bounds and leave the tiles' starts in
-// coords, otherwise coords holds the partition.
+// spmm_fixup_kernel for records of quarters: a wave per quarter finishes its deferred first row. The carries of
+// the quarters that the row crosses are folded tile by tile, and the tiles' sums left to right in front of the
+// last tile's, as the merge kernels fold them.
 template <typename S, typename P>
-inline void launch_spmm_wave(uint32_t n_rows, uint32_t nnz, uint32_t tiles, uint32_t tile_items, bool find,
-                             const uint32_t* row_off, const uint32_t* col, const typename S::value_t* vals,
-                             MergeCoord* coords, SpmmTileRec<S, 64>* recs, const P& pol, uint64_t x_bytes,
-                             hipStream_t s) {
+__global__ void __launch_bounds__(256) spmm_quarter_fixup_kernel(uint32_t quarters, const MergeCoord* __restrict__ coords,
+                                                                 const SpmmTileRec<S, 64>* __restrict__ recs, P pol) {
+    using acc_t = typename S::acc_t;
+    const uint32_t t = (blockIdx.x * 256 + threadIdx.x) / 64;
+    const uint32_t j = threadIdx.x % 64;
+    if (t == 0 || t >= quarters || (recs[t].flags & kTileDeferred) == 0u) return;
+    uint32_t u = t - 1;  // the nearest quarter before t that closes a row, or the first: 64 tested at a time
+    for (;;) {
+        const uint64_t hits = ballot(j <= u && (recs[u - (j <= u ? j : 0u)].flags & kTileHasEnd) != 0u);
+        if (hits) {
+            u -= static_cast<uint32_t>(__builtin_ctzll(hits));
+            break;
+        }
+        if (u < 64) {
+            u = 0;
+            break;
+        }
+        u -= 64;
+    }
+    acc_t tiles = S::identity(), tile = S::identity();
+    bool crossed = false;
+    auto add = [&](uint32_t v, acc_t carry) {
+        tile = S::merge(tile, carry);
+        if (v % kMergeWaves == kMergeWaves - 1) {
+            tiles = S::merge(tiles, tile);
+            tile = S::identity();
+            crossed = true;
+        }
+    };
+    uint32_t v = u;
+    for (; v + 8 <= t; v += 8) {
+        acc_t cv[8];
+#pragma unroll
+        for (uint32_t i = 0; i < 8; ++i) cv[i] = recs[v + i].carry[j];
+#pragma unroll
+        for (uint32_t i = 0; i < 8; ++i) add(v + i, cv[i]);
+    }
+    for (; v < t; ++v) add(v, recs[v].carry[j]);
+    const acc_t last = S::merge(tile, recs[t].head[j]);
+    pol.row_done(coords[t].x, j, S::finalize(crossed ? S::merge(tiles, last) : last), typename S::x_t(0));
+}
+
+// One pass of the wave kernel, over tiles of kMergeTile steps or (kParts > 1) quarters of them; x_bytes is the size of
+// the x array the policy reads. With `find` the waves search the whole matrix for their bounds and leave the tiles'
+// (quarters') starts in coords, otherwise coords holds the partition.
+template <typename S, uint32_t kParts = 1, typename P>
+inline void launch_spmm_wave(uint32_t n_rows, uint32_t nnz, bool find, const uint32_t* row_off, const uint32_t* col,
+                             const typename S::value_t* vals, MergeCoord* coords, SpmmTileRec<S, 64>* recs, const P& pol,
+                             uint64_t x_bytes, hipStream_t s) {
     const bool wide = x_bytes >= (1ull << 32);
+    constexpr bool kSplit = kParts > 1;
+    const uint32_t blocks = merge_num_tiles_for(n_rows, nnz, kSplit ? kQuarter : kMergeTile);
     auto go = [&](auto kernel) {
-        kernel<<<tiles, 256, 0, s>>>(n_rows, nnz, tile_items / 4, find, row_off, col, vals, coords, recs, pol);
+        kernel<<<blocks, kSplit ? kParts * kWave : 256, 0, s>>>(n_rows, nnz, find, row_off, col, vals, coords, recs, pol);
     };
     if (vals) {
-        if (wide) go(spmm_wave_kernel<S, true, true, P>);
-        else go(spmm_wave_kernel<S, true, false, P>);
+        if (wide) go(spmm_wave_kernel<S, true, true, kParts, P>);
+        else go(spmm_wave_kernel<S, true, false, kParts, P>);
     } else {
-        if (wide) go(spmm_wave_kernel<S, false, true, P>);
-        else go(spmm_wave_kernel<S, false, false, P>);
+        if (wide) go(spmm_wave_kernel<S, false, true, kParts, P>);
+        else go(spmm_wave_kernel<S, false, false, kParts, P>);
     }
 }
 

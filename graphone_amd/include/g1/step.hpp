@@ -262,18 +262,15 @@ step_pr_apply_kernel(uint32_t n, const float* __restrict__ y, float base, const 
     if (threadIdx.x == 0) partials[blockIdx.x] = ((s_q[0] + s_q[1]) + s_q[2]) + s_q[3];
 }
 
-// Semiring SpMM, Y = A (x) X with k dense columns stored row-major (X: n_cols x k, Y: n_rows x k), on the
-// merge-path tile kernels of the batched engines (spmm_tile_kernel + spmm_fixup_kernel at 64 columns per
-// pass): every tile holds the same number of rows plus nonzeros, so a hub row is spread over many tiles
-// instead of one wave. This policy reads and writes the 64-column chunk starting at column c0 of the
-// caller's arrays (row stride ld = k); lanes past the chunk's kc columns, and columns whose bit is clear in
-// the device mask (bit j of word j / 64; null: every column), read nothing and write nothing, so their Y
-// values stay. Plus-times folds in the single-source merge-path SpMV's order (64-bit sums), min-plus is
-// order-free.
+// Semiring SpMM, Y = A (x) X with k dense columns stored row-major (X: n_cols x k, Y: n_rows x k), on
+// spmm_wave_kernel at 64 columns per pass: every wave takes the same number of rows plus nonzeros, so a hub row is
+// spread over many waves instead of one. This policy reads and writes the 64-column chunk starting at column c0 of
+// the caller's arrays (row stride ld = k). Lanes past the chunk's kc columns, and columns whose bit is clear in the
+// device mask (bit j of word j / 64; null: every column), read column 0 and write nothing, so their Y values stay.
+// Plus-times folds in the single-source merge-path SpMV's order (64-bit sums), whichever way the work is split;
+// min-plus is order-free.
 template <typename T>
 struct StridedColumnsPolicy {
-    using aux_t = uint32_t;
-    static constexpr bool kHasAux = false;
     static constexpr bool kRowOld = false;
     static constexpr bool kScale = false;
     const T* X;
@@ -282,9 +279,11 @@ struct StridedColumnsPolicy {
     uint32_t c0;  // first column of the chunk
     uint32_t kc;  // columns in the chunk (<= 64)
     const unsigned long long* mask;
-    T neutral;    // what a skipped column reads (the semiring's absorbing x: INF for min-plus, 0 for plus-times)
-    uint32_t jc = 0;    // spmm_wave_kernel: the column this lane reads (its own, or 0 when it stores nothing)
+    uint32_t jc = 0;  // the column this lane reads (its own, or 0 when it stores nothing)
     bool mine = false;
+    __device__ __forceinline__ bool on(uint32_t j) const {
+        return j < kc && (!mask || ((mask[(c0 + j) >> 6] >> ((c0 + j) & 63u)) & 1ull));
+    }
     __device__ __forceinline__ void init(uint32_t j) {
         mine = on(j);
         jc = mine ? c0 + j : 0u;
@@ -297,14 +296,7 @@ struct StridedColumnsPolicy {
     __device__ __forceinline__ void store(uint32_t row, uint32_t, T y) const {
         if (mine) Y[static_cast<size_t>(row) * ld + jc] = y;
     }
-    __device__ __forceinline__ bool on(uint32_t j) const {
-        return j < kc && (!mask || ((mask[(c0 + j) >> 6] >> ((c0 + j) & 63u)) & 1ull));
-    }
-    __device__ __forceinline__ aux_t aux(uint32_t) const { return 0u; }
-    __device__ __forceinline__ T x(uint32_t u, aux_t, uint32_t j, bool has) const {
-        return (has && on(j)) ? X[static_cast<size_t>(u) * ld + c0 + j] : neutral;
-    }
-    __device__ __forceinline__ T row_old(uint32_t, uint32_t) const { return neutral; }
+    // the fixup kernels
     __device__ __forceinline__ uint64_t row_done(uint32_t row, uint32_t j, T y, T) const {
         if (on(j)) Y[static_cast<size_t>(row) * ld + c0 + j] = y;
         return 0ull;

@@ -205,12 +205,15 @@ g1_status g1_l1_delta_f64(uint32_t n, const float* a_dev, const float* b_dev, do
  * the reference's SpMM boundary (include/GraphOne/archi/blas/spmm/cuda/cuda.cuh:65-116, the GNN aggregation
  * of include/GraphOne/engine/blas_gnn.h:18-122) and serving batched multi-source steps:
  *   min-plus u32 : Y[r][j] = min over the nonzeros (r, c) of (X[c][j] == G1_INF ? G1_INF : A[r,c] + X[c][j])
- *   plus-times f32: Y[r][j] = sum over the nonzeros of A[r,c] * X[c][j], left to right per row with the
- *                  64-bit sum of the SpMV kernels
+ *   plus-times f32: Y[r][j] = sum over the nonzeros of A[r,c] * X[c][j], in 64 bits and in the order of the
+ *                  merge-path SpMV
  * col_mask_dev (device, ceil(k / 64) words; NULL = every column): only the columns whose bit is set are
  * computed, the others keep their Y values. values_dev NULL: unit values. The rows and nonzeros are
  * cut into merge-path tiles of equal size (a row of any length spreads over tiles), 64 columns per pass;
- * the workspace (the partition and the tiles' carries) is g1_spmm_workspace_bytes(n_rows, nnz) bytes. */
+ * the workspace (the partition and the tiles' carries) is g1_spmm_workspace_bytes(n_rows, nnz) bytes. One for records
+ * of 2048 rows and nonzeros each (that size for matrices of 4.2 million or more) is taken as well, at any size: a
+ * small matrix is then cut less finely. The plus-times fold order is a function of the matrix only, and that of
+ * g1_spmv_merge_plustimes_f32: column j has the bits of the SpMV with column j of X, whatever the workspace. */
 size_t g1_spmm_workspace_bytes(uint32_t n_rows, uint32_t nnz);
 g1_status g1_spmm_minplus_u32(uint32_t n_rows, uint32_t n_cols, uint32_t nnz, uint32_t k,
                               const uint32_t* row_offsets_dev, const uint32_t* col_indices_dev,

@@ -380,3 +380,49 @@ def test_spmm_nnz_near_2_32(gpu, short):
     xt = x[tail].astype(np.int64)
     assert dy.numpy().tolist() == [2, int(xt[:400].min()) + 1, INF, int(xt[400:].min()) + 1]
     assert dyf.numpy().tolist() == [float(np.float32(m - 700)), float(xt[:400].sum()), 0.0, float(xt[400:].sum())]
+
+
+@pytest.mark.parametrize("name", ["short", "runs", "parts", "quarters", "tiles", "hub", "mixed", "large"])
+def test_spmm_folds_like_spmv(gpu, name):
+    """Plus-times SpMM adds in the merge-path SpMV's order, whichever workspace it is given: bit for bit the SpMV of every
+    column. Products come as pairs of opposite sign that differ from the sum by 2^40, so that another order shows in
+    the result. Rows around the runs of 8 steps, the parts of 64, quarters of 512 and tiles of 2048 that they are
+    folded by (a row's end is a step too), rows over several of them, and more than 8,192 quarters."""
+    g1 = _g1()
+    rng = np.random.default_rng(len(name) + 5)
+    degs = {"short": rng.integers(0, 6, 4000), "runs": np.array([7] * 900 + [8] * 40), "parts": np.array([63, 64, 62, 0] * 60),
+            "quarters": np.array([511] * 9 + [512, 0, 510, 1030]), "tiles": np.array([2047] * 3 + [4095, 2049, 0, 0, 8191]),
+            "hub": np.array([3, 30011, 0, 1, 5, 70000, 2]), "mixed": rng.choice([0, 1, 5, 40, 300, 3000], 700),
+            "large": rng.choice([0, 3, 9, 200, 20000], 2000, p=[.2, .3, .298, .2, .002])}[name]
+    if name == "large":
+        degs = np.concatenate([degs, np.full(70000, 63)])
+    n_rows, m, half = len(degs), int(degs.sum()), 3000
+    rp = np.concatenate([[0], np.cumsum(degs)]).astype(np.uint32)
+    ci = rng.integers(0, half, m)
+    ci[1::2] = ci[0:m - m % 2:2] + half  # the partner of the one before it ...
+    for r in range(n_rows if name != "large" else 2000):  # ... somewhere in the row
+        ci[rp[r]:rp[r + 1]] = rng.permutation(ci[rp[r]:rp[r + 1]])
+    ci = ci.astype(np.uint32)
+    w = rng.integers(1, 3, m).astype(np.float32)
+    drp, dci, dw = _dev(rp), _dev(np.append(ci, 0).astype(np.uint32)), _dev(np.append(w, 0).astype(np.float32))
+    k = 67
+    big = rng.standard_normal((half, k)) * 2.0 ** rng.integers(0, 41, (half, k))
+    X = np.concatenate([big, -big + rng.standard_normal((half, k))]).astype(np.float32)
+    dX = _dev(X)
+    least = g1._lib.lib().g1_spmm_workspace_bytes(-(-(n_rows + m) // 2048) * 256, 0)
+    least = min(least, g1._lib.lib().g1_spmm_workspace_bytes(n_rows, m))
+    ws = g1.DeviceArray((g1._lib.lib().g1_spmm_workspace_bytes(n_rows, m) + 3) // 4 + 1, np.uint32)
+    mws = g1.merge_workspace(n_rows, m, drp)
+    for values in (dw, None):
+        got = []
+        for wsb in (g1._lib.lib().g1_spmm_workspace_bytes(n_rows, m), least):
+            dY = g1.DeviceArray(n_rows * k, np.float32)
+            _call("g1_spmm_plustimes_f32", n_rows, 2 * half, m, k, _p(drp), _p(dci), _p(values), _p(dX), _p(dY), None,
+                  _p(ws), C.c_size_t(wsb), None)
+            got.append(dY.numpy().reshape(n_rows, k))
+        assert np.array_equal(got[0].view(np.uint32), got[1].view(np.uint32))
+        for j in (0, 1, 31, 63, 64, 66):
+            y = g1.DeviceArray(n_rows, np.float32)
+            x = _dev(X[:, j])
+            g1.spmv("merge", "plustimes_f32", drp, dci, values, x, y, n_rows, 2 * half, m, mws)
+            assert np.array_equal(got[0][:, j].view(np.uint32), y.numpy().view(np.uint32)), j
