@@ -217,20 +217,21 @@ __global__ void __launch_bounds__(64) frontier_post_kernel(const unsigned long l
     }
 }
 
-// Waits until `*word` (in the graph's mailbox) is seq. The host spins on it, yielding its core between polls
+// Waits until here(*word) (a word of the graph's mailbox) holds. The host spins on it, yielding its core between polls
 // after the first 2048 (a dense iteration runs for hundreds of microseconds, and the query server polls from many
 // threads at once); every 1024 polls it asks the stream, and a stream that has drained (or failed) without the
 // post showing is an error.
-g1_status wait_post(const unsigned long long* word, unsigned long long seq, hipStream_t s) {
+template <typename F>
+g1_status wait_word(const unsigned long long* word, hipStream_t s, F&& here) {
     uint32_t polls = 0;
-    while (__atomic_load_n(word, __ATOMIC_ACQUIRE) != seq) {
+    while (!here(__atomic_load_n(word, __ATOMIC_ACQUIRE))) {
         if ((++polls & 1023u) == 0) {
             const hipError_t q = hipStreamQuery(s);
             if (q != hipErrorNotReady) {
-                if (__atomic_load_n(word, __ATOMIC_ACQUIRE) == seq) break;
+                if (here(__atomic_load_n(word, __ATOMIC_ACQUIRE))) break;
                 G1_HIP(q);
                 G1_HIP(hipStreamSynchronize(s));
-                G1_CHECK(__atomic_load_n(word, __ATOMIC_ACQUIRE) == seq, G1_ERR_INTERNAL,
+                G1_CHECK(here(__atomic_load_n(word, __ATOMIC_ACQUIRE)), G1_ERR_INTERNAL,
                          "post missing after the stream drained");
                 break;
             }
@@ -239,6 +240,10 @@ g1_status wait_post(const unsigned long long* word, unsigned long long seq, hipS
         else std::this_thread::yield();
     }
     return G1_OK;
+}
+
+g1_status wait_post(const unsigned long long* word, unsigned long long seq, hipStream_t s) {
+    return wait_word(word, s, [seq](unsigned long long w) { return w == seq; });
 }
 
 // Returns (E << 32) | nf of the frontier in counter set `set`, once the work enqueued on s before it is done.
@@ -306,11 +311,16 @@ uint32_t tail_batch(uint64_t edges) {
     return k;
 }
 
+constexpr uint32_t kAheadPost = 4;  // the mailbox word of a BFS level's post
+
 // Device-driven iteration loop of the push engines. Every launch reads its input frontier's counters
 // on the device and is a no-op once the frontier is empty, so the host enqueues iterations in batches
-// and reads back only the output counters of the last launch of a batch: 2, 4, 8, ... launches while the
-// frontier grows, tail_batch() once it shrinks. With profiling on, the batch is one launch so each
-// launch's counts can be attributed to it.
+// and reads back only the output counters of the last launch of a batch: batch0 (2) launches, twice as many each time
+// up to 32 while the frontier grows, tail_batch() once it shrinks, and batch0 again after a hand-back from the
+// single-workgroup kernel. With ahead the first two launches of the run's second
+// batch go out before the first batch's result is read, and the first of them posts whether its frontier is empty:
+// launch() gets the number to post under (0: none).
+// With profiling on, the batch is one launch so each launch's counts can be attributed to it.
 //
 // With pull_min_edges > 0 an iteration whose frontier has at least that many out-edges runs as one pull
 // step instead (pull(it): scatter, SpMV, apply). The host then needs each frontier's edge count before
@@ -321,7 +331,7 @@ template <typename Launch, typename AfterLaunch, typename Small, typename Pull>
 g1_status drive_push(g1_graph* g, hipStream_t s, Launch&& launch, AfterLaunch&& after, Small&& small,
                      bool small_first, uint32_t* launched, Pull&& pull, uint64_t pull_min_edges, uint32_t it0 = 0,
                      uint64_t first_edges = ~0ull, uint64_t single_min_edges = 0, uint32_t batch0 = 2,
-                     bool lazy_profile = false) {
+                     bool lazy_profile = false, bool ahead = false) {
     if (single_min_edges == 0) single_min_edges = pull_min_edges;
     // With profiling on, launches go one at a time so that `after` can attribute each one's counts, unless
     // the caller attributes them afterwards from the iteration history (lazy_profile): then the launches
@@ -341,6 +351,7 @@ g1_status drive_push(g1_graph* g, hipStream_t s, Launch&& launch, AfterLaunch&& 
             it = res[0];
             if (res[1] == 0) break;
             batch = batch0;
+            ahead = false;
             shrinking = false;
             // the frontier handed back is past the small kernel's size: read it so that this iteration can
             // already be a pull step or a dense launch
@@ -360,11 +371,30 @@ g1_status drive_push(g1_graph* g, hipStream_t s, Launch&& launch, AfterLaunch&& 
             if (single_min_edges && (!known || !shrinking || next_edges >= single_min_edges / 4)) b = 1;
             G1_CHECK(it + b <= kHistIters, G1_ERR_INTERNAL, "push engine exceeded %u iterations", kHistIters);
             for (uint32_t k = 0; k < b; ++k) {
-                G1_TRY(launch(it, k == 0 && known ? next_edges : 0));
+                G1_TRY(launch(it, k == 0 && known ? next_edges : 0, 0));
                 G1_TRY(after(it));
                 ++it;
             }
-            if (batch < 32) batch *= 2;
+            batch = std::min(2 * batch, 32u);
+        }
+        if (ahead && !one_by_one) {
+            ahead = false;
+            G1_CHECK(it + 2 <= kHistIters, G1_ERR_INTERNAL, "push engine exceeded %u iterations", kHistIters);
+            if (static_cast<uint32_t>(++g->post_seq) == 0) ++g->post_seq;
+            const uint32_t seq = static_cast<uint32_t>(g->post_seq);
+            for (uint32_t k = 0; k < 2; ++k) {
+                G1_TRY(launch(it, 0, k == 0 ? seq : 0));
+                G1_TRY(after(it));
+                ++it;
+            }
+            batch -= 2;
+            G1_TRY(wait_word(g->h_mbox + kAheadPost, s, [&](unsigned long long w) {
+                next = w;
+                return w >> 32 == seq;
+            }));
+            if (static_cast<uint32_t>(next) == 0) break;
+            known = shrinking = try_small = false;  // nothing is known of the frontier of iteration `it`
+            continue;
         }
         G1_TRY(read_frontier(g, it % 3, s, &next));
         if (static_cast<uint32_t>(next) == 0) break;
@@ -495,15 +525,17 @@ g1_status run_bfs_push(g1_graph* g, uint32_t src, uint32_t* depth, bool diropt, 
     memset(g->h_ctr, 0, 8 * sizeof(unsigned long long));  // the host mirror of the cleared counters
     G1_HIP(hipEventRecord(g->ev[0], s));
     int tok = -1;
-    auto launch = [&](uint32_t it, uint64_t) -> g1_status {
+    auto launch = [&](uint32_t it, uint64_t, uint32_t post_seq) -> g1_status {
         PushQueues pq = make_queues(g, it);
         tok = prof_begin(g, diropt ? "bfs_step_diropt" : "bfs_advance", s);
         if (diropt) {
             bfs_step_kernel<true><<<bfs_step_blocks(), kPushThreads, 0, s>>>(
-                n, g->m, g->row_off, g->col, g->t_row_off, g->t_col, depth, g->fb3, words, pq, it, g->hist);
+                n, g->m, g->row_off, g->col, g->t_row_off, g->t_col, depth, g->fb3, words, pq, it, g->hist,
+                g->h_mbox + kAheadPost, post_seq);
         } else {
             bfs_step_kernel<false><<<bfs_step_blocks(), kPushThreads, 0, s>>>(
-                n, g->m, g->row_off, g->col, g->t_row_off, g->t_col, depth, g->fb3, words, pq, it, g->hist);
+                n, g->m, g->row_off, g->col, g->t_row_off, g->t_col, depth, g->fb3, words, pq, it, g->hist,
+                g->h_mbox + kAheadPost, post_seq);
         }
         G1_LAUNCHED();
         prof_end(g, tok, s, 0.0);
@@ -533,13 +565,14 @@ g1_status run_bfs_push(g1_graph* g, uint32_t src, uint32_t* depth, bool diropt, 
         return run_small(g, s, pol, nullptr, diropt ? g->fb3 : nullptr, words, it0, res);
     };
     uint32_t launched = 0;
-    // A graph of a million edges or more is done within the first six levels or nearly so: they go out without a host
-    // read after the second (RMAT22 from the hub 189 -> 180 us, 1.5 M vertices 178 -> 170, push only 164 -> 149). On
-    // small graphs the frontier falls to the single-workgroup kernel's size sooner (4,096 vertices 107 -> 118).
-    const uint32_t first_batch = g->m >= (1u << 20) ? 6 : 2;
+    // From a million edges on (`ahead`) levels are long against a read, and few frontiers fit the single-workgroup kernel
+    // after two of them: the next two go out meanwhile. R-MAT, 2^21 vertices from the hub 146 -> 141 us, from a vertex
+    // of degree 3 199 -> 185, 1.0 M vertices 166 -> 158; a source without out-edges 60 -> 62 (six levels before the
+    // first read: 135, 183, 157 and 78), 40 levels of 40,000 vertices 1390 -> 1389 (1420). On 4,096 vertices the
+    // frontier falls to the single-workgroup kernel's size sooner (six levels first: 107 -> 118 us).
     auto no_pull = [](uint32_t) -> g1_status { return G1_OK; };
-    G1_TRY(drive_push(g, s, launch, after, small, g->max_out_deg <= kSmallCap, &launched, no_pull, 0, 0, ~0ull, 0,
-                      first_batch));
+    G1_TRY(drive_push(g, s, launch, after, small, g->max_out_deg <= kSmallCap, &launched, no_pull, 0, 0, ~0ull, 0, 2,
+                      false, g->m >= (1u << 20)));
     if (g->out_inv) G1_TRY(map_back<false>(g, depth, out, s));
     G1_HIP(hipEventRecord(g->ev[1], s));
     G1_TRY(collect_push_run(g, s, launched, out, st, true, false, g->out_inv != nullptr));
@@ -807,7 +840,7 @@ g1_status sssp_push_iterations(g1_graph* g, hipStream_t s, const DistBound& db, 
         sssp_noreturn_fraction() > 0.0 ? std::max<uint64_t>(static_cast<uint64_t>(sssp_noreturn_fraction() * g->m), 1)
                                        : ~0ull;
     int tok_c = -1;  // the collect launch of a no-return iteration (profiling)
-    auto launch = [&](uint32_t it, uint64_t edges) -> g1_status {
+    auto launch = [&](uint32_t it, uint64_t edges, uint32_t) -> g1_status {
         PushQueues pq = make_queues(g, it);
         tok_c = -1;
         if (edges >= noreturn_min) {
@@ -1048,7 +1081,7 @@ g1_status run_sssp_delta(g1_graph* g, uint32_t src, uint32_t* dist, g1_run_stats
     uint32_t it = 0, dense = 0, pulls = 0, buckets = 0;
     uint32_t limit = 0;
     int tok = -1, tok_c = -1;
-    auto light_launch = [&](uint32_t i, uint64_t edges) -> g1_status {
+    auto light_launch = [&](uint32_t i, uint64_t edges, uint32_t) -> g1_status {
         PushQueues pq = make_queues(g, i);
         tok_c = -1;
         if (edges >= noreturn_min) {

@@ -113,7 +113,7 @@ struct g1_graph {
     double* h_scalar = nullptr;           // pinned host scalar
     unsigned long long* h_hist = nullptr;  // pinned copy of the push engines' iteration history (lazy)
     unsigned long long* h_mbox = nullptr;  // coherent pinned mailbox: [0] post sequence, [1] nf, [2] E,
-                                           // [8], [12] sequence and value of the SpMV engines' last two posts
+                                           // [4] a BFS level's sequence and size, [8], [12] sequence and value of the SpMV engines' last two posts
     unsigned long long post_seq = 0;       // last sequence number posted to h_mbox
     hipEvent_t ev[2] = {nullptr, nullptr};
 

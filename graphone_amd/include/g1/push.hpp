@@ -1136,18 +1136,23 @@ __device__ __forceinline__ void pull_groups(uint32_t n, const uint32_t* __restri
 // pull when the frontier's out-edges exceed 1/14 of the edges not yet explored, push again when the
 // frontier falls below n/24 vertices. History: hist[2*it] = (E << 32) | nf, hist[2*it + 1] = edges
 // explored through this level | (pull << 63). Frontier bitmaps rotate over three buffers fb0..fb2
-// (`words` words each): read fb[it%3], write fb[(it+1)%3], clear fb[(it+2)%3].
+// (`words` words each): read fb[it%3], write fb[(it+1)%3], clear fb[(it+2)%3]. With seq (not 0) the host is told the
+// input frontier's size at once: *post = (seq << 32) | nf, one word in coherent pinned memory (a release of several
+// would write the L2 back first).
 template <bool kDirOpt>
 static __global__ void __launch_bounds__(kPushThreads)
 bfs_step_kernel(uint32_t n, uint32_t m, const uint32_t* __restrict__ row_off, const uint32_t* __restrict__ col,
                 const uint32_t* __restrict__ t_row_off, const uint32_t* __restrict__ t_col,
                 uint32_t* __restrict__ depth, uint32_t* __restrict__ fb, uint32_t words, PushQueues pq, uint32_t it,
-                unsigned long long* __restrict__ hist) {
+                unsigned long long* __restrict__ hist, unsigned long long* post, uint32_t seq) {
     __shared__ uint32_t s_vb[kSegments + 1];
     __shared__ uint32_t s_eb[kSegments + 1];
     const bool active = push_prologue(pq, s_vb, s_eb);
     const uint32_t nf = s_vb[kSegments];
     const uint32_t E = s_eb[kSegments];
+    if (seq && blockIdx.x == 0 && threadIdx.x == 0)
+        __hip_atomic_store(post, (static_cast<unsigned long long>(seq) << 32) | nf, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_SYSTEM);
     bool pull = false;
     unsigned long long explored = 0;
     if (kDirOpt) {

@@ -469,3 +469,25 @@ def test_views_run_concurrently(graphs):
         assert np.array_equal(r.view(np.uint32), want_r[k % len(srcs)].view(np.uint32)), k
     for v in views:
         v.close()
+
+
+def test_bfs_levels_ahead_of_the_read(gpu):
+    """From 2^20 edges on BFS enqueues its third and fourth level before it reads whether there is a third: runs that end
+    after one, two, three, four and five levels, that find nothing, and that go on for dozens of levels, on a graph
+    with a vertex past the single-workgroup kernel's size (12,000 out-edges), against the queue BFS."""
+    import graphone_amd as g1
+    rng = np.random.default_rng(5)
+    width, layers = 3000, 60
+    n = width * layers + 1
+    src = np.repeat(np.arange(width * (layers - 1)), 6)
+    dst = (src // width + 1) * width + rng.integers(0, width, src.size)
+    hub = np.zeros(12000, np.int64)
+    h = g1.HostGraph.from_edges(n, np.concatenate([src, hub]), np.concatenate([dst, rng.permutation(12000) + 1]))
+    assert h.m >= 1 << 20 and int(h.out_degrees().max()) > 8192
+    g = g1.Graph(h)
+    for s in [n - 1, n - 2, 0] + [width * (layers - back) + 7 for back in range(1, 8)]:
+        want = oracle.bfs_queue(h.row_offsets, h.col_indices, s)
+        for engine in ("advance", "diropt"):
+            got = g.bfs(s, engine)
+            assert np.array_equal(got.values, want), (s, engine)
+            assert got.stats["reached"] == int((want != g1.INF).sum()), (s, engine)
