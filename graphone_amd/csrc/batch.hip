@@ -111,8 +111,12 @@ uint32_t fill_blocks(size_t items) {
     return static_cast<uint32_t>(b ? b : 1);
 }
 
-// Words of the k = 64 activity bitmap (act_bits_kernel): two per 64 vertices.
-size_t act_words(size_t n) { return 2 * ((n + 63) / 64) + 2; }
+// Words of the k = 64 activity bitmap (act_bits_kernel), and with the groups' bitmap behind it.
+size_t act_words(size_t n) { return 16 * ((n + 511) / 512); }
+size_t act_all_words(size_t n) { return act_words(n) + (n + 2047) / 2048 + 1; }
+
+// Merge tiles past which the k = 64 min-plus kernel is built for eight waves a SIMD: more of them than the chip holds.
+constexpr uint32_t kMinPlusMany = 2048;
 
 // Merge tiles (rows + nonzeros per workgroup) the autotuner tries for the k = 64 min-plus kernel. Min is
 // order-free, so every partition gives the same bits; [kWaveTileOwn] is the graph's own partition (t_ws), shared
@@ -121,19 +125,22 @@ constexpr uint32_t kWaveTileItems[kWaveTileCount] = {kMergeTile / 4, kMergeTile 
 constexpr uint32_t kWaveTileOwn = 2;  // kWaveTileItems[kWaveTileOwn] == kMergeTile
 static_assert(sizeof(g1_graph::wave_coords) / sizeof(void*) == kWaveTileCount, "one partition per merge tile");
 
-// The merge partition of the in-edge CSR at kWaveTileItems[idx]; built once per graph and size (caller
-// holds g->mu), finished before it returns.
+// The merge partition of the in-edge CSR at kWaveTileItems[idx], and its quarters (wave_quarters); built once per graph
+// and size (caller holds g->mu), finished before it returns.
 g1_status ensure_wave_coords(g1_graph* g, uint32_t idx, hipStream_t s) {
-    if (idx == kWaveTileOwn || g->wave_coords[idx] || g->n == 0) return G1_OK;
-    const uint32_t tiles = merge_num_tiles_for(g->n, g->m, kWaveTileItems[idx]);
-    MergeCoord* c = nullptr;
-    G1_TRY(alloc_n(g, &c, static_cast<size_t>(tiles) + 1));
-    merge_partition_kernel<<<(tiles + 1 + 255) / 256, 256, 0, s>>>(g->t_row_off, g->n, g->m, tiles, c,
-                                                                   kWaveTileItems[idx]);
-    G1_LAUNCHED();
-    G1_HIP(hipStreamSynchronize(s));
-    g->wave_coords[idx] = c;
-    return G1_OK;
+    if (g->wave_quarters[idx] || g->n == 0) return G1_OK;
+    auto build = [&](uint32_t items, void** out) -> g1_status {
+        const uint32_t tiles = merge_num_tiles_for(g->n, g->m, items);
+        MergeCoord* c = nullptr;
+        G1_TRY(alloc_n(g, &c, static_cast<size_t>(tiles) + 1));
+        merge_partition_kernel<<<(tiles + 1 + 255) / 256, 256, 0, s>>>(g->t_row_off, g->n, g->m, tiles, c, items);
+        G1_LAUNCHED();
+        G1_HIP(hipStreamSynchronize(s));
+        *out = c;
+        return G1_OK;
+    };
+    if (idx != kWaveTileOwn && !g->wave_coords[idx]) G1_TRY(build(kWaveTileItems[idx], &g->wave_coords[idx]));
+    return build(kWaveTileItems[idx] / kMergeWaves, &g->wave_quarters[idx]);
 }
 
 // k = 64 plus-times SpMM on the wavefront kernel unless G1_PPR_WAVE=0 (same bits either way).
@@ -177,7 +184,7 @@ g1_status ensure_batch(g1_graph* g, uint32_t K, bool ppr, BatchWork** out, hipSt
         G1_TRY(alloc_n(g, &b->D, (n + 1) * K));  // row n: all unreached (read for inactive sources)
         G1_TRY(alloc_n(g, &b->mask[0], n));
         G1_TRY(alloc_n(g, &b->mask[1], n));
-        if (K == 64) G1_TRY(alloc_n(g, &b->act, act_words(n)));
+        if (K == 64) G1_TRY(alloc_n(g, &b->act, act_all_words(n)));
         if (K == 64 && minplus_u16() && (static_cast<uint64_t>(n) + 1) * 128 < (1ull << 32)) {
             G1_TRY(alloc_n(g, &b->D16, (n + 1) * 64));
             G1_TRY(alloc_n(g, &b->overflow, 64));
@@ -315,7 +322,7 @@ g1_status launch_rank64(g1_graph* g, const float* R_old, float* R_new, const flo
 // One min-plus SpMM iteration over the in-edges: D relaxed in place, change masks prev -> next, the
 // columns that changed ORed into *flag; then the fixup of rows that cross tiles. DT is the distance
 // storage (int16_t only at k = 64 with the wavefront kernel; overflow is then raised instead of storing
-// a distance >= 0xFFFF).
+// a distance of kCompactLimit or more).
 template <int K, typename DT = uint32_t>
 g1_status launch_minplus(g1_graph* g, DT* D, unsigned long long* mask_prev, unsigned long long* mask_next,
                          void* recs_v, bool weighted, unsigned long long* flag, hipStream_t s, uint32_t* act,
@@ -335,17 +342,26 @@ g1_status launch_minplus(g1_graph* g, DT* D, unsigned long long* mask_prev, unsi
                 coords = static_cast<const MergeCoord*>(g->wave_coords[tile_idx]);
                 fix_blocks = static_cast<uint32_t>((static_cast<uint64_t>(tiles) * K + 255) / 256);
             }
-            G1_CHECK(act != nullptr, G1_ERR_INTERNAL, "min-plus k = 64: activity bitmap missing");
+            G1_CHECK(act != nullptr && (g->wave_quarters[tile_idx] != nullptr || g->n == 0), G1_ERR_INTERNAL,
+                     "min-plus k = 64: activity bitmap or quarters missing");
             // The wavefront kernel writes only non-zero change masks, and reads activity as a bitmap.
             G1_TRY(g1_fill_u32(reinterpret_cast<uint32_t*>(mask_next), 0u, 2ull * g->n, reinterpret_cast<g1_stream_t>(s)));
-            act_bits_kernel<<<fill_blocks(static_cast<size_t>(g->n) / 4 + 64), 256, 0, s>>>(g->n, mask_prev, act);
+            uint32_t* const some = act + act_words(g->n);
+            act_bits_kernel<<<g->n / 2048 + 1, 256, 0, s>>>(g->n, mask_prev, act, reinterpret_cast<uint8_t*>(some));
             G1_LAUNCHED();
             auto go = [&](auto kernel) {
-                kernel<<<tiles, 256, 0, s>>>(g->n, kWaveTileItems[tile_idx], g->t_row_off, g->t_col, vals, coords, recs, D,
-                                             act, mask_next, flag, overflow);
+                kernel<<<tiles, 256, 0, s>>>(
+                    g->n, merge_num_tiles_for(g->n, g->m, kWaveTileItems[tile_idx] / kMergeWaves), g->t_row_off, g->t_col,
+                    vals, static_cast<const MergeCoord*>(g->wave_quarters[tile_idx]), recs, D, act, some, mask_next, flag,
+                    overflow);
             };
-            if (weighted) go(spmm_minplus_wave_kernel<true, DT>);
-            else go(spmm_minplus_wave_kernel<false, DT>);
+            if (tiles > kMinPlusMany) {
+                if (weighted) go(spmm_minplus_wave_kernel<true, true, DT>);
+                else go(spmm_minplus_wave_kernel<false, true, DT>);
+            } else {
+                if (weighted) go(spmm_minplus_wave_kernel<true, false, DT>);
+                else go(spmm_minplus_wave_kernel<false, false, DT>);
+            }
             G1_LAUNCHED();
             if (tiles > 1) {
                 if constexpr (sizeof(DT) == 2) {
@@ -935,6 +951,7 @@ g1_status session_create(g1_graph* g, int kind, uint32_t k, float restart, hipSt
     {
         std::lock_guard<std::mutex> lock(g->mu);  // lazily built graph arrays
         if (kind == kSessPpr) G1_TRY(ensure_pull_work(g, true));  // float weights, out-weight sums
+        else if (k == 64) G1_TRY(ensure_wave_coords(g, kWaveTileOwn, stream));
     }
     Session* ss = new Session();
     ss->g = g;
@@ -968,7 +985,7 @@ g1_status session_create(g1_graph* g, int kind, uint32_t k, float restart, hipSt
         if (hipGetLastError() != hipSuccess) return fail(set_error(G1_ERR_HIP, "session_create: launch"));
     } else {
         if ((st = sess_alloc(ss, &ss->D, (n + 1) * k)) != G1_OK) return fail(st);  // row n: unreached
-        if (k == 64 && (st = sess_alloc(ss, &ss->act, act_words(n))) != G1_OK) return fail(st);
+        if (k == 64 && (st = sess_alloc(ss, &ss->act, act_all_words(n))) != G1_OK) return fail(st);
         for (int i = 0; i < 2 && st == G1_OK; ++i) st = sess_alloc(ss, &ss->mask[i], n);
         if (st != G1_OK) return fail(st);
         // every column empty: D = INF, no source bits in either mask

@@ -609,11 +609,15 @@ __device__ __forceinline__ uint32_t wave_merge_search(const uint32_t* __restrict
 // sixteen before them fold: a nonzero adds its weight and takes the minimum, a row end (weight 0) compares the
 // minimum with its old distances, stores what improved and starts the next row. So a step costs two reads of
 // a lane, an address, an add and a minimum, and two scalar instructions; what bounds it is the 128 bytes of
-// distances it loads. Activity and indices of the next block load while a block folds.
+// distances it loads, and where next to no source is active the chain from a block's row ends to its sources to
+// their activity. Three blocks of that chain are under way at a time, a block's weights load when it turns out to have
+// an active source, the quarters' starts come from a partition of their own, and with kMany (more tiles than the chip
+// holds at once, built for eight waves a SIMD) a quarter whose first block is idle is looked over as a whole.
 // Measured on 2.1 M vertices, 33 M edges, 16-bit distances: a dense iteration 1.25 -> 0.69 ms (6.6 TB/s of
 // distance rows, the old ones with them), the batch 15.9 -> 9.2 ms, against a wave per tile that loaded 64
-// sources' rows, folded them around a bitmap of row starts and then loaded the old rows of what it closed. An
-// iteration with next to no active source takes 0.15 ms for its indices and activity (0.11 ms before).
+// sources' rows, folded them around a bitmap of row starts and then loaded the old rows of what it closed; with the
+// above 8.3 ms, and an iteration with one active source 0.11 ms (0.18 before it, 0.26 the wave per tile), on as many
+// edges between random vertices 0.12 (0.23, 0.16).
 //
 // Min is order-free, so the result does not depend on how rows are cut into tiles, quarters or blocks; rows that
 // cross tiles leave head / carry records in the SpmmTileRec layout and are finished by spmm_fixup_kernel
@@ -628,8 +632,8 @@ __device__ __forceinline__ uint32_t wave_merge_search(const uint32_t* __restrict
 // kCompactLimit (then a source row is one 128-byte line instead of two). 16-bit storage is exact or
 // void: -1 is the unreached distance, so a sign-extending load yields G1_INF for it and the distance
 // itself otherwise; a relaxation that would store a finite value >= kCompactLimit sets *overflow instead and
-// counts as no change (the run then still ends, and the caller reruns the batch with 32-bit storage). With 16-bit storage the weight is added with
-// unsigned saturation, which equals the semiring's combine because x + w cannot wrap (the caller only
+// counts as no change (the run then still ends, and the caller reruns the batch with 32-bit storage). With 16-bit
+// storage the weight is added with unsigned saturation, which equals the semiring's combine because x + w cannot wrap (the caller only
 // picks 16-bit storage when every weight is <= 0xFFFF0000).
 constexpr uint32_t kCompactLimit = 0x7FFFu;
 
@@ -639,46 +643,54 @@ __device__ __forceinline__ uint32_t widen_dist(DT raw) {
     return static_cast<uint32_t>(raw);
 }
 
-// act[v >> 5] bit (v & 31): mask[v] != 0 (the vertex changed in the last iteration). One wave per 64
-// vertices; act has 2 * ceil(n / 64) words.
+// act[v >> 5] bit (v & 31): mask[v] != 0 (the vertex changed in the last iteration); some[v >> 11] bit ((v >> 6) & 31):
+// any of the 64 vertices of v's group did. A wave takes eight groups (16 words of act, a byte of some), their masks
+// loaded together.
 static __global__ void __launch_bounds__(256) act_bits_kernel(uint32_t n, const unsigned long long* __restrict__ mask,
-                                                       uint32_t* __restrict__ act) {
+                                                       uint32_t* __restrict__ act, uint8_t* __restrict__ some) {
     const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t groups = (n + 63u) / 64u;
-    for (uint32_t gi = (blockIdx.x * 256u + threadIdx.x) / 64u; gi < groups; gi += gridDim.x * 4u) {
-        const uint32_t v = gi * 64u + lane;
-        const uint64_t b = ballot(v < n && mask[v] != 0ull);
-        if (lane < 2) act[2 * gi + lane] = static_cast<uint32_t>(b >> (32 * lane));
+    const uint32_t wi = blockIdx.x * 4u + threadIdx.x / 64u;
+    const uint32_t v0 = wi * 512u;
+    if (v0 >= n) return;
+    unsigned long long c[8];
+#pragma unroll
+    for (uint32_t t = 0; t < 8; ++t) {
+        const uint32_t v = v0 + t * 64u + lane;
+        c[t] = mask[v < n ? v : n - 1];
     }
+    uint32_t mine = 0;  // bit t: vertex `lane` of group t
+#pragma unroll
+    for (uint32_t t = 0; t < 8; ++t)
+        if (c[t] != 0ull && v0 + t * 64u + lane < n) mine |= 1u << t;
+    uint32_t word = 0, groups = 0;
+#pragma unroll
+    for (uint32_t t = 0; t < 8; ++t) {
+        const uint64_t b = ballot((mine >> t) & 1u);
+        if (lane / 2 == t) word = static_cast<uint32_t>(b >> (32 * (lane & 1u)));
+        groups |= (b != 0ull ? 1u : 0u) << t;
+    }
+    if (lane < 16) act[wi * 16u + lane] = word;
+    if (lane == 0) some[wi] = static_cast<uint8_t>(groups);
 }
 
-template <bool kWeighted, typename DT>
-__global__ void __launch_bounds__(256)
-spmm_minplus_wave_kernel(uint32_t n_rows, uint32_t tile_items, const uint32_t* __restrict__ row_offsets,
+template <bool kWeighted, bool kMany, typename DT>
+__global__ void __launch_bounds__(256, kMany ? 8 : 1)
+spmm_minplus_wave_kernel(uint32_t n_rows, uint32_t num_quarters, const uint32_t* __restrict__ row_offsets,
                          const uint32_t* __restrict__ col, const uint32_t* __restrict__ vals,
-                         const MergeCoord* __restrict__ coords, SpmmTileRec<MinPlusU32, 64>* __restrict__ recs,
-                         DT* __restrict__ D, const uint32_t* __restrict__ act_prev,
+                         const MergeCoord* __restrict__ quarters, SpmmTileRec<MinPlusU32, 64>* __restrict__ recs,
+                         DT* __restrict__ D, const uint32_t* __restrict__ act_prev, const uint32_t* __restrict__ some_prev,
                          unsigned long long* __restrict__ mask_next, unsigned long long* __restrict__ changed,
                          uint32_t* __restrict__ overflow) {
     __shared__ uint32_t s_mark[kMergeWaves][64];
     __shared__ uint32_t s_carry[kMergeWaves][64];
     __shared__ uint32_t s_ends[kMergeWaves];
-    __shared__ uint32_t s_row[kMergeWaves + 1];
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t tile = blockIdx.x;
-    const MergeCoord c0 = coords[tile], c1 = coords[tile + 1];
-    const uint64_t step0 = static_cast<uint64_t>(c0.x) + c0.y, step1 = static_cast<uint64_t>(c1.x) + c1.y;
-    auto quarter = [&](uint32_t w) { return step0 + w * (tile_items / 4) < step1 ? step0 + w * (tile_items / 4) : step1; };
-    const uint32_t r0 = wave_merge_search(row_offsets, c0.x, c1.x, quarter(wave));
-    if (lane == 0) {
-        s_row[wave] = r0;
-        if (wave == 0) s_row[kMergeWaves] = c1.x;
-    }
-    __syncthreads();
-    const uint32_t r_last = __builtin_amdgcn_readfirstlane(s_row[wave + 1]);
-    const uint32_t q0 = static_cast<uint32_t>(quarter(wave) - r0);
-    const uint32_t steps = static_cast<uint32_t>(quarter(wave + 1) - quarter(wave));
+    auto start = [&](uint32_t w) { return quarters[tile * kMergeWaves + w < num_quarters ? tile * kMergeWaves + w : num_quarters]; };
+    const MergeCoord c0 = start(0), begin = start(wave), end = start(wave + 1);
+    const uint32_t r0 = begin.x, r_last = end.x, q0 = begin.y;
+    const uint32_t steps = r_last - r0 + (end.y - q0);
     const bool continued = r0 < r_last && row_offsets[r0] < q0;  // its first row end closes an earlier quarter's row
 
     uint32_t acc = kInf;   // running minimum of the open row
@@ -703,19 +715,18 @@ spmm_minplus_wave_kernel(uint32_t n_rows, uint32_t tile_items, const uint32_t* _
         return D[static_cast<size_t>(u) * 64 + lane];
     };
 
-    // One block of 64 merge steps from row i, nonzero j on: the row-end mask, and the lane's row (a row end) or
-    // source and weight (a nonzero; a lane past the last step is a nonzero that `live` leaves out).
+    // One block of 64 merge steps from row i, nonzero j on: the row-end mask, and the lane's row (a row end) or source
+    // (a nonzero; a lane past the last step is a nonzero that `live` leaves out).
     struct Block {
-        uint64_t ends;
-        uint32_t id, w;
-        uint64_t live;
+        uint64_t ends, live;
+        uint32_t id;
     };
     uint32_t* mark = s_mark[wave];
-    auto load_block = [&](uint32_t i, uint32_t j, uint32_t left) -> Block {
+    // the ends of the 64 rows from row i on, a lane each: they say which steps of the block are row ends
+    auto load_ends = [&](uint32_t i) -> uint32_t { return i + lane < r_last ? row_offsets[i + 1 + lane] : kInf; };
+    auto load_block = [&](uint32_t i, uint32_t j, uint32_t left, uint32_t end) -> Block {
         Block b;
-        const uint32_t row = i + lane;
-        uint32_t at = 64;
-        if (row < r_last) at = row_offsets[row + 1] - j + lane;  // the step its end falls on
+        const uint32_t at = i + lane < r_last ? end - j + lane : 64u;  // the step its end falls on
         // (a wave's LDS operations run in program order, which the compiler must keep too)
         mark[lane] = 0u;
         asm volatile("" ::: "memory");
@@ -726,28 +737,41 @@ spmm_minplus_wave_kernel(uint32_t n_rows, uint32_t tile_items, const uint32_t* _
         const uint32_t before = mask_prefix(b.ends);
         b.live = ballot(lane < left && !is_end);
         b.id = i + before;
-        b.w = 0;
-        if (lane < left && !is_end) {
-            const uint32_t q = j + lane - before;
-            b.id = __builtin_nontemporal_load(col + q);
-            b.w = kWeighted ? __builtin_nontemporal_load(vals + q) : 1u;
-        }
+        if (lane < left && !is_end) b.id = __builtin_nontemporal_load(col + (j + lane - before));
         return b;
     };
     auto activity = [&](const Block& b) -> uint32_t { return (b.live >> lane) & 1ull ? act_prev[b.id >> 5] : 0u; };
 
+    // Three blocks are under way: the one that folds, whose sources' activity is there or on its way; the next, whose
+    // sources are; and the one after it, whose row ends are.
     uint64_t pending = 0;  // 1: the open row has an active nonzero in an earlier block
-    Block cur = load_block(r0, q0, steps);
-    uint32_t word = activity(cur);
     uint32_t i = r0, j = q0;
-    for (uint32_t s = 0; s < steps; s += 64) {
-        const uint32_t rows = static_cast<uint32_t>(__popcll(cur.ends));
+    Block cur = load_block(i, j, steps, load_ends(i));
+    uint32_t j_cur = j;
+    auto pass = [&](const Block& b) {
+        const uint32_t rows = static_cast<uint32_t>(__popcll(b.ends));
         i += rows;
         j += 64 - rows;
-        Block next{0, 0, 0, 0};
+    };
+    pass(cur);
+    Block next{0, 0, 0};
+    uint32_t j_next = j, ends2 = 0;
+    if (steps > 64) {
+        next = load_block(i, j, steps - 64, load_ends(i));
+        pass(next);
+        if (steps > 128) ends2 = load_ends(i);
+    }
+    uint32_t word = activity(cur);
+    for (uint32_t s = 0; s < steps; s += 64) {
+        Block next2{0, 0, 0};
+        const uint32_t j_next2 = j;
         uint32_t next_word = 0;
-        const bool more = s + 64 < steps;
-        if (more) next = load_block(i, j, steps - s - 64);
+        if (s + 128 < steps) {
+            next2 = load_block(i, j, steps - s - 128, ends2);
+            pass(next2);
+            if (s + 192 < steps) ends2 = load_ends(i);
+        }
+        if (s + 64 < steps) next_word = activity(next);
         const uint64_t active = ballot((word >> (cur.id & 31u)) & 1u) & cur.live;
         // A row end needs its row when a nonzero since the row end before it is active (or the row is pending):
         // adding the active bits to the runs of ones between the row ends carries into exactly those.
@@ -758,9 +782,31 @@ spmm_minplus_wave_kernel(uint32_t n_rows, uint32_t tile_items, const uint32_t* _
         pending = (sum < runs ? 1u : 0u) | (all < sum ? 1u : 0u);
         const bool idle = (active | need) == 0ull;
         const uint32_t id = ((active | need) >> lane) & 1ull ? cur.id : n_rows;
-        const uint32_t w = cur.w;
-        if (more) next_word = activity(next);
+        if (kMany && idle && s == 0 && steps > 128) {
+            // Where the first block is idle, the rest mostly is: the sources past the next block are looked at without
+            // their row ends, by their groups' activity first (a table that the L1 holds), and a quarter without an
+            // active one is done.
+            bool hit = ((next_word >> (next.id & 31u)) & 1u) != 0u;
+            const uint32_t left = end.y - j_next2;
+            for (uint32_t q = 0; q < left; q += 8 * 64) {
+                uint32_t id[8], group[8];
+#pragma unroll
+                for (uint32_t k = 0; k < 8; ++k) {
+                    const uint32_t at = q + k * 64 + lane;
+                    id[k] = at < left ? __builtin_nontemporal_load(col + j_next2 + at) : 0u;
+                }
+#pragma unroll
+                for (uint32_t k = 0; k < 8; ++k) group[k] = q + k * 64 + lane < left ? some_prev[id[k] >> 11] : 0u;
+#pragma unroll
+                for (uint32_t k = 0; k < 8; ++k)
+                    if ((group[k] >> ((id[k] >> 6) & 31u)) & 1u) hit |= ((act_prev[id[k] >> 5] >> (id[k] & 31u)) & 1u) != 0u;
+            }
+            if (ballot(hit) == 0ull) break;
+        }
         if (!idle) {
+            uint32_t w = 1;  // (a row end's: 0)
+            if (kWeighted) w = (active >> lane) & 1ull ? __builtin_nontemporal_load(vals + (j_cur + lane - mask_prefix(cur.ends))) : 0u;
+            else if ((cur.ends >> lane) & 1ull) w = 0;
             uint32_t x[kWaveChunk];
 #pragma unroll
             for (uint32_t t = 0; t < kWaveChunk; ++t) x[t] = dist(__builtin_amdgcn_readlane(id, t));
@@ -790,6 +836,9 @@ spmm_minplus_wave_kernel(uint32_t n_rows, uint32_t tile_items, const uint32_t* _
             }
         }
         cur = next;
+        next = next2;
+        j_cur = j_next;
+        j_next = j_next2;
         word = next_word;
     }
 

@@ -258,3 +258,28 @@ def test_ppr_batch64_scale_array(gpu, n):
         for c in (0, 2, 40, 66):
             single = g.ppr(seeds[c], restart=restart, max_iter=9, tol=0.0)
             assert np.array_equal(got.values[c].view(np.uint32), single.values.view(np.uint32)), (restart, c)
+
+
+def test_batch64_idle_iterations(gpu):
+    """A k = 64 min-plus batch of more merge tiles than the chip holds at once (its kernel then looks a whole quarter
+    over where the first block has no active source): 40 iterations with one changed vertex a source, at ids on both
+    ends of the activity bitmaps' words and bytes, then a dense spread from the path's end through 4.3 million
+    edges, into a hub of 30,000 in-edges as well; weighted and as BFS, on two merge tiles, against the oracle."""
+    import graphone_amd as g1
+    rng = np.random.default_rng(3)
+    n, m = 500_003, 4_300_000
+    path = np.array([0, 63, 64, 511, 512, 2047, 2048, n - 1, n - 3] + list(range(5000, 5031)))
+    body = np.setdiff1d(np.arange(n), path)
+    src = np.concatenate([rng.choice(body, m), rng.choice(body, 30000), path[:-1], np.full(5, path[-1])])
+    dst = np.concatenate([rng.choice(body, m), np.full(30000, body[7]), path[1:], rng.choice(body, 5)])
+    h = g1.HostGraph.from_edges(n, src, dst, rng.integers(1, 200, src.size).astype(np.uint32))
+    g = g1.Graph(h)
+    srcs = [int(path[0]), int(path[3]), int(path[8]), int(body[11])] * 16
+    for tile in (2048, 4096):
+        g.set_merge_tile(tile)
+        for weighted in (True, False):
+            got = g.sssp_batch(srcs, k=64, weighted=weighted).values
+            for c in range(4):
+                want = (oracle.dijkstra(h.row_offsets, h.col_indices, h.weights, srcs[c]) if weighted else
+                        oracle.bfs_queue(h.row_offsets, h.col_indices, srcs[c]))
+                assert np.array_equal(got[c], want) and np.array_equal(got[60 + c], want), (tile, weighted, c)
