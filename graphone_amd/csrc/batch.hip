@@ -156,7 +156,8 @@ bool ppr_wave() {
 // call, instead of gathering them. The gather is one of 4 bytes a nonzero beside the 256-byte rows, and past the L2 it
 // costs a line each: RMAT22 x 64 columns 4.0 -> 3.5 ms an iteration (198.6 -> 175.1 ms for 50), 2 M vertices 65.4 ->
 // 61.2 ms, 0.7 M 25.5 -> 24.0. Below 2^18 vertices iw is a small part of the L2 and the array a launch more (20,000
-// vertices 5.74 -> 5.78 ms). Past 128 in-edges a vertex the array would take more memory than a 64-column one.
+// vertices 5.74 -> 5.78 ms). Up to 128 in-edges a vertex the array takes no more memory than the two 64-column ones
+// (x and y) that the product does without; where there is no room for it the scales are gathered.
 bool scales_stream(const g1_graph* g) { return g->n >= (1u << 18) && g->m <= 128ull * g->n && g->m > 0; }
 
 g1_status ensure_batch(g1_graph* g, uint32_t K, bool ppr, BatchWork** out, hipStream_t s) {
@@ -195,12 +196,14 @@ g1_status ensure_batch(g1_graph* g, uint32_t K, bool ppr, BatchWork** out, hipSt
         if (K != 64 || !ppr_wave()) {  // (the wavefront kernel needs neither, see RankBatchPolicy)
             if (!b->X) G1_TRY(alloc_n(g, &b->X, n * K));
             if (!b->Y) G1_TRY(alloc_n(g, &b->Y, n * K));
-        } else if (scales_stream(g) && !b->iw_nz) {
-            G1_TRY(alloc_n(g, &b->iw_nz, g->m));
         }
-        G1_TRY(alloc_n(g, &b->R[1], n * K));
         G1_TRY(ensure_rank_partials(g));
         G1_TRY(ensure_pull_work(g, true));  // iw
+        G1_TRY(alloc_n(g, &b->R[1], n * K));
+        if (K == 64 && ppr_wave() && scales_stream(g) && alloc_n(g, &b->iw_nz, g->m) != G1_OK) {
+            (void)hipGetLastError();  // the failed allocation's, which the next launch check would report
+            b->iw_nz = nullptr;
+        }
     }
     *out = b;
     return G1_OK;
