@@ -177,19 +177,19 @@ g1_status ensure_batch(g1_graph* g, uint32_t K, bool ppr, BatchWork** out, hipSt
                                        sizeof(SpmmTileRec<MinPlusU32, 64>),
                                    spmm_records_bytes<PlusTimesF32, 64>(g->n, g->m));
         void* v = nullptr;
+        if (!b->changed) G1_TRY(alloc_n(g, &b->changed, 64));
         G1_TRY(graph_alloc(g, &v, rb + 256));
         b->recs = v;
-        G1_TRY(alloc_n(g, &b->changed, 64));
     }
-    if (!ppr && !b->D) {
-        G1_TRY(alloc_n(g, &b->D, (n + 1) * K));  // row n: all unreached (read for inactive sources)
-        G1_TRY(alloc_n(g, &b->mask[0], n));
-        G1_TRY(alloc_n(g, &b->mask[1], n));
-        if (K == 64) G1_TRY(alloc_n(g, &b->act, act_all_words(n)));
-        if (K == 64 && minplus_u16() && (static_cast<uint64_t>(n) + 1) * 128 < (1ull << 32)) {
+    if (!ppr && !b->D) {  // (D last: a call after one that ran out of memory allocates what is missing)
+        for (int i = 0; i < 2; ++i)
+            if (!b->mask[i]) G1_TRY(alloc_n(g, &b->mask[i], n));
+        if (K == 64 && !b->act) G1_TRY(alloc_n(g, &b->act, act_all_words(n)));
+        if (K == 64 && minplus_u16() && (static_cast<uint64_t>(n) + 1) * 128 < (1ull << 32) && !b->D16) {
+            if (!b->overflow) G1_TRY(alloc_n(g, &b->overflow, 64));
             G1_TRY(alloc_n(g, &b->D16, (n + 1) * 64));
-            G1_TRY(alloc_n(g, &b->overflow, 64));
         }
+        G1_TRY(alloc_n(g, &b->D, (n + 1) * K));  // row n: all unreached (read for inactive sources)
     }
     if (ppr && !b->R[1]) {
         if (!b->R[0]) G1_TRY(alloc_n(g, &b->R[0], n * K));
