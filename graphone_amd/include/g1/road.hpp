@@ -228,7 +228,7 @@ road_query_kernel(const uint32_t* __restrict__ row_off, const uint32_t* __restri
                     v[r] = col[e];
                     if (kSssp) {
                         w[r] = wts[e];
-                    dw[r] = __hip_atomic_load(&ds[u[r]], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);  // (BFS: unused)
+                        dw[r] = __hip_atomic_load(&ds[u[r]], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
                     }
                 }
                 RoadRow row[R];
@@ -338,8 +338,9 @@ road_lds_kernel(uint32_t n, const uint32_t* __restrict__ row_off, const uint32_t
     const road_global<uint32_t> gq[2] = {to_global(Q.q[0]), to_global(Q.q[1])};
     const road_global<uint32_t> far[2] = {to_global(Q.far[0]), to_global(Q.far[1])};
     // The second load of an edge: its weight, or (BFS) its target again. Without a branch between them the two are in
-    // flight together (30 sources of a 150x200 grid 642 -> 629 us with the pointers above). road_query_kernel keeps its branch: its
-    // second load comes with the distance, which a BFS has no use for (48 sources of a 610x377 grid: 4.07 against 4.19 ms).
+    // flight together (30 sources of a 150x200 grid 642 -> 629 us with the pointers above). road_query_kernel keeps its
+    // branch: its second load comes with the distance, which a BFS has no use for (48 sources of a 610x377 grid: 4.07
+    // against 4.19 ms).
     const uint32_t* const second = kSssp ? wts : col;
     const uint32_t words = (n + 1) / 2, fwords = (n + 31) / 32;
     for (uint32_t i = tid; i < words; i += kRoadThreads) s_d[i] = 0xFFFFFFFFu;

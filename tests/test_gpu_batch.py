@@ -5,6 +5,10 @@ Min-plus columns (SSSP distances, BFS depths) are compared with the oracle's Dij
 with g1_sssp's BLAS engine (apps/sssp_blas.cu:17-84); personalized PageRank columns with g1_ppr
 (apps/pagerank_blas.cu:16-125 with a restart vector) bit for bit, and with the FP64 oracle within L1 1e-5.
 """
+import os
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 
@@ -283,3 +287,33 @@ def test_batch64_idle_iterations(gpu):
                 want = (oracle.dijkstra(h.row_offsets, h.col_indices, h.weights, srcs[c]) if weighted else
                         oracle.bfs_queue(h.row_offsets, h.col_indices, srcs[c]))
                 assert np.array_equal(got[c], want) and np.array_equal(got[60 + c], want), (tile, weighted, c)
+
+
+def test_switched_off_wave_kernels_give_the_same_bits(gpu, tmp_path):
+    """G1_PPR_WAVE=0 (the 64-column PPR product by rounds, with x and y arrays and a rank kernel) and G1_MINPLUS_WAVE=0
+    with G1_MINPLUS_U16=0 (the min-plus batch on the chunked kernel): the bits of the default kernels, more seeds than
+    a tile holds and fewer, columns that converge before others."""
+    import graphone_amd as g1
+    code = """
+import sys
+import numpy as np
+import graphone_amd as g1
+h = g1.HostGraph.rmat(13, 12, seed=9).assign_weights(1, 300, seed=10)
+g = g1.Graph(h)
+rng = np.random.default_rng(4)
+out = {}
+for count in (5, 70):
+    ids = rng.integers(0, h.n, count)
+    out[f"ppr{count}"] = g.ppr_batch(ids, max_iter=31, tol=1e-4, k=64).values.view(np.uint32)
+    out[f"sssp{count}"] = g.sssp_batch(ids, k=64).values
+np.savez(sys.argv[1], **out)
+"""
+    got = []
+    for name, env in (("on", {}), ("off", {"G1_PPR_WAVE": "0", "G1_MINPLUS_WAVE": "0", "G1_MINPLUS_U16": "0"})):
+        path = str(tmp_path / f"{name}.npz")
+        root = os.path.dirname(os.path.dirname(os.path.abspath(g1.__file__)))
+        subprocess.run([sys.executable, "-c", code, path], check=True, timeout=100,
+                       env={**os.environ, **env, "PYTHONPATH": root})
+        got.append(np.load(path))
+    for key in got[0].files:
+        assert np.array_equal(got[0][key], got[1][key]), key

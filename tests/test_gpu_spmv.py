@@ -1,7 +1,7 @@
 """Semiring SpMV parity on the GPU (merge-path and CSR-vector) against the oracle's naive fold
 (restating include/GraphOne/archi/blas/spmv/cpu/naive.hpp:5-20).
 
-min-plus u32: bit-exact. plus-times f32 (Kahan): within 2e-6 relative of the FP64 fold per row, and the
+min-plus u32: bit-exact. plus-times f32 (32-bit products, 64-bit sums): within 2e-6 relative of the FP64 fold per row, and the
 result is deterministic (identical bits on a re-run).
 """
 import numpy as np
