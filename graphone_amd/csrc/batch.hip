@@ -152,6 +152,13 @@ bool ppr_wave() {
     return on;
 }
 
+// Whether an iteration of the k = 64 PPR is the fused product (launch_rank64) and the L1 pass, or y = A x and the rank
+// kernel. The fusion saves 12 of 20 bytes an element and costs a multiplication and a scale a nonzero; while the 64
+// columns are in the caches the bytes are nothing. 50 iterations, y and x arrays against fused: 5,000 vertices 4.0 and
+// 4.3 ms, 50,000 4.8 and 5.2, 130,000 6.1 and 6.3, 200,000 7.2 and 7.2 (4 in-edges a vertex 6.3 and 6.0), 300,000 10.6
+// and 9.9.
+bool ppr_fused(const g1_graph* g) { return ppr_wave() && g->n >= (1u << 17); }
+
 // Whether the k = 64 PPR product reads its sources' scales (iw) from an array in the in-edges' order, filled once per
 // call, instead of gathering them. The gather is one of 4 bytes a nonzero beside the 256-byte rows, and past the L2 it
 // costs a line each: RMAT22 x 64 columns 4.0 -> 3.5 ms an iteration (198.6 -> 175.1 ms for 50), 2 M vertices 65.4 ->
@@ -193,14 +200,14 @@ g1_status ensure_batch(g1_graph* g, uint32_t K, bool ppr, BatchWork** out, hipSt
     }
     if (ppr && !b->R[1]) {
         if (!b->R[0]) G1_TRY(alloc_n(g, &b->R[0], n * K));
-        if (K != 64 || !ppr_wave()) {  // (the wavefront kernel needs neither, see RankBatchPolicy)
+        if (K != 64 || !ppr_fused(g)) {  // (the fused product needs neither, see RankBatchPolicy)
             if (!b->X) G1_TRY(alloc_n(g, &b->X, n * K));
             if (!b->Y) G1_TRY(alloc_n(g, &b->Y, n * K));
         }
         G1_TRY(ensure_rank_partials(g));
         G1_TRY(ensure_pull_work(g, true));  // iw
         G1_TRY(alloc_n(g, &b->R[1], n * K));
-        if (K == 64 && ppr_wave() && scales_stream(g) && alloc_n(g, &b->iw_nz, g->m) != G1_OK) {
+        if (K == 64 && ppr_fused(g) && scales_stream(g) && alloc_n(g, &b->iw_nz, g->m) != G1_OK) {
             (void)hipGetLastError();  // the failed allocation's, which the next launch check would report
             b->iw_nz = nullptr;
         }
@@ -531,7 +538,7 @@ g1_status ppr_tile_run(g1_graph* g, BatchWork* b, const uint32_t* seeds_host, ui
     auto iteration = [&](int cur, hipStream_t st) -> g1_status {
         bool fused = false;
         if constexpr (K == 64) {
-            if (ppr_wave()) {
+            if (ppr_fused(g)) {
                 G1_TRY(launch_rank64(g, b->R[cur], b->R[cur ^ 1], b->iw_nz, restart, state, b->recs, st));
                 rank_delta_batch_kernel<K><<<rank_apply_grid<K>(nb), 256, 0, st>>>(n, b->R[cur], b->R[cur ^ 1], g->rpart,
                                                                                  nb, state);

@@ -966,9 +966,9 @@ struct PlusTimesBatchPolicy {
 // rank times its out-weight's inverse (the product rank_apply_batch_kernel would have stored, so the same bits),
 // and a row's sum goes straight to its new rank. Columns in state[0] (converged, or padding) are not stored:
 // rank_delta_batch_kernel carries their ranks over. Saves y written and read and x written, 12 of 20 bytes an element
-// beside the gathers, for a multiplication a nonzero and its source's scale (which streams beside the weights on large graphs, see
-// scales_stream in batch.hip): 0.7 M vertices x 64 columns 0.38 (product) + 0.17 ms (apply) an
-// iteration before, 0.40 + 0.06 (L1 partials) here; a graph of 20,000 vertices takes 4 % longer (114 us an iteration).
+// beside the gathers, for a multiplication a nonzero and its source's scale (which streams beside the weights on
+// large graphs, see scales_stream in batch.hip): 0.7 M vertices x 64 columns 0.38 (product) + 0.17 ms (apply) an
+// iteration before, 0.40 + 0.06 (L1 partials) here. Small graphs keep the two (ppr_fused).
 struct RankBatchPolicy {
     using aux_t = uint32_t;
     static constexpr bool kHasAux = false;

@@ -317,3 +317,22 @@ np.savez(sys.argv[1], **out)
         got.append(np.load(path))
     for key in got[0].files:
         assert np.array_equal(got[0][key], got[1][key]), key
+
+
+@pytest.mark.parametrize("n", [(1 << 17) - 1, 1 << 17])
+def test_ppr_batch64_fusion_line(gpu, n):
+    """Below 2^17 vertices an iteration of the 64-column PPR is a product and a rank kernel, from there one kernel that
+    writes the ranks: a column has the single-seed run's bits and iteration either way, with fewer seeds than columns
+    and columns that converge at different iterations."""
+    import graphone_amd as g1
+    rng = np.random.default_rng(n)
+    m = 300_001
+    src, dst = rng.integers(0, n, m) // 3, rng.integers(0, n, m)
+    h = g1.HostGraph.from_edges(n, src, dst, rng.integers(1, 50, m).astype(np.uint32), directed=True)
+    g = g1.Graph(h)
+    seeds = [0, n - 1, int(src[5]), int(src[6]), int(dst[9])]
+    for tol, iters in ((0.0, 7), (1e-3, 40)):
+        got = g.ppr_batch(seeds, max_iter=iters, tol=tol, k=64)
+        for c, s in enumerate(seeds):
+            single = g.ppr(s, max_iter=iters, tol=tol)
+            assert np.array_equal(got.values[c].view(np.uint32), single.values.view(np.uint32)), (tol, c)
