@@ -1320,7 +1320,7 @@ g1_status run_minplus_pull(g1_graph* g, uint32_t src, uint32_t* d, bool weighted
     auto launch = [&](uint32_t, unsigned long long* post, unsigned long long seq) -> g1_status {
         if (engine == G1_ENGINE_BLAS_CSRVEC) {
             const int tok = prof_begin(g, "spmv_csrvec_minplus", s);
-            G1_TRY(launch_spmv_csrvec<MinPlusU32>(n, g->t_row_off, g->t_col, vals, g->xu, g->yu, lanes, s, g->t_long,
+            G1_TRY(launch_spmv_csrvec<MinPlusU32>(n, g->m, g->t_row_off, g->t_col, vals, g->xu, g->yu, lanes, s, g->t_long,
                                                   g->t_nlong, g->long_min));
             prof_end(g, tok, s, spmv_bytes);
         } else {
@@ -1423,7 +1423,7 @@ g1_status run_pagerank(g1_graph* g, float alpha, uint32_t seed, float restart, u
             delta = g->h_scalar[0];
             if (delta <= tol || it >= max_iter) break;
             if (engine == G1_ENGINE_BLAS_CSRVEC)
-                G1_TRY(launch_spmv_csrvec<PlusTimesF32>(n, t_ro, t_ci, vals, g->xf, g->yf, lanes, s, lrows, nlong,
+                G1_TRY(launch_spmv_csrvec<PlusTimesF32>(n, g->m, t_ro, t_ci, vals, g->xf, g->yf, lanes, s, lrows, nlong,
                                                               g->long_min));
             else
                 G1_TRY(launch_spmv_merge<PlusTimesF32>(n, g->m, t_ro, t_ci, vals, g->xf, g->yf, ws, s));
@@ -1445,7 +1445,7 @@ g1_status run_pagerank(g1_graph* g, float alpha, uint32_t seed, float restart, u
             int tok;
             if (engine == G1_ENGINE_BLAS_CSRVEC) {
                 tok = prof_begin(g, "spmv_csrvec_plustimes", s);
-                G1_TRY(launch_spmv_csrvec<PlusTimesF32>(n, t_ro, t_ci, vals, g->xf, g->yf, lanes, s, lrows, nlong,
+                G1_TRY(launch_spmv_csrvec<PlusTimesF32>(n, g->m, t_ro, t_ci, vals, g->xf, g->yf, lanes, s, lrows, nlong,
                                                         g->long_min));
             } else {
                 tok = prof_begin(g, "spmv_merge_plustimes", s);

@@ -36,7 +36,7 @@ g1_status spmv_csrvec_exported(uint32_t n_rows, uint32_t n_cols, uint32_t nnz, c
     if (lanes == 0) lanes = csrvec_lanes(n_rows, nnz);
     G1_CHECK(lanes <= 64 && (lanes & (lanes - 1)) == 0, G1_ERR_INVALID_ARG,
              "spmv_csrvec: lanes must be a power of two in 1..64, got %u", lanes);
-    return launch_spmv_csrvec<S>(n_rows, row_offsets, col, vals, x, y, lanes, as_stream(stream));
+    return launch_spmv_csrvec<S>(n_rows, nnz, row_offsets, col, vals, x, y, lanes, as_stream(stream));
 }
 
 // Scratch of g1_spmv_merge_minplus_u32_noalloc: the merge-path coordinates and tile records of one

@@ -800,7 +800,8 @@ sssp_pull_rows_kernel(uint32_t n, const uint32_t* __restrict__ t_row_off, const 
         const uint32_t row = huge_rows[blockIdx.x];
         if (xb[row] != 255u) return;  // not visited (uniform across the workgroup)
         acc_t acc = S::identity();
-        csrvec_fold<S, true, kPushThreads>(t_col, t_w, xb, t_row_off[row] + threadIdx.x, t_row_off[row + 1], acc);
+        csrvec_fold<S, true, kPushThreads>(t_col, t_w, xb, t_row_off[row], threadIdx.x, t_row_off[row + 1],
+                                           csrvec_top(t_row_off[n]), acc);
         s_acc[threadIdx.x] = acc;
         __syncthreads();
 #pragma unroll

@@ -115,3 +115,30 @@ def test_merge_rejects_small_workspace(gpu):
     with pytest.raises(g1.G1Error) as e:
         g1.spmv("merge", "minplus_u32", d_rp, d_ci, None, d_x, d_y, 1, 1, 1, tiny)
     assert e.value.status == 1
+
+
+@pytest.mark.parametrize("lanes", [0, 1, 16])
+def test_csrvec_nnz_near_2_32(gpu, lanes):
+    """CSR-vector rows up to nonzero 2^32 - 2, the most a matrix may have: a lane's next entry lies past 2^32 there. All
+    but the last four rows hold source 0 1,024 times; sums are whole numbers."""
+    import ctypes as C
+
+    import graphone_amd as g1
+    m, n_rows = (1 << 32) - 2, 1 << 22
+    rp = np.minimum(np.arange(n_rows + 1, dtype=np.int64) * 1024, m).astype(np.uint32)
+    tail = np.random.default_rng(lanes).integers(1, 500, 4 * 1024 - 2).astype(np.uint32)
+    ci = g1.DeviceArray(m, np.uint32)
+    ci.fill(0)
+    g1._lib.call("g1_memcpy_h2d", C.c_void_p(ci.ptr + 4 * (m - tail.size)), tail.ctypes.data_as(C.c_void_p),
+                 C.c_size_t(tail.nbytes), None)
+    x = np.random.default_rng(1).integers(2, 1000, 500).astype(np.uint32)
+    x[0] = 1
+    x[tail[-1]] = 0
+    parts = np.split(x[tail].astype(np.int64), [1024, 2048, 3072])
+    drp = g1.DeviceArray.from_numpy(rp)
+    for op, dtype, first, last in (("minplus_u32", np.uint32, 2, [int(p.min()) + 1 for p in parts]),
+                                   ("plustimes_f32", np.float32, 1024, [float(p.sum()) for p in parts])):
+        dx, y = g1.DeviceArray.from_numpy(x.astype(dtype)), g1.DeviceArray(n_rows, dtype)
+        g1.spmv("csrvec", op, drp, ci, None, dx, y, n_rows, 500, m, lanes=lanes)
+        got = y.numpy()
+        assert np.all(got[:-4] == first) and got[-4:].tolist() == last, op
