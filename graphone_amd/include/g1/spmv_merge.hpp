@@ -79,7 +79,7 @@ __device__ __forceinline__ MergeCoord merge_path_search(uint64_t diag, const uin
     uint32_t lo = diag > nnz ? static_cast<uint32_t>(diag - nnz) : 0u;
     uint32_t hi = diag < n_rows ? static_cast<uint32_t>(diag) : n_rows;
     while (lo < hi) {
-        const uint32_t mid = (lo + hi) >> 1;
+        const uint32_t mid = lo + ((hi - lo) >> 1);
         if (static_cast<uint64_t>(row_end[mid]) + mid + 1 <= diag) lo = mid + 1; else hi = mid;
     }
     return MergeCoord{lo, static_cast<uint32_t>(diag - lo)};
